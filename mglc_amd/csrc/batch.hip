@@ -157,14 +157,9 @@ __global__ __launch_bounds__(256) void k_batch_init(const BatchArgs b) {
             if constexpr (EY[al] != 0) un = mac<EY[al]>(un, v);
             if constexpr (EZ[al] != 0) un = mac<EZ[al]>(un, w);
             const double feq = rho * weight(al) * (1.0 + 3.0 * un + 4.5 * un * un - 1.5 * us2);
-            f[al] = S::SHIFT ? R(feq - weight(al)) : R(feq);
+            f[al] = S::SHIFT ? R((feq - weight(al)) * b.scale) : R(feq);
         });
-        Moments<R, S::SHIFT> q;
-        q.rho = R(rho);
-        q.drho = R(rho - 1.0);
-        q.u = R(u);
-        q.v = R(v);
-        q.w = R(w);
+        const Moments<R> q = moments_of<S>(rho, u, v, w, b.scale);
         if (k == in.nz - 1) b.lid_rho[in.lid_off + i + (long long)in.nx * j] = rho;
         InstView a;
         a.snu = in.snu;
@@ -176,7 +171,7 @@ __global__ __launch_bounds__(256) void k_batch_init(const BatchArgs b) {
         const unsigned h = cell_random<S>(c, 0u);
         sfor<Q>([&](auto A) {
             constexpr int al = decltype(A)::value;
-            S::st(dst + (long long)al * in.ps + c, f[al], b.scale, store_random<S, al>(h));
+            st<S>(dst + (long long)al * in.ps + c, f[al], store_random<S, al>(h));
         });
     }
 }

@@ -278,14 +278,9 @@ __global__ __launch_bounds__(256) void k_cavity_init(const StepArgs a, const dou
         if constexpr (EY[al] != 0) un = mac<EY[al]>(un, v);
         if constexpr (EZ[al] != 0) un = mac<EZ[al]>(un, w);
         const double feq = rho * weight(al) * (1.0 + 3.0 * un + 4.5 * un * un - 1.5 * us2);
-        f[al] = S::SHIFT ? R(feq - weight(al)) : R(feq);
+        f[al] = S::SHIFT ? R((feq - weight(al)) * a.scale) : R(feq);
     });
-    Moments<R, S::SHIFT> q;
-    q.rho = R(rho);
-    q.drho = R(rho - 1.0);
-    q.u = R(u);
-    q.v = R(v);
-    q.w = R(w);
+    const Moments<R> q = moments_of<S>(rho, u, v, w, a.scale);
     a.rho[m] = rho;
     a.u[m] = u;
     a.v[m] = v;
@@ -296,7 +291,7 @@ __global__ __launch_bounds__(256) void k_cavity_init(const StepArgs a, const dou
     const unsigned h = cell_random<S>(c, a.seed);
     sfor<Q>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        S::st(dst + (long long)al * a.ps + c, f[al], a.scale, store_random<S, al>(h));
+        st<S>(dst + (long long)al * a.ps + c, f[al], store_random<S, al>(h));
     });
 }
 
@@ -433,36 +428,12 @@ struct Table {
         {k_cavity_interior<S, COLL_BGK, false>, k_cavity_interior<S, COLL_BGK, true>}};
 };
 
-// FP16 MRT at the default store scale 2^12, folded into the inverse
-// transform (StoreF16K12): the same bits as StoreF16, 19 multiplies fewer
-// per cell.
-struct TableK12 {
-    using S = StoreF16K12;
-    // step[macro][halo][loop]
-    static constexpr StepFn step[2][2][2] = {
-        {{k_cavity_step<S, COLL_MRT, false, false, false>, k_cavity_step<S, COLL_MRT, false, false, true>},
-         {k_cavity_step<S, COLL_MRT, false, true, false>, k_cavity_step<S, COLL_MRT, false, true, true>}},
-        {{k_cavity_step<S, COLL_MRT, true, false, false>, k_cavity_step<S, COLL_MRT, true, false, true>},
-         {k_cavity_step<S, COLL_MRT, true, true, false>, k_cavity_step<S, COLL_MRT, true, true, true>}}};
-    static constexpr ShellFn shell[2][2] = {
-        {k_cavity_shell<S, COLL_MRT, false, false>, k_cavity_shell<S, COLL_MRT, false, true>},
-        {k_cavity_shell<S, COLL_MRT, true, false>, k_cavity_shell<S, COLL_MRT, true, true>}};
-    static constexpr InteriorFn interior[2] = {k_cavity_interior<S, COLL_MRT, false>,
-                                               k_cavity_interior<S, COLL_MRT, true>};
-};
-
 }  // namespace
 
 
 namespace {
 
 void loopback_masks(const lbm_ctx* c, unsigned* pack, unsigned* unpack);
-
-// FP16-stored MRT on the VALU at scale 2^12: the folded-scale kernels.
-bool folds_scale(const lbm_ctx* c) {
-    return c->p.storage == LBM_STORE_F16 && c->p.collision != LBM_BGK && c->p.transform != 2 &&
-           c->scale == 4096.0f;
-}
 
 StepArgs make_args(const lbm_ctx* c) {
     StepArgs a{};
@@ -506,7 +477,6 @@ StepFn step_fn(const lbm_ctx* c, bool macro, bool loop) {
     case LBM_STORE_F32: return Table<StoreF32>::step[coll][macro][halo][loop];
     case LBM_STORE_F16:
         if (coll == COLL_MRT && c->p.transform == 2) return Table<StoreF16>::stepx[macro][halo][loop];
-        if (folds_scale(c)) return TableK12::step[macro][halo][loop];
         return Table<StoreF16>::step[coll][macro][halo][loop];
     default: return Table<StoreF64>::step[coll][macro][halo][loop];
     }
@@ -626,9 +596,7 @@ int launch_shell(lbm_ctx* c, const StepArgs& a, bool macro, bool loop) {
     ShellFn fn;
     switch (c->p.storage) {
     case LBM_STORE_F32: fn = Table<StoreF32>::shell[coll][macro][loop]; break;
-    case LBM_STORE_F16:
-        fn = folds_scale(c) ? TableK12::shell[macro][loop] : Table<StoreF16>::shell[coll][macro][loop];
-        break;
+    case LBM_STORE_F16: fn = Table<StoreF16>::shell[coll][macro][loop]; break;
     default: fn = Table<StoreF64>::shell[coll][macro][loop];
     }
     const int bx = c->block.x;
@@ -645,7 +613,7 @@ int launch_interior(lbm_ctx* c, const StepArgs& a, bool macro) {
     InteriorFn fn;
     switch (c->p.storage) {
     case LBM_STORE_F32: fn = Table<StoreF32>::interior[coll][macro]; break;
-    case LBM_STORE_F16: fn = folds_scale(c) ? TableK12::interior[macro] : Table<StoreF16>::interior[coll][macro]; break;
+    case LBM_STORE_F16: fn = Table<StoreF16>::interior[coll][macro]; break;
     default: fn = Table<StoreF64>::interior[coll][macro];
     }
     const dim3 grid((c->p.nx + c->block.x - 1) / c->block.x, (j1 - j0 + c->block.y - 1) / c->block.y, k1 - k0);

@@ -1,8 +1,8 @@
 // collide.hpp -- per-cell device arithmetic of the D3Q19 step: moments
-// (macro), equilibria, BGK and MRT relaxation, and the population storage
-// formats.  Everything here is unrolled at compile time over the lattice
-// tables of lattice.hpp, so zero coefficients cost nothing and +-1
-// coefficients are plain adds.
+// (macro), the collision (MRT, BGK, with and without a body force), the
+// temperature's collision, and the population storage formats.  Everything
+// here is unrolled at compile time over the lattice tables of lattice.hpp, so
+// zero coefficients cost nothing and +-1 coefficients are plain adds.
 //
 // Two arithmetic spaces:
 //   absolute  (SHIFT = false): registers hold f itself.  FP64 storage uses
@@ -40,34 +40,35 @@ __device__ __forceinline__ R mac(R acc, R x) {
 }
 
 // ---- storage formats ----------------------------------------------------------
+// Registers hold populations in stored units: FP64 f itself, FP32 f - w, FP16
+// (f - w) * 2^k as FP32.  The collision is linear in the populations apart from
+// the velocity (a ratio) and rho = 1 + drho, so it runs in those units and only
+// these two need the scale: no population is scaled on load or store, and a
+// power-of-two scale changes no bit of the result.
 // Stores are non-temporal: the next step reads the written lattice only after
 // the whole sweep, so caching the lines on the way out buys nothing (measured
 // 2-4% faster at 256^3).
-// Every st() takes a 32-bit random word; only the FP16 format uses it.
+// Every cvt() and st() takes a 32-bit random word; only the FP16 format uses it.
 struct StoreF64 {
-    static constexpr int FOLD_LOG2 = 0;  // the store scale the MRT inverse folds in (0: none)
     using T = double;
     using Real = double;
     static constexpr bool SHIFT = false;
+    static constexpr bool SCALED = false;
     static constexpr bool RANDOM = false;
     static constexpr int BYTES = 8;
-    __device__ __forceinline__ static Real val(T v, float) { return v; }
-    __device__ __forceinline__ static Real ld(const T* p, float) { return *p; }
-    __device__ __forceinline__ static T cvt(Real v, float, unsigned) { return v; }
-    __device__ __forceinline__ static void st(T* p, Real v, float, unsigned) { __builtin_nontemporal_store(v, p); }
+    __device__ __forceinline__ static Real val(T v) { return v; }
+    __device__ __forceinline__ static T cvt(Real v, unsigned) { return v; }
 };
 
 struct StoreF32 {
-    static constexpr int FOLD_LOG2 = 0;  // the store scale the MRT inverse folds in (0: none)
     using T = float;
     using Real = float;
     static constexpr bool SHIFT = true;
+    static constexpr bool SCALED = false;
     static constexpr bool RANDOM = false;
     static constexpr int BYTES = 4;
-    __device__ __forceinline__ static Real val(T v, float) { return v; }
-    __device__ __forceinline__ static Real ld(const T* p, float) { return *p; }
-    __device__ __forceinline__ static T cvt(Real v, float, unsigned) { return v; }
-    __device__ __forceinline__ static void st(T* p, Real v, float, unsigned) { __builtin_nontemporal_store(v, p); }
+    __device__ __forceinline__ static Real val(T v) { return v; }
+    __device__ __forceinline__ static T cvt(Real v, unsigned) { return v; }
 };
 
 // FP32 -> IEEE binary16 with stochastic rounding, on gfx950's conversion
@@ -97,38 +98,24 @@ __device__ __forceinline__ unsigned mix32(unsigned x) {
 // IEEE binary16 holding (f - w) * 2^k.  The scale is an exact power of two,
 // so scaling adds no rounding; the store rounds stochastically.
 struct StoreF16 {
-    static constexpr int FOLD_LOG2 = 0;  // the store scale the MRT inverse folds in (0: none)
     using T = _Float16;
     using Real = float;
     static constexpr bool SHIFT = true;
+    static constexpr bool SCALED = true;
     static constexpr bool RANDOM = true;
     static constexpr int BYTES = 2;
-    __device__ __forceinline__ static Real val(T v, float inv_scale) {
-        // fma with +0 rather than a product: one mixed-precision fma
-        // (v_fma_mix_f32) instead of a conversion and a multiply; the value
-        // is the same (the scale is a power of two)
-        return __builtin_fmaf(static_cast<float>(v), inv_scale, 0.0f);
-    }
-    __device__ __forceinline__ static Real ld(const T* p, float inv_scale) { return val(*p, inv_scale); }
-    // the stored value: v scaled, rounded stochastically to FP16
-    __device__ __forceinline__ static T cvt(Real v, float scale, unsigned rnd) {
-        return to_half_stochastic(v * scale, rnd);
-    }
-    __device__ __forceinline__ static void st(T* p, Real v, float scale, unsigned rnd) {
-        __builtin_nontemporal_store(cvt(v, scale, rnd), p);
-    }
+    __device__ __forceinline__ static Real val(T v) { return static_cast<float>(v); }
+    __device__ __forceinline__ static T cvt(Real v, unsigned rnd) { return to_half_stochastic(v, rnd); }
 };
 
-// FP16 storage at the default scale 2^12 with the scale folded into the MRT
-// inverse transform's coefficients (exact: a power of two), so the store
-// converts without a multiply; the bits equal StoreF16's at scale 2^12.
-struct StoreF16K12 : StoreF16 {
-    static constexpr int FOLD_LOG2 = 12;
-    __device__ __forceinline__ static T cvt(Real v, float, unsigned rnd) { return to_half_stochastic(v, rnd); }
-    __device__ __forceinline__ static void st(T* p, Real v, float scale, unsigned rnd) {
-        __builtin_nontemporal_store(cvt(v, scale, rnd), p);
-    }
-};
+template <class S>
+__device__ __forceinline__ typename S::Real ld(const typename S::T* p) {
+    return S::val(*p);
+}
+template <class S>
+__device__ __forceinline__ void st(typename S::T* p, typename S::Real v, unsigned rnd) {
+    __builtin_nontemporal_store(S::cvt(v, rnd), p);
+}
 
 // Random words for the stores of cell c at step `seed`: one avalanche hash
 // per cell, then a Weyl step per population.  Each word is uniform over cells
@@ -151,61 +138,226 @@ __device__ __forceinline__ unsigned store_random(unsigned h) {
 }
 
 // ---- macroscopic moments (macro.f90:6-25) ---------------------------------------
-// Sums run a = 0..18 in order, as the reference accumulates them.
-template <class R, bool SHIFT>
+template <class R>
 struct Moments {
-    R rho;   // density
-    R drho;  // rho - 1 (shifted space only; absolute space leaves it unused)
+    R rho;       // density
+    R sum;       // sum of the populations, in stored units: rho, or (rho - 1) * 2^k
+    R j[3];      // sum of e_a f_a, in stored units
     R u, v, w;
 };
 
-template <class R, bool SHIFT>
-__device__ __forceinline__ Moments<R, SHIFT> moments(const R f[Q]) {
-    R s = f[0], jx = R(-0.0), jy = R(-0.0), jz = R(-0.0);
-    sfor<Q - 1>([&](auto am1) {
-        constexpr int a = decltype(am1)::value + 1;
-        s = s + f[a];
-        if constexpr (EX[a] != 0) jx = mac<EX[a]>(jx, f[a]);
-        if constexpr (EY[a] != 0) jy = mac<EY[a]>(jy, f[a]);
-        if constexpr (EZ[a] != 0) jz = mac<EZ[a]>(jz, f[a]);
-    });
-    Moments<R, SHIFT> m;
-    if constexpr (SHIFT) {
-        m.drho = s;
-        m.rho = R(1) + s;
-    } else {
-        m.rho = s;
-        m.drho = s - R(1);
-    }
-    m.u = jx / m.rho;
-    m.v = jy / m.rho;
-    m.w = jz / m.rho;
+__device__ __forceinline__ float rcp_near(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double rcp_near(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// a / b given r = rcp_near(b), within a rounding or so of the exact quotient
+// (the residual of the first product corrects it): three quotients by one rho
+// cost one reciprocal and nine multiply-adds instead of three divisions.
+template <class R>
+__device__ __forceinline__ R quotient(R a, R b, R r) {
+    const R q = a * r;
+    return fma_(fma_(-q, b, a), r, q);
+}
+
+// rho, from the sum of the populations in stored units.
+template <class S>
+__device__ __forceinline__ typename S::Real density(typename S::Real sum, float inv_scale) {
+    using R = typename S::Real;
+    if constexpr (S::SCALED) return fma_(sum, inv_scale, R(1));
+    else if constexpr (S::SHIFT) return R(1) + sum;
+    else return sum;
+}
+
+// rho - 1 in stored units.
+template <class S>
+__device__ __forceinline__ typename S::Real excess(typename S::Real sum) {
+    if constexpr (S::SHIFT) return sum;
+    else return sum - 1.0;
+}
+
+// rho as the macro fields hold it.
+template <class S>
+__device__ __forceinline__ double density_f64(typename S::Real sum, float inv_scale) {
+    if constexpr (S::SCALED) return 1.0 + double(sum * inv_scale);
+    else if constexpr (S::SHIFT) return 1.0 + double(sum);
+    else return sum;
+}
+
+// Sums of the populations and of e_a f_a from the sums and differences of
+// opposite pairs, which the collision uses again (the compiler keeps one copy).
+// No contraction here or in relax(): every kernel that updates a cell makes
+// the same operations, so they agree bit for bit.
+template <class R>
+__device__ __forceinline__ void population_sums(const R f[Q], R& sum, R j[3]) {
+#pragma clang fp contract(off)
+    const R axis = ((f[1] + f[2]) + (f[3] + f[4])) + (f[5] + f[6]);
+    const R diag = (((f[7] + f[10]) + (f[8] + f[9])) + ((f[11] + f[14]) + (f[12] + f[13]))) +
+                   ((f[15] + f[18]) + (f[16] + f[17]));
+    sum = (f[0] + axis) + diag;
+    const R xy1 = f[7] - f[10], xy2 = f[8] - f[9];      // (1,1,0), (-1,1,0)
+    const R xz1 = f[11] - f[14], xz2 = f[12] - f[13];   // (1,0,1), (-1,0,1)
+    const R yz1 = f[15] - f[18], yz2 = f[16] - f[17];   // (0,1,1), (0,-1,1)
+    j[0] = (f[1] - f[2]) + ((xy1 - xy2) + (xz1 - xz2));
+    j[1] = (f[3] - f[4]) + ((xy1 + xy2) + (yz1 - yz2));
+    j[2] = (f[5] - f[6]) + ((xz1 + xz2) + (yz1 + yz2));
+}
+
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ Moments<R> moments(const R f[Q], float inv_scale) {
+#pragma clang fp contract(off)
+    Moments<R> m;
+    population_sums(f, m.sum, m.j);
+    m.rho = density<S>(m.sum, inv_scale);
+    const R r = rcp_near(m.rho), k = S::SCALED ? R(inv_scale) : R(1);
+    m.u = quotient(m.j[0] * k, m.rho, r);
+    m.v = quotient(m.j[1] * k, m.rho, r);
+    m.w = quotient(m.j[2] * k, m.rho, r);
     return m;
 }
 
-// ---- BGK (collision.f90:192-198, feq of initial.f90:63-73) ---------------------------
-// f_post = f - (f - feq)/tau.  In shifted space the w-part of feq is dropped:
-// geq = w (drho + rho (3 e.u + 4.5 (e.u)^2 - 1.5 u.u)).
-template <class R, bool SHIFT>
-__device__ __forceinline__ void collide_bgk(R f[Q], const Moments<R, SHIFT>& m, R omega) {
-    const R us2 = m.u * m.u + m.v * m.v + m.w * m.w;
-    sfor<Q>([&](auto A) {
-        constexpr int a = decltype(A)::value;
-        R un = R(-0.0);
-        if constexpr (EX[a] != 0) un = mac<EX[a]>(un, m.u);
-        if constexpr (EY[a] != 0) un = mac<EY[a]>(un, m.v);
-        if constexpr (EZ[a] != 0) un = mac<EZ[a]>(un, m.w);
-        constexpr R wa = R(weight(a));
-        R feq;
-        if constexpr (SHIFT)
-            feq = wa * (m.drho + m.rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
-        else
-            feq = m.rho * wa * (R(1) + R(3) * un + R(4.5) * un * un - R(1.5) * us2);
-        f[a] = f[a] - omega * (f[a] - feq);
+// Moments of a cell whose fields are given (the equilibrium starts).
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ Moments<R> moments_of(double rho, double u, double v, double w, float scale) {
+    Moments<R> m;
+    m.rho = R(rho);
+    m.sum = S::SHIFT ? R((rho - 1.0) * scale) : R(rho);
+    m.j[0] = R(rho * u * scale);
+    m.j[1] = R(rho * v * scale);
+    m.j[2] = R(rho * w * scale);
+    m.u = R(u);
+    m.v = R(v);
+    m.w = R(w);
+    return m;
+}
+
+// ---- the collision (collision.f90:15-202, evolution_f.F90:58-129) --------------------
+// The reference relaxes 19 moments m = M f.  Its rates are Snu on every even
+// moment that is not conserved (e, eps, the stress rows 9..15), Sq on every odd
+// one (q, m16..m18) and 0 on rho and j, and its equilibrium moments are those
+// of the quadratic equilibrium f_eq (apart from row 12, below).  A space of
+// moments that relaxes at one rate needs no basis: the even moments are the
+// sums s = f_a + f_abar of opposite pairs (and f_0), the odd ones the
+// differences d = f_a - f_abar (j, which must not change, is seen to below).
+// So M, the rates and M^-1 are exactly
+//   f_a, f_abar  +=  Snu/2 (s_eq - s)  +-  Sq/2 (d_eq - d).
+// BGK is the case Sq = Snu = 1/tau.  Against the 19 x 19 transforms the step
+// kernel went from 533 to 389 VALU instructions in FP32 and from 646 to 509 in
+// FP16, which is bound by their issue: 266 -> 249 ms for 800 steps of 256^3
+// with the fields copied out (about 255 -> 234 us a step).  FP64 and FP32,
+// bound by memory, kept their time.
+// The form updates f by the change alone, so a population's rounding error is
+// that of the change and two sums instead of that of ten moments: after 300
+// FP32 steps at 256^3 the velocity is 1e-7 off FP64 where it was 4e-6.
+// Mass and momentum are kept by construction, not by coefficients that cancel:
+// f_0 loses what the pair sums gain, and the differences along the axes are
+// what the diagonals leave of the momentum's gain.  Rounded weights
+// (1/18, 1/36, 1/6) do not add up to 1, and in FP32 their few 1e-8 per step
+// act on every cell the same way: mass drifted by 2.4e-7 in 20000 steps.  The
+// FP64 path is compared with the reference's program, whose rounded M^-1 sums
+// to 1 - 2^-54 over a population's column of rho: it loses that share of rho
+// per step (1.1e-12 in 20000 steps), and so does f_0 here.
+//   base  Snu times the sum (rho or its excess), in stored units
+//   C     Snu j: even part    w (base - 3/2 u.C + 9/2 (e.u)(e.C)) - Snu/2 s
+//   B2    Sq j / 12: odd part of the diagonals   e.B2 - Sq/2 d
+//   gain  half the momentum the collision adds (the body force), if any
+//   k12   row 12's equilibrium of the cavity code lacks rho (collision.f90:85;
+//         evolution_f.F90:75 has it): Snu (rho - 1)(v^2 - w^2) / 2 along row 12
+//         of M^-1, which is -+1/12 on the y / z axes, +-1/24 on the xy / xz
+//         diagonals
+constexpr double REFERENCE_LOSS = 0x1p-54;
+template <bool ROW12, bool GAIN, class R>
+__device__ __forceinline__ void relax(R f[Q], R sum, R base, const R (&C)[3], const R (&B2)[3], const R (&gain)[3], R u, R v,
+                                      R w, R hs, R hd, R k12) {
+#pragma clang fp contract(off)
+    const R bb = fma_(R(-1.5), fma_(u, C[0], fma_(v, C[1], w * C[2])), base);
+    R bax[3], bdi[3];  // the part common to a direction class: axes x, y, z; planes xy, xz, yz
+    bax[0] = bax[1] = bax[2] = R(1.0 / 18.0) * bb;
+    bdi[0] = bdi[1] = bdi[2] = R(1.0 / 36.0) * bb;
+    if constexpr (ROW12) {
+        bax[1] = fma_(R(-1.0 / 12.0), k12, bax[1]);
+        bax[2] = fma_(R(1.0 / 12.0), k12, bax[2]);
+        bdi[0] = fma_(R(1.0 / 24.0), k12, bdi[0]);
+        bdi[1] = fma_(R(-1.0 / 24.0), k12, bdi[1]);
+    }
+    const R U[3] = {u, v, w};
+    const R C1[3] = {R(0.25) * C[0], R(0.25) * C[1], R(0.25) * C[2]};
+    const R C2[3] = {R(0.125) * C[0], R(0.125) * C[1], R(0.125) * C[2]};
+    R x[NPAIR], y[NPAIR];  // what both members of a pair gain, and what the first gains over the second
+    sfor<NPAIR>([&](auto P) {
+        constexpr int p = decltype(P)::value, a = PAIR_A[p], b = OPP[a];
+        constexpr int ex = EX[a], ey = EY[a], ez = EZ[a];
+        const R s = f[a] + f[b];
+        if constexpr (a < 7) {
+            constexpr int d = ex ? 0 : (ey ? 1 : 2);
+            x[p] = fma_(-hs, s, fma_(U[d], C1[d], bax[d]));
+        } else {
+            constexpr int d = ex ? 0 : 1, e = ez ? 2 : 1, pl = ez == 0 ? 0 : (ey == 0 ? 1 : 2);
+            constexpr bool plus = (ex + ey + ez) == 2;  // else (-1 on d, +1 on e)
+            const R eu = plus ? U[e] + U[d] : U[e] - U[d];
+            const R ec = plus ? C2[e] + C2[d] : C2[e] - C2[d];
+            const R eb = plus ? B2[e] + B2[d] : B2[e] - B2[d];
+            x[p] = fma_(-hs, s, fma_(eu, ec, bdi[pl]));
+            y[p] = fma_(-hd, f[a] - f[b], eb);
+        }
+    });
+    // pairs 3..8: (1,1,0), (-1,1,0), (1,0,1), (-1,0,1), (0,1,1), (0,-1,1)
+    static_assert(PAIR_A[3] == 7 && PAIR_A[4] == 8 && PAIR_A[5] == 11 && PAIR_A[6] == 12 && PAIR_A[7] == 15 &&
+                  PAIR_A[8] == 16, "pair order");
+    y[0] = (y[4] - y[3]) + (y[6] - y[5]);
+    y[1] = (y[8] - y[7]) - (y[3] + y[4]);
+    y[2] = -(y[5] + y[6]) - (y[7] + y[8]);
+    if constexpr (GAIN)
+        for (int d = 0; d < 3; ++d) y[d] = y[d] + gain[d];
+    R even = (((x[0] + x[1]) + x[2]) + ((x[3] + x[4]) + (x[5] + x[6]))) + (x[7] + x[8]);
+    if constexpr (sizeof(R) == 8) even = fma_(R(0.5 * REFERENCE_LOSS), sum, even);
+    f[0] = fma_(R(-2), even, f[0]);
+    sfor<NPAIR>([&](auto P) {
+        constexpr int p = decltype(P)::value, a = PAIR_A[p], b = OPP[a];
+        f[a] = (f[a] + x[p]) + y[p];
+        f[b] = (f[b] + x[p]) - y[p];
     });
 }
 
-// ---- MRT (collision.f90:15-202) ------------------------------------------------------
+// One isothermal collision with rates snu, sq (BGK: both 1/tau, no row 12).
+template <class S, bool ROW12, class R = typename S::Real>
+__device__ __forceinline__ void collide_flow(R f[Q], const Moments<R>& m, R snu, R sq, R row12) {
+#pragma clang fp contract(off)
+    const R b2 = R(1.0 / 12.0) * sq;
+    const R C[3] = {snu * m.j[0], snu * m.j[1], snu * m.j[2]};
+    const R B2[3] = {b2 * m.j[0], b2 * m.j[1], b2 * m.j[2]};
+    R k12 = R(0);
+    if constexpr (ROW12) k12 = (row12 * excess<S>(m.sum)) * fma_(m.v, m.v, -(m.w * m.w));
+    relax<ROW12, false>(f, m.sum, snu * m.sum, C, B2, C, m.u, m.v, m.w, R(0.5) * snu, R(0.5) * sq, k12);
+}
+
+// The collision with the Guo source (evolution_f.F90:58-129): source moments
+// scaled by 1 - s/2, momentum (rate 0) by 1, so it gains F.  m.j, m.u hold
+// rho u = j + F0/2 with the force F0 of the last collision.  The source joins
+// the equilibrium: C = Snu rho u + (2 - Snu) F, B = Sq rho u + (1 - Sq/2) F.
+// The rate of the momentum rows of M^-1 (e / 10) is 0, not Sq: what Sq would
+// take from them, Sq/2 (F - F0), is given back to every population.  Forces
+// in stored units.
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ void collide_forced(R f[Q], const Moments<R>& m, const R (&F)[3], const R (&F0)[3], R snu,
+                                               R sq) {
+#pragma clang fp contract(off)
+    const R kc = R(2) - snu, kb = fma_(R(-0.5), sq, R(1)), kg = R(0.05) * sq;
+    R C[3], B2[3], gain[3];
+    for (int d = 0; d < 3; ++d) {
+        C[d] = fma_(snu, m.j[d], kc * F[d]);
+        B2[d] = fma_(R(1.0 / 12.0), fma_(sq, m.j[d], kb * F[d]), kg * (F[d] - F0[d]));
+        gain[d] = R(0.5) * F[d];
+    }
+    relax<false, true>(f, m.sum, snu * m.sum, C, B2, gain, m.u, m.v, m.w, R(0.5) * snu, R(0.5) * sq, R(0));
+}
+
+// ---- moment transforms -----------------------------------------------------------------
+// For the matrix-core form of the FP16 step and the refill of uncovered nodes,
+// which replaces moments.
 // m = M f computed from the opposite-pair sums s_p = f_a + f_abar (even rows)
 // and differences d_p = f_a - f_abar (odd rows); f_post = M^-1 m* likewise
 // from even/odd partial sums E, O with f_a = E + O, f_abar = E - O.
@@ -232,17 +384,14 @@ __device__ __forceinline__ void mrt_forward(const R f[Q], R m[Q]) {
     });
 }
 
-// FOLD: the result times 2^FOLD, the scale folded into the coefficients
-// (exact for a power of two: the same bits as scaling the result).
-template <class R, int FOLD = 0>
+template <class R>
 __device__ __forceinline__ void mrt_inverse(const R m[Q], R f[Q]) {
-    constexpr double SC = double(1LL << FOLD);
     {
         R acc = R(-0.0);
         sfor<Q>([&](auto K) {
             constexpr int k = decltype(K)::value;
             constexpr int c = basis(k, 0);
-            if constexpr (c != 0) acc = acc + R(double(c) / double(row_norm2(k)) * SC) * m[k];
+            if constexpr (c != 0) acc = acc + R(double(c) / double(row_norm2(k))) * m[k];
         });
         f[0] = acc;
     }
@@ -253,7 +402,7 @@ __device__ __forceinline__ void mrt_inverse(const R m[Q], R f[Q]) {
             constexpr int k = decltype(K)::value;
             constexpr int c = basis(k, a);
             if constexpr (c != 0) {
-                constexpr R coef = R(double(c) / double(row_norm2(k)) * SC);
+                constexpr R coef = R(double(c) / double(row_norm2(k)));
                 if constexpr (row_is_odd(k)) o = o + coef * m[k];
                 else e = e + coef * m[k];
             }
@@ -263,23 +412,16 @@ __device__ __forceinline__ void mrt_inverse(const R m[Q], R f[Q]) {
     });
 }
 
-// Equilibrium moments (collision.f90:73-91).  In shifted space M w =
-// (1, -11, 3, 0, ...) is subtracted, leaving drho in rows 0..2.
+// Equilibrium moments (collision.f90:73-91) of rho = 1 + drho with M w =
+// (1, -11, 3, 0, ...) subtracted, which leaves drho in rows 0..2.
 // meq12_rho selects the thermal form -rho/2 (v^2 - w^2) (evolution_f.F90:75);
 // the cavity form has no rho (collision.f90:85).
-template <class R, bool SHIFT>
-__device__ __forceinline__ void mrt_meq(const Moments<R, SHIFT>& q, bool meq12_rho, R meq[Q]) {
-    const R rho = q.rho, u = q.u, v = q.v, w = q.w;
+template <class R>
+__device__ __forceinline__ void mrt_meq(R rho, R drho, R u, R v, R w, bool meq12_rho, R meq[Q]) {
     const R us2 = u * u + v * v + w * w;
-    if constexpr (SHIFT) {
-        meq[0] = q.drho;
-        meq[1] = R(-11) * q.drho + R(19) * rho * us2;
-        meq[2] = R(3) * q.drho - R(11.0 / 2.0) * rho * us2;
-    } else {
-        meq[0] = rho;
-        meq[1] = rho * (R(-11) + R(19) * us2);
-        meq[2] = rho * (R(3) - R(11.0 / 2.0) * us2);
-    }
+    meq[0] = drho;
+    meq[1] = R(-11) * drho + R(19) * rho * us2;
+    meq[2] = R(3) * drho - R(11.0 / 2.0) * rho * us2;
     meq[3] = rho * u;
     meq[4] = R(-2.0 / 3.0) * rho * u;
     meq[5] = rho * v;
@@ -305,92 +447,13 @@ constexpr int rate_kind() {
     return (k == 0 || k == 3 || k == 5 || k == 7) ? 0 : ((k == 4 || k == 6 || k == 8 || k >= 16) ? 2 : 1);
 }
 
-template <class R, bool SHIFT, int FOLD = 0>
-__device__ __forceinline__ void collide_mrt(R f[Q], const Moments<R, SHIFT>& q, R snu, R sq,
-                                            bool meq12_rho) {
-    R m[Q], meq[Q];
-    mrt_forward(f, m);
-    mrt_meq(q, meq12_rho, meq);
-    sfor<Q>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        constexpr int kind = rate_kind<k>();
-        if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]);
-        else if constexpr (kind == 2) m[k] = m[k] - sq * (m[k] - meq[k]);
-    });
-    mrt_inverse<R, FOLD>(m, f);
-}
-
-}  // namespace lbm
-
-// ---- buoyancy-driven flow (evolution_f.F90, evolution_g.F90) -------------------------
-namespace lbm {
-
-// MRT with the Guo source in moment space (evolution_f.F90:58-129):
-// m* = m - s (m - meq) + (1 - s/2) S, meq in the thermal form (meq(12) with rho).
-// R = double, SHIFT = false: absolute FP64 arithmetic in the reference's
-// operation order.  SHIFT = true: f holds f - w and rho = 1 + drho; M w =
-// (1, -11, 3, 0, ...) leaves drho in meq rows 0..2 (the relaxation and the
-// source are unchanged, being differences and forces).
-template <class R, bool SHIFT>
-__device__ __forceinline__ void collide_mrt_forced(R f[Q], R rho, R drho, R u, R v, R w, R Fx, R Fy, R Fz,
-                                                   R snu, R sq) {
-    R m[Q], meq[Q], S[Q];
-    mrt_forward(f, m);
-    const R us2 = u * u + v * v + w * w;
-    if constexpr (SHIFT) {
-        meq[0] = drho;
-        meq[1] = R(-11.0) * drho + R(19.0) * rho * us2;
-        meq[2] = R(3.0) * drho - R(11.0 / 2.0) * rho * us2;
-    } else {
-        meq[0] = rho;
-        meq[1] = R(-11.0) * rho + R(19.0) * rho * us2;
-        meq[2] = R(3.0) * rho - R(11.0 / 2.0) * rho * us2;
-    }
-    meq[3] = rho * u;
-    meq[4] = R(-2.0 / 3.0) * meq[3];
-    meq[5] = rho * v;
-    meq[6] = R(-2.0 / 3.0) * meq[5];
-    meq[7] = rho * w;
-    meq[8] = R(-2.0 / 3.0) * meq[7];
-    meq[9] = rho * (R(2.0) * u * u - v * v - w * w);
-    meq[10] = R(-0.5) * meq[9];
-    meq[11] = rho * (v * v - w * w);
-    meq[12] = R(-0.5) * meq[11];
-    meq[13] = rho * (u * v);
-    meq[14] = rho * (v * w);
-    meq[15] = rho * (w * u);
-    meq[16] = meq[17] = meq[18] = R(0.0);
-    const R uF = u * Fx + v * Fy + w * Fz;
-    S[0] = R(0.0);
-    S[1] = R(38.0) * uF;
-    S[2] = R(-11.0) * uF;
-    S[3] = Fx;
-    S[4] = R(-2.0 / 3.0) * Fx;
-    S[5] = Fy;
-    S[6] = R(-2.0 / 3.0) * Fy;
-    S[7] = Fz;
-    S[8] = R(-2.0 / 3.0) * Fz;
-    S[9] = R(4.0) * u * Fx - R(2.0) * v * Fy - R(2.0) * w * Fz;
-    S[10] = R(-2.0) * u * Fx + v * Fy + w * Fz;
-    S[11] = R(2.0) * v * Fy - R(2.0) * w * Fz;
-    S[12] = -v * Fy + w * Fz;
-    S[13] = u * Fy + v * Fx;
-    S[14] = v * Fz + w * Fy;
-    S[15] = u * Fz + w * Fx;
-    S[16] = S[17] = S[18] = R(0.0);
-    sfor<Q>([&](auto K) {
-        constexpr int k = decltype(K)::value;
-        constexpr int kind = rate_kind<k>();
-        if constexpr (kind == 0) m[k] = m[k] + S[k];
-        else if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]) + (R(1.0) - R(0.5) * snu) * S[k];
-        else m[k] = m[k] - sq * (m[k] - meq[k]) + (R(1.0) - R(0.5) * sq) * S[k];
-    });
-    mrt_inverse(m, f);
-}
-
 // D3Q7 MRT for the temperature (evolution_g.F90:1-57): n = N g,
 // neq = (T, T u, T v, T w, T paraA, 0, 0), rates (0, Qd x3, Qnu x3),
-// g_post = N^-1 n*, N^-1 = N^T diag(1/|row|^2).  g is stored unshifted.
+// g_post = N^-1 n*, N^-1 = N^T diag(1/|row|^2).  g is stored unshifted; T
+// in g's units.  (In pair form, as the flow, this would keep T in FP32 where the
+// rounded 1/7, 1/42, ... move it by 4e-8 per step, 2.8e-5 of the change of T
+// over 120 steps at 128^3; the transforms stay so that FP32 fields do not move by
+// more than their own rounding from one version to the next.)
 template <class R>
 __device__ __forceinline__ void collide_d3q7(R g[Q7], R T, R u, R v, R w, R para_a, R qd, R qnu) {
     R n[Q7];

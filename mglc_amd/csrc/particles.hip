@@ -232,8 +232,8 @@ __device__ __forceinline__ double stream_rho_avg(const PArgs& a) {
 
 // Absolute population a of a stored state at storage index c.
 template <class S>
-__device__ __forceinline__ double abs_pop(const typename S::T* buf, long long ps, long long c, int a, float inv) {
-    const double g = double(S::ld(buf + (long long)a * ps + c, inv));
+__device__ __forceinline__ double abs_pop(const typename S::T* buf, long long ps, long long c, int a) {
+    const double g = double(ld<S>(buf + (long long)a * ps + c));
     return S::SHIFT ? g + weight(a) : g;
 }
 
@@ -356,9 +356,9 @@ __device__ __forceinline__ LinkWork link_begin(const PArgs& a, const SphereNow& 
     const long long c1 = ci1 + (long long)a.px * (cj1 + (long long)a.ny * ck1);
     const long long c2 = ci2 + (long long)a.px * (cj2 + (long long)a.ny * ck2);
     w.o2 = near ? a.owner[ci2 + (long long)a.nx * (cj2 + (long long)a.ny * ck2)] : 0;
-    w.fa = abs_pop<S>(src, a.ps, c, al, a.inv_scale);
-    w.s1 = abs_pop<S>(src, a.ps, c1, near ? al : bd, a.inv_scale);
-    w.s2 = abs_pop<S>(src, a.ps, near ? c2 : c, near ? al : bd, a.inv_scale);
+    w.fa = abs_pop<S>(src, a.ps, c, al);
+    w.s1 = abs_pop<S>(src, a.ps, c1, near ? al : bd);
+    w.s2 = abs_pop<S>(src, a.ps, near ? c2 : c, near ? al : bd);
     return w;
 }
 
@@ -390,7 +390,7 @@ __device__ __forceinline__ void link_end(const PArgs& a, const SphereNow& sp, co
               6.0 * weight(al) * rho_avg * iq * i12 * eu;
     }
     const long long cs = w.c + EX[al] + (long long)EY[al] * a.px + (long long)EZ[al] * a.pxy;
-    S::st(src_w + (long long)bd * a.ps + cs, S::SHIFT ? R(val - weight(bd)) : R(val), a.scale, 0u);
+    st<S>(src_w + (long long)bd * a.ps + cs, S::SHIFT ? R(val - weight(bd)) : R(val), 0u);
     const double dFx = (EX[al] - ux - wx) * fa - (EX[bd] - ux - wx) * val;
     const double dFy = (EY[al] - uy - wy) * fa - (EY[bd] - uy - wy) * val;
     const double dFz = (EZ[al] - uz - wz) * fa - (EZ[bd] - uz - wz) * val;
@@ -616,15 +616,15 @@ __device__ __forceinline__ void pull_node(const PArgs& a, int i, int j, int k, t
         constexpr int bd = decltype(B)::value;
         constexpr int ex = EX[bd], ey = EY[bd], ez = EZ[bd];
         if constexpr (bd == 0) {
-            f[0] = S::ld(src + c, a.inv_scale);
+            f[0] = ld<S>(src + c);
         } else {
             bool in = true;
             if constexpr (ex != 0) in = in && (unsigned)(i - ex) < (unsigned)a.nx;
             if constexpr (ey != 0) in = in && (unsigned)(j - ey) < (unsigned)a.ny;
             if constexpr (ez != 0) in = in && (unsigned)(k - ez) < (unsigned)a.nz;
             const long long off = (long long)ex + (long long)ey * a.px + (long long)ez * a.pxy;
-            f[bd] = in ? S::ld(src + (long long)bd * a.ps + (c - off), a.inv_scale)
-                       : S::ld(src + (long long)OPP[bd] * a.ps + c, a.inv_scale);
+            f[bd] = in ? ld<S>(src + (long long)bd * a.ps + (c - off))
+                       : ld<S>(src + (long long)OPP[bd] * a.ps + c);
         }
     });
 }
@@ -636,8 +636,8 @@ __device__ __forceinline__ double pulled_rho(const PArgs& a, int i, int j, int k
     using R = typename S::Real;
     R f[Q];
     pull_node<S>(a, i, j, k, f);
-    const Moments<R, S::SHIFT> mo = moments<R, S::SHIFT>(f);
-    return S::SHIFT ? 1.0 + double(mo.drho) : double(mo.rho);
+    const Moments<R> mo = moments<S>(f, a.inv_scale);
+    return density_f64<S>(mo.sum, a.inv_scale);
 }
 
 // Every node: the pulls (pull_node), then macro (fluid.F90:164-184) on fluid
@@ -659,9 +659,9 @@ __global__ __launch_bounds__(256) void k_particle_step(const PArgs a) {
         const int c = i + a.px * (j + a.ny * k);
         R f[Q];
         pull_node<S>(a, i, j, k, f);
-        const Moments<R, S::SHIFT> mo = moments<R, S::SHIFT>(f);
+        const Moments<R> mo = moments<S>(f, a.inv_scale);
         if (a.owner[m] < 0) {
-            const double rho = S::SHIFT ? 1.0 + double(mo.drho) : double(mo.rho);
+            const double rho = density_f64<S>(mo.sum, a.inv_scale);
             rho_fluid = rho;
             n_fluid = 1.0;
             if constexpr (MACRO) {  // other steps: rho goes into the block sums only
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(256) void k_particle_step(const PArgs a) {
         T* __restrict__ dst = static_cast<T*>(a.dst);
         sfor<Q>([&](auto B) {
             constexpr int bd = decltype(B)::value;
-            S::st(dst + (long long)bd * a.ps + c, f[bd], a.scale, 0u);
+            st<S>(dst + (long long)bd * a.ps + c, f[bd], 0u);
         });
     }
     // the block's sums of rho and count over its fluid nodes (fixed order)
@@ -713,7 +713,7 @@ __device__ __forceinline__ double streamed_pop_at(const PArgs& a, const typename
         idx = in_box(a, si, sj, sk) ? (long long)al * a.ps + si + (long long)a.px * (sj + (long long)a.ny * sk)
                                     : (long long)OPP[al] * a.ps + c;
     }
-    const double g = double(S::ld(src + idx, a.inv_scale));
+    const double g = double(ld<S>(src + idx));
     return S::SHIFT ? g + weight(al) : g;
 }
 
@@ -992,16 +992,13 @@ __global__ __launch_bounds__(256) void k_particle_init_fields(const PArgs a) {
         const double fe = weight(bd) * a.rho0;
         f[bd] = S::SHIFT ? R(fe - weight(bd)) : R(fe);
     });
-    Moments<R, S::SHIFT> mo;
-    mo.rho = R(a.rho0);
-    mo.drho = R(a.rho0 - 1.0);
-    mo.u = mo.v = mo.w = R(0);
+    const Moments<R> mo = moments_of<S>(a.rho0, 0.0, 0.0, 0.0, a.scale);
     collide<S, COLL>(f, mo, a);
     const int c = i + a.px * (j + a.ny * k);
     T* __restrict__ dst = static_cast<T*>(a.dst);
     sfor<Q>([&](auto B) {
         constexpr int bd = decltype(B)::value;
-        S::st(dst + (long long)bd * a.ps + c, f[bd], a.scale, 0u);
+        st<S>(dst + (long long)bd * a.ps + c, f[bd], 0u);
     });
 }
 
@@ -1075,8 +1072,8 @@ __device__ __forceinline__ void refill_node(const PArgs& a, int i, int j, int k,
     mrt_inverse(mm, fr);
     R f[Q];
     for (int al = 0; al < Q; ++al) f[al] = S::SHIFT ? R(fr[al] - weight(al)) : R(fr[al]);
-    const Moments<R, S::SHIFT> mo = moments<R, S::SHIFT>(f);
-    const double rho_new = S::SHIFT ? 1.0 + double(mo.drho) : double(mo.rho);
+    const Moments<R> mo = moments<S>(f, a.inv_scale);
+    const double rho_new = density_f64<S>(mo.sum, a.inv_scale);
     atomicAdd(&a.chain->ref, to_fix(rho_new - a.rho_solid));
     a.rho[m] = rho_new;
     a.u[m] = double(mo.u);
@@ -1085,7 +1082,7 @@ __device__ __forceinline__ void refill_node(const PArgs& a, int i, int j, int k,
     collide<S, COLL>(f, mo, a);
     const long long c = i + (long long)a.px * (j + (long long)a.ny * k);
     T* __restrict__ dst = static_cast<T*>(a.dst);
-    for (int al = 0; al < Q; ++al) S::st(dst + (long long)al * a.ps + c, f[al], a.scale, 0u);
+    for (int al = 0; al < Q; ++al) st<S>(dst + (long long)al * a.ps + c, f[al], 0u);
 }
 
 // The uncovered nodes of each sphere, appended to the refill list.  The

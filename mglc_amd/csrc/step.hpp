@@ -52,17 +52,13 @@ struct NoPost {
 enum { COLL_MRT = 0, COLL_BGK = 1 };
 
 template <class S, int COLL, class Args>
-__device__ __forceinline__ void collide(typename S::Real f[Q],
-                                        const Moments<typename S::Real, S::SHIFT>& q,
-                                        const Args& a) {
+__device__ __forceinline__ void collide(typename S::Real f[Q], const Moments<typename S::Real>& q, const Args& a) {
     using R = typename S::Real;
-    if constexpr (COLL == COLL_BGK) {
-        static_assert(S::FOLD_LOG2 == 0, "a folded store scale is an MRT form");
-        collide_bgk<R, S::SHIFT>(f, q, R(a.snu));
-    } else {
-        // f returned times 2^FOLD_LOG2 when the store folds its scale in
-        collide_mrt<R, S::SHIFT, S::FOLD_LOG2>(f, q, R(a.snu), R(a.sq), a.meq12_rho != 0);
-    }
+    const R snu = R(a.snu);
+    if constexpr (COLL == COLL_BGK)
+        collide_flow<S, false>(f, q, snu, snu, R(0));
+    else
+        collide_flow<S, true>(f, q, snu, R(a.sq), a.meq12_rho ? R(0) : R(0.5) * snu);
 }
 
 // Value pulled from outside the domain for population al at cell (i, j, k):
@@ -106,17 +102,18 @@ __device__ __forceinline__ typename S::Real pull_outside(const Args& a, const ty
                 idx = a.hoff[fz] + (long long)cross_slot(fz, al, -1) * a.nx * a.ny + (i - ex) +
                       (long long)a.nx * (j - ey);
             }
-            return S::ld(h + idx, a.inv_scale);
+            return ld<S>(h + idx);
         }
         lid = top && !((a.halo_faces >> LBM_FACE_ZP) & 1);
     }
-    R val = S::ld(src + (long long)OPP[al] * a.ps + c, a.inv_scale);
+    R val = ld<S>(src + (long long)OPP[al] * a.ps + c);
     if constexpr (ez == -1 && ex != 0) {
         // moving lid (bounce_back.f90:77-78): f(14) = f_post(11) - rho/6 U0,
         // f(13) = f_post(12) - rho/6 (-U0); the lid is applied last, so it
         // wins over the side walls on these two populations.
         if (lid) {
-            const double t = rho_lid / 6.0 * a.u_lid;
+            double t = rho_lid / 6.0 * a.u_lid;
+            if constexpr (S::SCALED) t *= double(a.scale);
             val = (ex > 0) ? R(double(val) + t) : R(double(val) - t);
         }
     }
@@ -142,33 +139,29 @@ __device__ __forceinline__ void mfma_cell(const Args& a, const _Float16* src, _F
     });
     if (i == 0 || i == a.nx - 1) {
         // an x-face lane: halfway bounce-back or the halo (no lid here: not
-        // the top layer), back in the stored form (exact: a power-of-two scale)
+        // the top layer), back in the stored form (exact)
         sfor<Q>([&](auto A) {
             constexpr int al = decltype(A)::value;
             if constexpr (EX[al] != 0) {
                 if ((unsigned)(i - EX[al]) >= (unsigned)a.nx)
-                    h[al] = (_Float16)(pull_outside<S, al, HALO>(a, src, i, j, k, c, false, 0.0) * a.scale);
+                    h[al] = (_Float16)pull_outside<S, al, HALO>(a, src, i, j, k, c, false, 0.0);
             }
         });
     }
     const int lane = __lane_id();
     float m[Q];
     mrt_forward_mfma(h, m, lane);
-    Moments<float, true> q;
-    q.drho = m[0] * a.inv_scale;
-    q.rho = 1.0f + q.drho;
-    q.u = m[3] * a.inv_scale / q.rho;
-    q.v = m[5] * a.inv_scale / q.rho;
-    q.w = m[7] * a.inv_scale / q.rho;
+    const float drho = m[0] * a.inv_scale, rho = 1.0f + drho;
+    const float u = m[3] * a.inv_scale / rho, v = m[5] * a.inv_scale / rho, w = m[7] * a.inv_scale / rho;
     if constexpr (MACRO) {
         const long long mm = i + (long long)a.nx * (j + (long long)a.ny * k);
-        a.rho[mm] = 1.0 + double(q.drho);
-        a.u[mm] = double(q.u);
-        a.v[mm] = double(q.v);
-        a.w[mm] = double(q.w);
+        a.rho[mm] = 1.0 + double(drho);
+        a.u[mm] = double(u);
+        a.v[mm] = double(v);
+        a.w[mm] = double(w);
     }
     float meq[Q];
-    mrt_meq<float, true>(q, a.meq12_rho != 0, meq);
+    mrt_meq(rho, drho, u, v, w, a.meq12_rho != 0, meq);
     const float snu = float(a.snu), sq = float(a.sq);
     sfor<Q>([&](auto K) {
         constexpr int kk = decltype(K)::value;
@@ -232,7 +225,7 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
             if constexpr (XSEL && EX[al] != 0) {
                 if ((unsigned)(i - EX[al]) >= (unsigned)a.nx) off -= EX[al];
             }
-            f[al] = S::ld(src + ((long long)al * a.ps + c - off), a.inv_scale);
+            f[al] = ld<S>(src + ((long long)al * a.ps + c - off));
         });
         if (i == 0 || i == a.nx - 1) {
             sfor<Q>([&](auto A) {
@@ -249,7 +242,7 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
             constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
             const T* base = src + (long long)al * a.ps;
             if constexpr (ex == 0 && ey == 0 && ez == 0) {
-                f[al] = S::ld(base + c, a.inv_scale);
+                f[al] = ld<S>(base + c);
             } else {
                 bool in = true;
                 if constexpr (ex != 0) in = in && (unsigned)(i - ex) < (unsigned)a.nx;
@@ -257,7 +250,7 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
                 if constexpr (ez != 0) in = in && (unsigned)(k - ez) < (unsigned)a.nz;
                 if (in) {
                     const long long off = (long long)ex + (long long)ey * a.px + (long long)ez * a.pxy;
-                    f[al] = S::ld(base + (c - off), a.inv_scale);
+                    f[al] = ld<S>(base + (c - off));
                 } else {
                     f[al] = pull_outside<S, al, HALO>(a, src, i, j, k, c, top, rho_lid);
                 }
@@ -265,11 +258,11 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
         });
     }
 
-    const Moments<R, S::SHIFT> q = moments<R, S::SHIFT>(f);
-    if (top) a.lid_rho[lid_idx] = S::SHIFT ? 1.0 + double(q.drho) : double(q.rho);
+    const Moments<R> q = moments<S>(f, a.inv_scale);
+    if (top) a.lid_rho[lid_idx] = density_f64<S>(q.sum, a.inv_scale);
     if constexpr (MACRO) {
         const long long m = i + (long long)a.nx * (j + (long long)a.ny * k);
-        a.rho[m] = S::SHIFT ? 1.0 + double(q.drho) : double(q.rho);
+        a.rho[m] = density_f64<S>(q.sum, a.inv_scale);
         a.u[m] = double(q.u);
         a.v[m] = double(q.v);
         a.w[m] = double(q.w);
@@ -279,7 +272,7 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
     T stored[Q];
     sfor<Q>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        stored[al] = S::cvt(f[al], a.scale, store_random<S, al>(h));
+        stored[al] = S::cvt(f[al], store_random<S, al>(h));
         __builtin_nontemporal_store(stored[al], dst + (long long)al * a.ps + c);
     });
     if (post.active()) post.store(stored);

@@ -65,15 +65,39 @@ using ForceT = std::conditional_t<std::is_same_v<S, StoreF64>, double, float>;
 // (lines shared by neighbouring blocks evicted sooner), and the cavity, batch
 // and particle kernels ran 2-17 % slower, so those keep ordinary loads.
 template <class S>
-__device__ __forceinline__ typename S::Real ld_stream(const typename S::T* p, float inv_scale) {
+__device__ __forceinline__ typename S::Real ld_stream(const typename S::T* p) {
     if constexpr (S::BYTES == 2)
-        return S::val(__builtin_nontemporal_load(p), inv_scale);
+        return S::val(__builtin_nontemporal_load(p));
     else
-        return S::ld(p, inv_scale);
+        return ld<S>(p);
 }
 
-// One step of the buoyancy-driven cavity.  S = StoreF64: FP64 arithmetic in
-// the reference's order.  StoreF32 / StoreF16: f stored as f - w (FP16
+// Macro of the flow (evolution_f.F90:346-370) with the force F0 of the last
+// collision (stored units): j holds J = sum e f + F0/2, u = J / rho.
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ Moments<R> thermal_moments(const R f[Q], const R (&F0)[3], float inv_scale) {
+#pragma clang fp contract(off)
+    Moments<R> m;
+    population_sums(f, m.sum, m.j);
+    m.rho = density<S>(m.sum, inv_scale);
+    for (int d = 0; d < 3; ++d) m.j[d] = fma_(R(0.5), F0[d], m.j[d]);
+    const R r = rcp_near(m.rho), k = S::SCALED ? R(inv_scale) : R(1);
+    m.u = quotient(m.j[0] * k, m.rho, r);
+    m.v = quotient(m.j[1] * k, m.rho, r);
+    m.w = quotient(m.j[2] * k, m.rho, r);
+    return m;
+}
+
+// macroT (evolution_g.F90:202-218): T = sum g, in stored units.
+template <class R>
+__device__ __forceinline__ R temperature_sum(const R g[Q7]) {
+    R T = g[0];
+    sfor<Q7 - 1>([&](auto Am1) { T = T + g[decltype(Am1)::value + 1]; });
+    return T;
+}
+
+// One step of the buoyancy-driven cavity.  S = StoreF64: FP64 arithmetic.
+// StoreF32 / StoreF16: f stored as f - w (FP16
 // scaled by 2^k with stochastic rounding), g stored unshifted (scaled the
 // same way in FP16), the force in FP32, all arithmetic in FP32; the macro
 // fields are written as FP64 for the FP64 reductions.
@@ -97,7 +121,7 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
         constexpr int al = decltype(A)::value;
         constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
         if constexpr (al == 0) {
-            f[0] = ld_stream<S>(fsrc + c, a.inv_scale);
+            f[0] = ld_stream<S>(fsrc + c);
         } else {
             bool in = true;
             if constexpr (ex != 0) in = in && (unsigned)(i - ex) < (unsigned)a.nx;
@@ -107,11 +131,11 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
             if constexpr (HALO) {
                 // from the halo where every crossed face borders a neighbour,
                 // else bounce-back (no lid: top = false)
-                f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off), a.inv_scale)
+                f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off))
                            : pull_outside<S, al, true>(a, fsrc, i, j, k, c, false, 0.0);
             } else {
-                f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off), a.inv_scale)
-                           : ld_stream<S>(fsrc + (OPP[al] * a.ps + c), a.inv_scale);
+                f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off))
+                           : ld_stream<S>(fsrc + (OPP[al] * a.ps + c));
             }
         }
     });
@@ -122,7 +146,7 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
         constexpr int al = decltype(A)::value;
         constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
         if constexpr (al == 0) {
-            g[0] = ld_stream<S>(gsrc + c, a.inv_scale);
+            g[0] = ld_stream<S>(gsrc + c);
         } else {
             constexpr int axis = ex != 0 ? 0 : (ey != 0 ? 1 : 2);
             constexpr int e = ex + ey + ez;
@@ -132,63 +156,54 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
             const long long off = (long long)ex + (long long)ey * a.px + (long long)ez * a.pxy;
             constexpr int face = e > 0 ? 2 * axis : 2 * axis + 1;  // the face the pull enters through
             if (in) {
-                g[al] = ld_stream<S>(gsrc + (al * a.ps + c - off), a.inv_scale);
+                g[al] = ld_stream<S>(gsrc + (al * a.ps + c - off));
             } else if (HALO && ((a.halo_faces >> face) & 1)) {
                 // what arrives through `face`: the neighbour's D3Q7 population al
                 const long long p = axis == 0 ? j + (long long)a.ny * k
                                               : (axis == 1 ? i + (long long)a.nx * k : i + (long long)a.nx * j);
-                g[al] = ld_stream<S>(static_cast<const ST*>(a.halo) + (a.hoff[GREGION0 + face] + p), a.inv_scale);
+                g[al] = ld_stream<S>(static_cast<const ST*>(a.halo) + (a.hoff[GREGION0 + face] + p));
             } else {
-                const R bb = ld_stream<S>(gsrc + (OPP7[al] * a.ps + c), a.inv_scale);
-                g[al] = (a.taxis == axis) ? -bb + R(a.cw) * R(e > 0 ? a.t_hot : a.t_cold) : bb;
+                const R bb = ld_stream<S>(gsrc + (OPP7[al] * a.ps + c));
+                R held = R(a.cw) * R(e > 0 ? a.t_hot : a.t_cold);
+                if constexpr (S::SCALED) held *= R(a.scale);
+                g[al] = (a.taxis == axis) ? -bb + held : bb;
             }
         }
     });
 
     // macro (evolution_f.F90:346-370) with the force of the last collision
-    const R Fz0 = R(force[2 * a.ps + c]);
-    const R Fx0 = ROT ? R(force[c]) : R(0.0);
-    const R Fy0 = ROT ? R(force[a.ps + c]) : R(0.0);
-    R s = f[0], jx = R(-0.0), jy = R(-0.0), jz = R(-0.0);
-    sfor<Q - 1>([&](auto Am1) {
-        constexpr int al = decltype(Am1)::value + 1;
-        s = s + f[al];
-        if constexpr (EX[al] != 0) jx = mac<EX[al]>(jx, f[al]);
-        if constexpr (EY[al] != 0) jy = mac<EY[al]>(jy, f[al]);
-        if constexpr (EZ[al] != 0) jz = mac<EZ[al]>(jz, f[al]);
-    });
-    const R rho = S::SHIFT ? R(1.0) + s : s;
-    const R drho = S::SHIFT ? s : s - R(1.0);
-    const R u = (jx + R(0.5) * Fx0) / rho;
-    const R v = (jy + R(0.5) * Fy0) / rho;
-    const R w = (jz + R(0.5) * Fz0) / rho;
+    const R unit = S::SCALED ? R(a.scale) : R(1);
+    const R F0[3] = {ROT ? R(force[c]) * unit : R(0), ROT ? R(force[a.ps + c]) * unit : R(0),
+                     R(force[2 * a.ps + c]) * unit};
+    const Moments<R> q = thermal_moments<S>(f, F0, a.inv_scale);
+    const R u = q.u, v = q.v, w = q.w;
     // macroT (evolution_g.F90:202-218)
-    R T = g[0];
-    sfor<Q7 - 1>([&](auto Am1) { T = T + g[decltype(Am1)::value + 1]; });
+    const R Ts = temperature_sum(g), T = S::SCALED ? Ts * R(a.inv_scale) : Ts;  // stored units, T
     if constexpr (MACRO) {
         const long long m = i + (long long)a.nx * (j + (long long)a.ny * k);
-        a.rho[m] = S::SHIFT ? 1.0 + double(drho) : double(rho);
+        a.rho[m] = density_f64<S>(q.sum, a.inv_scale);
         a.u[m] = double(u);
         a.v[m] = double(v);
         a.w[m] = double(w);
         a.T[m] = double(T);
     }
     // next collision: force from this step's fields (evolution_f.F90:103-105)
-    const R Fx = ROT ? R(-2.0) * rho * v * R(a.omega_rot) : R(0.0);
-    const R Fy = ROT ? R(2.0) * rho * u * R(a.omega_rot) : R(0.0);
-    const R Fz = rho * R(a.g_beta) * (T - R(a.t_ref));
-    collide_mrt_forced<R, S::SHIFT>(f, rho, drho, u, v, w, Fx, Fy, Fz, R(a.snu), R(a.sq));
-    collide_d3q7<R>(g, T, u, v, w, R(a.para_a), R(a.qd), R(a.qnu));
+    const R Fx = ROT ? R(-2.0) * q.rho * v * R(a.omega_rot) : R(0.0);
+    const R Fy = ROT ? R(2.0) * q.rho * u * R(a.omega_rot) : R(0.0);
+    const R Fz = q.rho * R(a.g_beta) * (T - R(a.t_ref));
+    const R F[3] = {Fx * unit, Fy * unit, Fz * unit};
+    collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
+    collide_d3q7<R>(g, Ts, u, v, w, R(a.para_a), R(a.qd), R(a.qnu));
     ST* fdst = static_cast<ST*>(a.fdst);
     ST* gdst = static_cast<ST*>(a.gdst);
     const unsigned h = cell_random<S>(c, a.seed);
     sfor<Q>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        S::st(fdst + (al * a.ps + c), f[al], a.scale, store_random<S, al>(h));
+        st<S>(fdst + (al * a.ps + c), f[al], store_random<S, al>(h));
     });
     sfor<Q7>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        S::st(gdst + (al * a.ps + c), g[al], a.scale, store_random<S, Q + al>(h));
+        st<S>(gdst + (al * a.ps + c), g[al], store_random<S, Q + al>(h));
     });
     force[2 * a.ps + c] = FT(Fz);
     if constexpr (ROT) {
@@ -222,20 +237,21 @@ __global__ __launch_bounds__(256) void k_thermal_init(const ThermalArgs a, const
         constexpr int al = decltype(A)::value;
         const double un = u * EX[al] + v * EY[al] + w * EZ[al];
         const double feq = rho * weight(al) * (1.0 + 3.0 * un + 4.5 * un * un - 1.5 * us2);
-        f[al] = S::SHIFT ? R(feq - weight(al)) : R(feq);
+        f[al] = S::SHIFT ? R((feq - weight(al)) * a.scale) : R(feq);
     });
     const double wt0 = (1.0 - a.para_a) / 7.0, wt1 = (a.para_a + 6.0) / 42.0;
     sfor<Q7>([&](auto A) {
         constexpr int al = decltype(A)::value;
         const double un = u * EX[al] + v * EY[al] + w * EZ[al];
-        g[al] = R((al == 0 ? wt0 : wt1) * T * (1.0 + 21.0 / (6.0 + a.para_a) * un));
+        g[al] = R((al == 0 ? wt0 : wt1) * T * (1.0 + 21.0 / (6.0 + a.para_a) * un) * a.scale);
     });
     const double Fx = -2.0 * rho * v * a.omega_rot;
     const double Fy = 2.0 * rho * u * a.omega_rot;
     const double Fz = rho * a.g_beta * (T - a.t_ref);
-    collide_mrt_forced<R, S::SHIFT>(f, R(rho), R(rho - 1.0), R(u), R(v), R(w), R(Fx), R(Fy), R(Fz), R(a.snu),
-                                    R(a.sq));
-    collide_d3q7<R>(g, R(T), R(u), R(v), R(w), R(a.para_a), R(a.qd), R(a.qnu));
+    // f = f_eq carries the whole of rho u: no force before it (F0 = 0)
+    const R F[3] = {R(Fx * a.scale), R(Fy * a.scale), R(Fz * a.scale)}, F0[3] = {R(0), R(0), R(0)};
+    collide_forced<S>(f, moments_of<S>(rho, u, v, w, a.scale), F, F0, R(a.snu), R(a.sq));
+    collide_d3q7<R>(g, R(T * a.scale), R(u), R(v), R(w), R(a.para_a), R(a.qd), R(a.qnu));
     using Tst = typename S::T;
     Tst* fdst = static_cast<Tst*>(a.fdst);
     Tst* gdst = static_cast<Tst*>(a.gdst);
@@ -243,11 +259,11 @@ __global__ __launch_bounds__(256) void k_thermal_init(const ThermalArgs a, const
     const unsigned h = cell_random<S>(c, a.seed);
     sfor<Q>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        fdst[al * a.ps + c] = S::cvt(f[al], a.scale, store_random<S, al>(h));
+        fdst[al * a.ps + c] = S::cvt(f[al], store_random<S, al>(h));
     });
     sfor<Q7>([&](auto A) {
         constexpr int al = decltype(A)::value;
-        gdst[al * a.ps + c] = S::cvt(g[al], a.scale, store_random<S, Q + al>(h));
+        gdst[al * a.ps + c] = S::cvt(g[al], store_random<S, Q + al>(h));
     });
     force[c] = FT(Fx);
     force[a.ps + c] = FT(Fy);
