@@ -26,95 +26,40 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <utility>
 
+#include "block.hpp"
 #include "collide.hpp"
 #include "context.hpp"
 #include "halo.hpp"
+#include "pair.hpp"
 #include "step.hpp"
 
 using namespace lbm;
 
+// The step kernels of a context.  Several steps per launch: the isothermal box
+// with walls on all sides in the library's own launch shape (a caller's block
+// shape, occupancy cap or transform names the one-step kernel).
+struct StepPlan {
+    enum Kind { ONE, PAIR, BLOCK } kind = ONE;
+    PairTiles pair{};
+    BlockTiles block{};
+};
+
 namespace {
 
-// The looped-back exchange folded into the step: every stored population
-// that leaves through a face is also written where the looped-back unpack
-// puts it in the next step's halo (a.halo_out) -- the incoming region of the
-// opposite face, same slot and plane index as k_halo_pack and k_halo_unpack
-// use, and for a diagonal population leaving through an edge the same edge
-// region -- for the regions in a.loop_mask (those the next step reads; all
-// of them when the exchange is only rehearsed).  The step then needs no pack
-// or unpack kernel.  (Across GPUs the same stores would go to the
-// neighbour's halo over the peer link.)
-// Only cells on the box's faces store anything and the hook is skipped (one
-// branch) elsewhere.  The x faces are the one lane at each end of a row: it
-// writes its five leaving populations through a base pointer computed once;
-// the rows on y or z faces (whole waves) write theirs and the edges'.
-template <class S>
-struct LoopbackHalo {
-    const StepArgs& a;
-    int i, j, k;
-    bool xlo, xhi, ylo, yhi, zlo, zhi;  // the cell lies on that face of the box
-    __device__ __forceinline__ LoopbackHalo(const StepArgs& args, int ci, int cj, int ck)
-        : a(args), i(ci), j(cj), k(ck), xlo(ci == 0), xhi(ci == args.nx - 1), ylo(cj == 0),
-          yhi(cj == args.ny - 1), zlo(ck == 0), zhi(ck == args.nz - 1) {}
-    __device__ __forceinline__ bool active() const { return xlo || xhi || ylo || yhi || zlo || zhi; }
-
-    // the populations leaving through x face `leave` (sign SX), into the
-    // incoming region of the opposite face
-    template <int SX, class T>
-    __device__ __forceinline__ void x_face(T* out, const T (&v)[Q]) const {
-        constexpr int leave = SX > 0 ? LBM_FACE_XP : LBM_FACE_XM, arrive = leave ^ 1;
-        if (!((a.loop_mask >> arrive) & 1u)) return;
-        const long long plane = (long long)a.ny * a.nz;
-        T* b = out + a.hoff[arrive] + j + (long long)a.ny * k;
-        sfor<Q>([&](auto A) {
-            constexpr int al = decltype(A)::value;
-            if constexpr (EX[al] == SX) {
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                b[slot * plane] = v[al];
-            }
-        });
+StepPlan make_plan(const lbm_params& p, int device) {
+    StepPlan s;
+    if (p.thermal || p.halo_faces || p.block_x || p.block_y || p.waves_per_cu || p.transform == 2) return s;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return s;
     }
-
-    template <class T>
-    __device__ __forceinline__ void store(const T (&v)[Q]) const {
-        T* out = static_cast<T*>(a.halo_out);
-        if (xhi) x_face<+1>(out, v);
-        if (xlo) x_face<-1>(out, v);
-        if (!(ylo || yhi || zlo || zhi)) return;  // uniform over a wave: its row
-        const unsigned m = a.loop_mask;
-        sfor<Q>([&](auto A) {
-            constexpr int al = decltype(A)::value;
-            constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
-            const bool lx = ex > 0 ? xhi : (ex < 0 ? xlo : false);
-            bool ly = false, lz = false;
-            if constexpr (ey != 0) {
-                constexpr int leave = ey > 0 ? LBM_FACE_YP : LBM_FACE_YM, arrive = leave ^ 1;
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                ly = ey > 0 ? yhi : ylo;
-                if (ly && ((m >> arrive) & 1u))
-                    out[a.hoff[arrive] + (long long)slot * a.nx * a.nz + i + (long long)a.nx * k] = v[al];
-            }
-            if constexpr (ez != 0) {
-                constexpr int leave = ez > 0 ? LBM_FACE_ZP : LBM_FACE_ZM, arrive = leave ^ 1;
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                lz = ez > 0 ? zhi : zlo;
-                if (lz && ((m >> arrive) & 1u))
-                    out[a.hoff[arrive] + (long long)slot * a.nx * a.ny + i + (long long)a.nx * j] = v[al];
-            }
-            if constexpr (al >= 7) {
-                // a diagonal population: on its edge when it leaves through both
-                // faces (an edge always has a y or z component)
-                constexpr int r = edge_region(al), fa = edge_free_axis(al);
-                const bool on = (ex == 0 || lx) && (ey == 0 || ly) && (ez == 0 || lz);
-                if (on && ((m >> r) & 1u)) out[a.hoff[r] + (fa == 0 ? i : (fa == 1 ? j : k))] = v[al];
-            }
-        });
-    }
-};
+    if (block_plan(p.nx, p.ny, p.nz, cus, &s.block)) s.kind = StepPlan::BLOCK;
+    else if (pair_plan(p.nx, p.ny, p.nz, p.storage, cus, &s.pair)) s.kind = StepPlan::PAIR;
+    return s;
+}
 
 // One lattice update per thread.  Block = (bx, by) with bx a multiple of 64:
 // one wavefront per x-row segment of 64 cells, so every population load and
@@ -128,7 +73,7 @@ __global__ __launch_bounds__(256) void k_cavity_step(const StepArgs a) {
     const int k = blockIdx.z;
     if (i >= a.nx || j >= a.ny) return;
     if constexpr (LOOP)
-        cavity_cell<S, COLL, MACRO, HALO, MX>(a, i, j, k, LoopbackHalo<S>{a, i, j, k});
+        cavity_cell<S, COLL, MACRO, HALO, MX>(a, i, j, k, LoopbackHalo<S>{a, a.halo_out, i, j, k});
     else
         cavity_cell<S, COLL, MACRO, HALO, MX>(a, i, j, k);
 }
@@ -164,7 +109,7 @@ __global__ __launch_bounds__(256) void k_cavity_shell(const StepArgs a, const Sh
         k = r.k0 + (t - q * r.nzr);
     }
     if constexpr (LOOP)
-        cavity_cell<S, COLL, MACRO, true>(a, i, j, k, LoopbackHalo<S>{a, i, j, k});
+        cavity_cell<S, COLL, MACRO, true>(a, i, j, k, LoopbackHalo<S>{a, a.halo_out, i, j, k});
     else
         cavity_cell<S, COLL, MACRO, true>(a, i, j, k);
 }
@@ -693,7 +638,7 @@ InitFn init_fn(const lbm_ctx* c) {
 void release(lbm_ctx* c) {
     for (void* b : c->buf)
         if (b) (void)hipFree(b);
-    if (c->lid_rho) (void)hipFree(c->lid_rho);
+    if (c->lid_mem) (void)hipFree(c->lid_mem);
     if (c->macro) (void)hipFree(c->macro);
     if (c->prev) (void)hipFree(c->prev);
     if (c->red) (void)hipFree(c->red);
@@ -702,6 +647,7 @@ void release(lbm_ctx* c) {
     thermal_release(c);
     particles_release(c);
     if (c->hin_next) (void)hipFree(c->hin_next);
+    delete c->plan;
 }
 
 }  // namespace
@@ -941,11 +887,16 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
             c->step_lds_halo = p->waves_per_cu ? reserve : 0u;
         }
     }
+    c->plan = new (std::nothrow) StepPlan(make_plan(*p, c->device));
     const size_t lat = (size_t)c->ps * Q * c->elem;
-    hipError_t e = hipSuccess;
+    hipError_t e = c->plan ? hipSuccess : hipErrorOutOfMemory;
     for (auto& b : c->buf)
         if (e == hipSuccess) e = hipMalloc(&b, lat);
-    if (e == hipSuccess) e = hipMalloc(&c->lid_rho, sizeof(double) * p->nx * p->ny);
+    if (e == hipSuccess) e = hipMalloc(&c->lid_mem, sizeof(double) * 2 * p->nx * p->ny);
+    if (e == hipSuccess) {
+        c->lid_rho = c->lid_mem;
+        c->lid_next = c->lid_mem + (size_t)p->nx * p->ny;
+    }
     if (e == hipSuccess) e = hipMalloc(&c->macro, sizeof(double) * 4 * c->n);
     if (e == hipSuccess) e = hipMalloc(&c->prev, sizeof(double) * 2 * c->n);
     if (e == hipSuccess) e = hipMalloc(&c->red, sizeof(double) * RED_MAX_SUMS * (RED_BLOCKS + 1));
@@ -957,7 +908,7 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
         (void)hipGetLastError();
         return lbm_fail(LBM_ERR_NOMEM, "lbm_create: hipMalloc failed: %s", hipGetErrorString(e));
     }
-    c->device_bytes = (long long)(2 * lat + sizeof(double) * (p->nx * p->ny + 6 * c->n) +
+    c->device_bytes = (long long)(2 * lat + sizeof(double) * (2 * p->nx * p->ny + 6 * c->n) +
                                   sizeof(double) * RED_MAX_SUMS * (RED_BLOCKS + 1) + 2 * c->elem * c->htotal);
     if (p->thermal) {
         int rc = thermal_alloc(c);
@@ -1111,15 +1062,46 @@ int lbm_step(lbm_ctx* c, int nsteps) {
     }
     const unsigned lds = c->p.halo_faces ? c->step_lds_halo : c->step_lds;  // by default the halo-reading
                                                                             // kernel keeps every wave
-    for (int s = 0; s < nsteps; ++s) {
+    // as many steps per launch as the plan makes; what is left of the count goes
+    // first, one by one
+    PairArgs pa;
+    BlockArgs ba;
+    const StepPlan& plan = *c->plan;
+    const int group = plan.kind == StepPlan::BLOCK ? plan.block.steps : (plan.kind == StepPlan::PAIR ? 2 : 1);
+    for (int s = 0; s < nsteps;) {
         a.src = c->buf[c->cur];
         a.dst = c->buf[1 - c->cur];
         a.seed = (unsigned)(c->itc + s + 1);
         a.halo = c->hin;
         a.halo_out = c->hin_next;
-        hipLaunchKernelGGL(step_fn(c, s == nsteps - 1, loop), grid, c->block, lds, c->stream, a);
+        const int take = (nsteps - s) % group ? 1 : group;
+        const bool macro = s + take == nsteps;
+        int rc = LBM_OK;
+        if (take == 1) {
+            hipLaunchKernelGGL(step_fn(c, macro, loop), grid, c->block, lds, c->stream, a);
+        } else if (plan.kind == StepPlan::BLOCK) {
+            static_cast<StepArgs&>(ba) = a;
+            ba.b = plan.block;
+            ba.lid_out = c->lid_next;
+            ba.halo[0] = c->hin_next;
+            ba.halo[1] = c->hin;
+            rc = lbm_launch_block(ba, c->p.storage, c->p.collision, macro, loop, c->stream);
+        } else {
+            static_cast<StepArgs&>(pa) = a;
+            pa.t = plan.pair;
+            pa.lid_out = c->lid_next;
+            pa.halo_mid = c->hin_next;
+            pa.halo_out = c->hin;
+            rc = lbm_launch_pair(pa, c->p.storage, c->p.collision, macro, loop, c->stream);
+        }
+        if (rc) return rc;
+        if (take > 1) {
+            std::swap(c->lid_rho, c->lid_next);
+            a.lid_rho = c->lid_rho;
+        }
+        if (loop && take % 2) swap_halos(c);  // an even number of steps leaves the buffers in place
+        s += take;
         c->cur = 1 - c->cur;
-        if (loop) swap_halos(c);
     }
     c->itc += nsteps;
     return lbm_check_launch();

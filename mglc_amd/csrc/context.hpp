@@ -26,6 +26,7 @@ constexpr int RED_BLOCKS = 1024;
 constexpr int RED_MAX_SUMS = 4;
 
 struct ParticleState;  // moving spheres (particles.hip)
+struct StepPlan;       // how many steps a launch makes, and its tiles (cavity.hip)
 
 struct lbm_ctx {
     lbm_params p{};
@@ -36,7 +37,9 @@ struct lbm_ctx {
     size_t elem = 8;
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;                 // buffer holding the current f_post
-    double* lid_rho = nullptr;
+    double* lid_mem = nullptr;   // both lid densities (nx * ny each): the current one, and the one a launch of
+    double* lid_rho = nullptr;   // several steps writes, swapped after it
+    double* lid_next = nullptr;
     double* macro = nullptr;     // rho, u, v, w (4 * n)
     double* prev = nullptr;      // up, vp (2 * n)
     double* red = nullptr;       // per-block partials + totals of the FP64 reductions
@@ -66,6 +69,7 @@ struct lbm_ctx {
     void* hin_next = nullptr;
     bool halo_fresh = false;
     bool in_step = false;
+    StepPlan* plan = nullptr;
 };
 
 // Thermal path (thermal.hip).

@@ -49,6 +49,87 @@ struct NoPost {
     __device__ __forceinline__ void store(const T (&)[Q]) const {}
 };
 
+// The looped-back exchange folded into the step: every stored population
+// that leaves through a face is also written where the looped-back unpack
+// puts it in the next step's halo -- the incoming region of the
+// opposite face, same slot and plane index as k_halo_pack and k_halo_unpack
+// use, and for a diagonal population leaving through an edge the same edge
+// region -- for the regions in a.loop_mask (those the next step reads; all
+// of them when the exchange is only rehearsed).  The step then needs no pack
+// or unpack kernel.  (Across GPUs the same stores would go to the
+// neighbour's halo over the peer link.)
+// Only cells on the box's faces store anything and the hook is skipped (one
+// branch) elsewhere.  The x faces are the one lane at each end of a row: it
+// writes its five leaving populations through a base pointer computed once;
+// the rows on y or z faces (whole waves) write theirs and the edges'.
+template <class S>
+struct LoopbackHalo {
+    const StepArgs& a;
+    void* halo_out;  // the halo written
+    int i, j, k;
+    bool xlo, xhi, ylo, yhi, zlo, zhi;  // the cell lies on that face of the box
+    __device__ __forceinline__ LoopbackHalo(const StepArgs& args, void* out, int ci, int cj, int ck)
+        : a(args), halo_out(out), i(ci), j(cj), k(ck), xlo(ci == 0), xhi(ci == args.nx - 1), ylo(cj == 0),
+          yhi(cj == args.ny - 1), zlo(ck == 0), zhi(ck == args.nz - 1) {}
+    __device__ __forceinline__ bool active() const { return xlo || xhi || ylo || yhi || zlo || zhi; }
+
+    // the populations leaving through x face `leave` (sign SX), into the
+    // incoming region of the opposite face
+    template <int SX, class T>
+    __device__ __forceinline__ void x_face(T* out, const T (&v)[Q]) const {
+        constexpr int leave = SX > 0 ? LBM_FACE_XP : LBM_FACE_XM, arrive = leave ^ 1;
+        if (!((a.loop_mask >> arrive) & 1u)) return;
+        const long long plane = (long long)a.ny * a.nz;
+        T* b = out + a.hoff[arrive] + j + (long long)a.ny * k;
+        sfor<Q>([&](auto A) {
+            constexpr int al = decltype(A)::value;
+            if constexpr (EX[al] == SX) {
+                constexpr int slot = cross_slot(arrive, al, -1);
+                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
+                b[slot * plane] = v[al];
+            }
+        });
+    }
+
+    template <class T>
+    __device__ __forceinline__ void store(const T (&v)[Q]) const {
+        T* out = static_cast<T*>(halo_out);
+        if (xhi) x_face<+1>(out, v);
+        if (xlo) x_face<-1>(out, v);
+        if (!(ylo || yhi || zlo || zhi)) return;  // uniform over a wave: its row
+        const unsigned m = a.loop_mask;
+        sfor<Q>([&](auto A) {
+            constexpr int al = decltype(A)::value;
+            constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
+            const bool lx = ex > 0 ? xhi : (ex < 0 ? xlo : false);
+            bool ly = false, lz = false;
+            if constexpr (ey != 0) {
+                constexpr int leave = ey > 0 ? LBM_FACE_YP : LBM_FACE_YM, arrive = leave ^ 1;
+                constexpr int slot = cross_slot(arrive, al, -1);
+                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
+                ly = ey > 0 ? yhi : ylo;
+                if (ly && ((m >> arrive) & 1u))
+                    out[a.hoff[arrive] + (long long)slot * a.nx * a.nz + i + (long long)a.nx * k] = v[al];
+            }
+            if constexpr (ez != 0) {
+                constexpr int leave = ez > 0 ? LBM_FACE_ZP : LBM_FACE_ZM, arrive = leave ^ 1;
+                constexpr int slot = cross_slot(arrive, al, -1);
+                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
+                lz = ez > 0 ? zhi : zlo;
+                if (lz && ((m >> arrive) & 1u))
+                    out[a.hoff[arrive] + (long long)slot * a.nx * a.ny + i + (long long)a.nx * j] = v[al];
+            }
+            if constexpr (al >= 7) {
+                // a diagonal population: on its edge when it leaves through both
+                // faces (an edge always has a y or z component)
+                constexpr int r = edge_region(al), fa = edge_free_axis(al);
+                const bool on = (ex == 0 || lx) && (ey == 0 || ly) && (ez == 0 || lz);
+                if (on && ((m >> r) & 1u)) out[a.hoff[r] + (fa == 0 ? i : (fa == 1 ? j : k))] = v[al];
+            }
+        });
+    }
+};
+
 enum { COLL_MRT = 0, COLL_BGK = 1 };
 
 template <class S, int COLL, class Args>
@@ -59,6 +140,17 @@ __device__ __forceinline__ void collide(typename S::Real f[Q], const Moments<typ
         collide_flow<S, false>(f, q, snu, snu, R(0));
     else
         collide_flow<S, true>(f, q, snu, R(a.sq), a.meq12_rho ? R(0) : R(0.5) * snu);
+}
+
+// The moving lid on the two populations that come down along x
+// (bounce_back.f90:77-78): f(14) = f_post(11) - rho/6 U0, f(13) = f_post(12) -
+// rho/6 (-U0); val is the bounced value, forward for f(13).
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ R lid_bounce(R val, double rho_lid, double u_lid, float scale, bool forward) {
+#pragma clang fp contract(off)
+    double t = rho_lid / 6.0 * u_lid;
+    if constexpr (S::SCALED) t = t * double(scale);
+    return forward ? R(double(val) + t) : R(double(val) - t);
 }
 
 // Value pulled from outside the domain for population al at cell (i, j, k):
@@ -108,13 +200,10 @@ __device__ __forceinline__ typename S::Real pull_outside(const Args& a, const ty
     }
     R val = ld<S>(src + (long long)OPP[al] * a.ps + c);
     if constexpr (ez == -1 && ex != 0) {
-        // moving lid (bounce_back.f90:77-78): f(14) = f_post(11) - rho/6 U0,
-        // f(13) = f_post(12) - rho/6 (-U0); the lid is applied last, so it
-        // wins over the side walls on these two populations.
+        // the lid is applied last, so it wins over the side walls on these two
+        // populations
         if (lid) {
-            double t = rho_lid / 6.0 * a.u_lid;
-            if constexpr (S::SCALED) t *= double(a.scale);
-            val = (ex > 0) ? R(double(val) + t) : R(double(val) - t);
+            val = lid_bounce<S>(val, rho_lid, a.u_lid, a.scale, ex > 0);
         }
     }
     return val;

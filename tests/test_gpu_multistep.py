@@ -1,0 +1,61 @@
+"""The kernels that make several steps per launch (pair.hpp: two steps, tiles
+walked along z; block.hpp: two or three, one block of cells per workgroup)
+against the one-step kernel, which a caller's block shape selects: every cell
+makes the same operations, so fields, lid density and residual agree bit for
+bit.  Shapes sit at the tiles' edges: one cell past a tile, boxes thinner than
+a tile, one plane per chunk, odd numbers of steps (the rest goes one by one)."""
+import numpy as np
+import pytest
+
+from mglc_amd.lbm import Cavity, CavityConfig
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2, 2, 2), (3, 5, 4), (17, 17, 17), (24, 9, 31), (33, 30, 20),   # blocks, three and two steps
+          (65, 65, 65), (33, 14, 200), (64, 40, 70), (97, 66, 50), (130, 27, 45), (66, 130, 30)]  # pairs
+
+
+def run(shape, start, counts, **kw):
+    nx, ny, nz = shape
+    with Cavity(CavityConfig(nx, ny, nz, tauf=0.58, U0=0.1, **kw)) as c:
+        c.load_fields(*start)
+        errs = []
+        for n in counts:
+            c.step(n)
+            errs.append(c.check())
+        return c.macro(), errs
+
+
+def start_fields(shape, seed=3):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(seed)
+    return [np.ones((nz, ny, nx))] + [rng.uniform(-0.02, 0.02, (nz, ny, nx)) for _ in range(3)]
+
+
+@pytest.mark.parametrize("storage,collision,loop", [("f64", "mrt", 0), ("f64", "bgk", 1), ("f32", "mrt", 1),
+                                                    ("f32", "bgk", 0), ("f16", "mrt", 0)])
+@pytest.mark.parametrize("shape", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
+def test_several_steps_per_launch_equal_single_steps(shape, storage, collision, loop):
+    start = start_fields(shape)
+    kw = dict(storage=storage, collision=collision, halo_loopback=loop)
+    print(f"[gpu] multistep {shape} {kw}", flush=True)
+    got, errs = run(shape, start, (7, 1, 6), **kw)
+    ref, errs1 = run(shape, start, (7, 1, 6), block_x=64, block_y=1, **kw)
+    for g, r, name in zip(got, ref, ("rho", "u", "v", "w")):
+        assert np.array_equal(g, r), (name, float(np.abs(g - r).max()))
+    assert errs == errs1
+
+
+def test_restart_between_groups_of_steps():
+    """A state saved after an odd number of steps goes on in another context."""
+    shape = (65, 40, 70)
+    start = start_fields(shape)
+    with Cavity(CavityConfig(*shape, tauf=0.58)) as a, Cavity(CavityConfig(*shape, tauf=0.58)) as b:
+        a.load_fields(*start)
+        a.step(5)
+        b.load_state(a.save_state())
+        a.step(9)
+        b.step(4)
+        b.step(5)
+        for g, r in zip(a.macro(), b.macro()):
+            assert np.array_equal(g, r)
