@@ -28,36 +28,31 @@
 #include <new>
 #include <utility>
 
-#include "block.hpp"
 #include "collide.hpp"
 #include "context.hpp"
 #include "halo.hpp"
-#include "pair.hpp"
+#include "plan.hpp"
 #include "step.hpp"
 
 using namespace lbm;
-
-// The step kernels of a context.  Several steps per launch: the isothermal box
-// with walls on all sides in the library's own launch shape (a caller's block
-// shape, occupancy cap or transform names the one-step kernel).
-struct StepPlan {
-    enum Kind { ONE, PAIR, BLOCK } kind = ONE;
-    PairTiles pair{};
-    BlockTiles block{};
-};
 
 namespace {
 
 StepPlan make_plan(const lbm_params& p, int device) {
     StepPlan s;
-    if (p.thermal || p.halo_faces || p.block_x || p.block_y || p.waves_per_cu || p.transform == 2) return s;
+    if (p.halo_faces || p.block_x || p.block_y || p.waves_per_cu || p.transform == 2) return s;
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) {
         (void)hipGetLastError();
         return s;
     }
-    if (block_plan(p.nx, p.ny, p.nz, cus, &s.block)) s.kind = StepPlan::BLOCK;
-    else if (pair_plan(p.nx, p.ny, p.nz, p.storage, cus, &s.pair)) s.kind = StepPlan::PAIR;
+    if (p.thermal) {
+        if (thermal_pair_plan(p, cus, &s.pair)) s.kind = StepPlan::PAIR;
+    } else if (block_plan(p.nx, p.ny, p.nz, cus, &s.block)) {
+        s.kind = StepPlan::BLOCK;
+    } else if (pair_plan(p.nx, p.ny, p.nz, p.storage, cus, &s.pair)) {
+        s.kind = StepPlan::PAIR;
+    }
     return s;
 }
 
@@ -583,6 +578,15 @@ int fresh_loopback_halo(lbm_ctx* c) {
 
 }  // namespace
 
+bool step_capturing(const lbm_ctx* c) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;  // cannot tell: one step per launch is always right
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 int halo_loopback_exchange(lbm_ctx* c) {
     unsigned pmask, umask;
     loopback_masks(c, &pmask, &umask);
@@ -1067,7 +1071,7 @@ int lbm_step(lbm_ctx* c, int nsteps) {
     PairArgs pa;
     BlockArgs ba;
     const StepPlan& plan = *c->plan;
-    const int group = plan.kind == StepPlan::BLOCK ? plan.block.steps : (plan.kind == StepPlan::PAIR ? 2 : 1);
+    const int group = plan.kind == StepPlan::ONE || step_capturing(c) ? 1 : plan.kind == StepPlan::BLOCK ? plan.block.steps : 2;
     for (int s = 0; s < nsteps;) {
         a.src = c->buf[c->cur];
         a.dst = c->buf[1 - c->cur];

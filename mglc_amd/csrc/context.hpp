@@ -59,6 +59,8 @@ struct lbm_ctx {
     // the body force of the last collision, T and its previous check value
     void* gbuf[2] = {nullptr, nullptr};  // 7 * ps each
     void* force = nullptr;       // Fx, Fy, Fz of the last collision (3 * ps; FP64 with FP64 storage, else FP32)
+    void* force_next = nullptr;  // what a launch of two steps writes, swapped with force after it (where they run)
+    void* force_mem = nullptr;   // both
     double* temp = nullptr;      // T (n)
     double* prev_t = nullptr;    // wp, Tp for the thermal check (2 * n)
     ParticleState* part = nullptr;  // moving spheres, when attached
@@ -71,6 +73,11 @@ struct lbm_ctx {
     bool in_step = false;
     StepPlan* plan = nullptr;
 };
+
+// The context's stream is being captured into a graph: then steps go one per
+// launch, so that an even number of them leaves every buffer where it was and
+// the graph can be replayed.
+bool step_capturing(const lbm_ctx* c);
 
 // Thermal path (thermal.hip).
 // The looped-back exchange of every region the next step reads (pack from the

@@ -49,6 +49,14 @@ struct PairTable {
 
 namespace lbm {
 
+bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
+    switch (storage) {
+    case LBM_STORE_F64: return pair_plan(nx, ny, nz, PairShape<StoreF64>::NT, Q, 8, cus, out);
+    case LBM_STORE_F32: return pair_plan(nx, ny, nz, PairShape<StoreF32>::NT, Q, 4, cus, out);
+    }
+    return false;  // FP16: see below
+}
+
 // The tiles, and whether two steps go faster this way.
 //
 // Time goes by turns (planes) of the busiest CU: with one block per CU a launch
@@ -64,12 +72,9 @@ namespace lbm {
 // 5 us and 5.2 TB/s of its traffic.
 // FP16 keeps the one-step kernel: it is bound by VALU issue, of which the rim
 // takes a third more (276 against 238 us a step at 256^3).
-bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
-    if (storage == LBM_STORE_F16) return false;
-    const bool f64 = storage == LBM_STORE_F64;
-    const int nt = f64 ? PairShape<StoreF64>::NT : PairShape<StoreF32>::NT;
-    const double bytes = f64 ? 8.0 : 4.0;
-    const bool cached = double(nx) * ny * nz * 38.0 * bytes < 200e6;
+bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out) {
+    const double bytes = elem, share = pops / 19.0;
+    const bool cached = double(nx) * ny * nz * 2 * pops * bytes < 200e6;
     const long long plane = ((long long)nx + 15) / 16 * 16 * ny;
     if (plane * (long long)bytes >= PLANE_RANGE) return false;  // the lanes' offsets
     double best = 1e30;
@@ -100,7 +105,7 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
             const long long rounds = (blocks + cus - 1) / cus;
             const double busy = double(blocks) / double(rounds * cus);
             const double moved = t.h * (t.w * bytes + 128.0) + t.tx * t.ty * bytes;
-            double turn = (cached ? 5.0e-4 : 7.7e-4) * moved * (0.5 + 0.5 * busy);
+            double turn = (cached ? 5.0e-4 : 7.7e-4) * share * moved * (0.5 + 0.5 * busy);
             if (!cached && t.tx % 16 != 0 && t.ntx > 1) turn *= 1.2;
             if (turn < 4.3) turn = 4.3;
             const double time = (double(rounds) * (t.cz + 2) * turn + 4.0) / 2;
@@ -112,8 +117,10 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
     };
     for (int tx = 32; tx < nx && tx <= 128; tx += 32) consider(tx);
     for (int n = 1; n <= 4; ++n) consider((nx + n - 1) / n);
-    const double one = double(nx) * ny * nz * 38.0 * bytes / 5.2e6 + 5.0;
-    return best < 0.95 * one;
+    const double one = double(nx) * ny * nz * 2 * pops * bytes / 5.2e6 + 5.0;
+    // (a margin for what the model misses: 0.85 on small boxes, where FP32 with
+    // temperature at 51^3 took 10.9 us in pairs, 8.8 one by one)
+    return best < (one < 12.0 ? 0.85 : 0.95) * one;
 }
 
 }  // namespace lbm

@@ -273,6 +273,10 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
 // the one-step kernel is faster.
 bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out);
 
+// The same for a two-step kernel with blocks of nt threads that moves `pops`
+// values of `elem` bytes per cell and step each way.
+bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out);
+
 }  // namespace lbm
 
 // Launch the two-step kernel (walls only) for `a` on `stream`.

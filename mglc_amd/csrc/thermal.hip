@@ -20,10 +20,12 @@
 
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 #include "collide.hpp"
 #include "context.hpp"
 #include "halo.hpp"
+#include "plan.hpp"
 #include "step.hpp"
 
 using namespace lbm;
@@ -86,6 +88,26 @@ __device__ __forceinline__ Moments<R> thermal_moments(const R f[Q], const R (&F0
     m.v = quotient(m.j[1] * k, m.rho, r);
     m.w = quotient(m.j[2] * k, m.rho, r);
     return m;
+}
+
+// A population of g bounced (bb) off a held wall (evolution_g.F90:60-197):
+// -bb + (6 + paraA)/21 Twall, in stored units.
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ R held_wall(const ThermalArgs& a, R bb, bool hot) {
+#pragma clang fp contract(off)
+    R wall = R(a.cw) * R(hot ? a.t_hot : a.t_cold);
+    if constexpr (S::SCALED) wall = wall * R(a.scale);
+    return wall - bb;
+}
+
+// The force of the next collision (evolution_f.F90:103-105) from this step's
+// fields.
+template <bool ROT, class R>
+__device__ __forceinline__ void body_force(const ThermalArgs& a, const Moments<R>& q, R T, R (&F)[3]) {
+#pragma clang fp contract(off)
+    F[0] = ROT ? R(-2.0) * q.rho * q.v * R(a.omega_rot) : R(0.0);
+    F[1] = ROT ? R(2.0) * q.rho * q.u * R(a.omega_rot) : R(0.0);
+    F[2] = q.rho * R(a.g_beta) * (T - R(a.t_ref));
 }
 
 // macroT (evolution_g.F90:202-218): T = sum g, in stored units.
@@ -164,9 +186,7 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
                 g[al] = ld_stream<S>(static_cast<const ST*>(a.halo) + (a.hoff[GREGION0 + face] + p));
             } else {
                 const R bb = ld_stream<S>(gsrc + (OPP7[al] * a.ps + c));
-                R held = R(a.cw) * R(e > 0 ? a.t_hot : a.t_cold);
-                if constexpr (S::SCALED) held *= R(a.scale);
-                g[al] = (a.taxis == axis) ? -bb + held : bb;
+                g[al] = (a.taxis == axis) ? held_wall<S>(a, bb, e > 0) : bb;
             }
         }
     });
@@ -187,11 +207,9 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
         a.w[m] = double(w);
         a.T[m] = double(T);
     }
-    // next collision: force from this step's fields (evolution_f.F90:103-105)
-    const R Fx = ROT ? R(-2.0) * q.rho * v * R(a.omega_rot) : R(0.0);
-    const R Fy = ROT ? R(2.0) * q.rho * u * R(a.omega_rot) : R(0.0);
-    const R Fz = q.rho * R(a.g_beta) * (T - R(a.t_ref));
-    const R F[3] = {Fx * unit, Fy * unit, Fz * unit};
+    R Fnew[3];  // next collision: force from this step's fields
+    body_force<ROT>(a, q, T, Fnew);
+    const R F[3] = {Fnew[0] * unit, Fnew[1] * unit, Fnew[2] * unit};
     collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
     collide_d3q7<R>(g, Ts, u, v, w, R(a.para_a), R(a.qd), R(a.qnu));
     ST* fdst = static_cast<ST*>(a.fdst);
@@ -205,11 +223,245 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
         constexpr int al = decltype(A)::value;
         st<S>(gdst + (al * a.ps + c), g[al], store_random<S, Q + al>(h));
     });
-    force[2 * a.ps + c] = FT(Fz);
+    force[2 * a.ps + c] = FT(Fnew[2]);
     if constexpr (ROT) {
-        force[c] = FT(Fx);
-        force[a.ps + c] = FT(Fy);
+        force[c] = FT(Fnew[0]);
+        force[a.ps + c] = FT(Fnew[1]);
     }
+}
+
+// ---- two steps in one pass ---------------------------------------------------------
+// As pair.hpp does for the isothermal step (the tiles, the planes in LDS, the
+// loads a plane ahead, the dropped stores): 26 populations per cell, so the LDS
+// of a CU holds two planes of 384 cells in FP64 and 768 in FP32.  The force of
+// the first step stays in the thread that made it; the one read and the one
+// written lie in two arrays, since a rim cell's force is read by blocks that do
+// not own it.  Same operations as k_thermal_step, same bits.
+constexpr int QT = Q + Q7;
+
+struct ThermalPairArgs : ThermalArgs {
+    void* force_out;
+    PairTiles t;
+};
+
+template <class S>
+struct ThermalPairShape;
+template <>
+struct ThermalPairShape<StoreF64> {
+    static constexpr int NT = 384, WAVES = 2;
+};
+template <>
+struct ThermalPairShape<StoreF32> {
+    static constexpr int NT = 768, WAVES = 3;
+};
+
+// Population n of a cell's 26: flow (0..18), then temperature, with its
+// velocity and the opposite one's number.
+constexpr int vel_of(int n) { return n < Q ? n : n - Q; }
+constexpr int opp_of(int n) { return n < Q ? OPP[n] : Q + OPP7[n - Q]; }
+
+template <class S, bool ROT, bool MACRO, bool EDGE, int NT>
+__device__ __forceinline__ void thermal_pair(const ThermalPairArgs& a, int x0, int y0, int zs,
+                                             typename S::T (&buf)[2][QT][NT]) {
+    using T = typename S::T;
+    using R = typename S::Real;
+    using FT = ForceT<S>;
+    const PairTiles& t = a.t;
+    const int tid = threadIdx.x;
+    const int cell = min(tid, t.w * t.h - 1);
+    const int lx = cell % t.w, ly = cell / t.w;
+    const int i = x0 + lx, j = y0 + ly;
+    const bool own = tid < t.w * t.h && lx >= t.hx && lx < t.hx + t.tx && ly >= t.hy && ly < t.hy + t.ty &&
+                     i < a.nx && j < a.ny;
+    const int ci = min(max(i, 0), a.nx - 1), cj = min(max(j, 0), a.ny - 1);
+    const int ze = min(zs + t.cz, a.nz);
+    const int cxy = ci + a.px * cj;
+    const int nbw = t.w;
+    const int col = own || EDGE ? tid : nbw + 1;
+    auto fresh = [](int v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    // the pull of population n at plane k comes from inside the box (z: uniform)
+    auto z_inside = [&](int ez, int k) { return ez == 0 || (ez > 0 ? k > 0 : k < a.nz - 1); };
+    // population N of g, bounced (bb) off a wall that may be held at a temperature
+    auto held = [&](auto N, R bb) {
+        constexpr int v = vel_of(decltype(N)::value);
+        constexpr int axis = EX[v] != 0 ? 0 : (EY[v] != 0 ? 1 : 2);
+        return a.taxis == axis ? held_wall<S>(a, bb, EX[v] + EY[v] + EZ[v] > 0) : bb;
+    };
+
+    T in[QT];
+    FT fin[3];  // the force of the last collision
+    auto load = [&](int k) {
+        const int cl = fresh(cxy);
+        const long long plane = (long long)a.pxy * k;
+        sfor<QT>([&](auto N) {
+            constexpr int n = decltype(N)::value, v = vel_of(n);
+            constexpr int ex = EX[v], ey = EY[v], ez = EZ[v];
+            const T* s = static_cast<const T*>(n < Q ? a.fsrc : a.gsrc) + plane;
+            constexpr int own_pop = n < Q ? n : n - Q, opp_pop = n < Q ? OPP[n < Q ? n : 0] : OPP7[n < Q ? 0 : n - Q];
+            const bool zok = z_inside(ez, k);
+            const long long from = (long long)own_pop * a.ps - (ex + (long long)ey * a.px + (long long)ez * a.pxy);
+            const long long bounced = (long long)opp_pop * a.ps;
+            if constexpr (EDGE && (ex != 0 || ey != 0)) {
+                bool ok = zok;
+                if constexpr (ex != 0) ok = ok && (unsigned)(ci - ex) < (unsigned)a.nx;
+                if constexpr (ey != 0) ok = ok && (unsigned)(cj - ey) < (unsigned)a.ny;
+                in[n] = s[cl + (ok ? from : bounced)];
+            } else {
+                in[n] = plane_load<T>(plane_of(s + (zok ? from : bounced)), (unsigned)cl * (unsigned)sizeof(T));
+            }
+        });
+        const FT* fp = static_cast<const FT*>(a.force) + plane;
+        for (int d = ROT ? 0 : 2; d < 3; ++d)
+            fin[d] = plane_load<FT>(plane_of(fp + d * a.ps), (unsigned)cl * (unsigned)sizeof(FT));
+    };
+    // held walls: the pulls of g that came back from one (k: the plane)
+    auto walls = [&](R(&g)[Q7], int k) {
+        sfor<Q7 - 1>([&](auto Am1) {
+            constexpr int n = Q + decltype(Am1)::value + 1, v = vel_of(n);
+            std::integral_constant<int, n> N;
+            if constexpr (EZ[v] != 0) {
+                if (!z_inside(EZ[v], k)) g[v] = held(N, g[v]);
+            } else if constexpr (EDGE) {
+                const bool ok = EX[v] != 0 ? (unsigned)(ci - EX[v]) < (unsigned)a.nx
+                                           : (unsigned)(cj - EY[v]) < (unsigned)a.ny;
+                if (!ok) g[v] = held(N, g[v]);
+            }
+        });
+    };
+    // macro, force and collision of one cell (k_thermal_step's own): F0 the last
+    // force, F the new one
+    struct Fields {
+        double rho;
+        R u, v, w, T;
+    };
+    auto update = [&](R(&f)[Q], R(&g)[Q7], const R(&F0)[3], R(&F)[3]) {
+        const Moments<R> q = thermal_moments<S>(f, F0, a.inv_scale);
+        const R Ts = temperature_sum(g);
+        body_force<ROT>(a, q, Ts, F);
+        collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
+        collide_d3q7<R>(g, Ts, q.u, q.v, q.w, R(a.para_a), R(a.qd), R(a.qnu));
+        return Fields{density_f64<S>(q.sum, a.inv_scale), q.u, q.v, q.w, Ts};
+    };
+    R made[3], before[3];  // the first step's force on the plane just made, and on the one below
+    auto produce = [&](int p) {
+        R f[Q], g[Q7], F0[3] = {R(0), R(0), R(0)};
+        sfor<QT>([&](auto N) {
+            constexpr int n = decltype(N)::value;
+            if constexpr (n < Q) f[n] = S::val(in[n]);
+            else g[n - Q] = S::val(in[n]);
+        });
+        for (int d = ROT ? 0 : 2; d < 3; ++d) F0[d] = R(fin[d]);
+        walls(g, p);
+        update(f, g, F0, made);
+        sfor<QT>([&](auto N) {
+            constexpr int n = decltype(N)::value;
+            buf[p & 1][n][tid] = S::cvt(n < Q ? f[n < Q ? n : 0] : g[n < Q ? 0 : n - Q], 0u);
+        });
+    };
+    auto pull = [&](auto N, int k, int c) {
+        constexpr int n = decltype(N)::value, v = vel_of(n);
+        constexpr int ex = EX[v], ey = EY[v], ez = EZ[v];
+        const bool zok = z_inside(ez, k);
+        const int plane = ez == 0 ? (k & 1) : ((k + 1) & 1);
+        const int from = (plane * QT + n) * NT - (ex + ey * nbw), bounced = ((k & 1) * QT + opp_of(n)) * NT;
+        const T* b = &buf[0][0][0];
+        if constexpr (EDGE && (ex != 0 || ey != 0)) {
+            bool ok = zok && own;
+            if constexpr (ex != 0) ok = ok && (unsigned)(i - ex) < (unsigned)a.nx;
+            if constexpr (ey != 0) ok = ok && (unsigned)(j - ey) < (unsigned)a.ny;
+            return S::val(b[c + (ok ? from : bounced)]);
+        } else {
+            return S::val(b[c + (zok ? from : bounced)]);
+        }
+    };
+    R up[6];  // the flow's five pulls along e_z = +1, and the temperature's
+    auto take_up = [&](int k) {
+        const int c = fresh(col);
+        sfor<Q>([&](auto A) {
+            constexpr int al = decltype(A)::value;
+            if constexpr (EZ[al] > 0) up[up_slot(al)] = pull(A, k, c);
+        });
+        up[5] = pull(std::integral_constant<int, Q + 5>{}, k, c);
+    };
+    auto finish = [&](int k) {
+        R f[Q], g[Q7], F[3] = {R(0), R(0), R(0)};
+        const int c = fresh(col);
+        sfor<QT>([&](auto N) {
+            constexpr int n = decltype(N)::value, v = vel_of(n);
+            if constexpr (n < Q) f[n] = EZ[v] > 0 ? up[EZ[v] > 0 ? up_slot(v) : 0] : pull(N, k, c);
+            else g[n - Q] = EZ[v] > 0 ? up[5] : pull(N, k, c);
+        });
+        walls(g, k);
+        const Fields m = update(f, g, before, F);
+        if constexpr (MACRO) {
+            if (own) {
+                const long long mc = i + (long long)a.nx * (j + (long long)a.ny * k);
+                a.rho[mc] = m.rho;
+                a.u[mc] = double(m.u);
+                a.v[mc] = double(m.v);
+                a.w[mc] = double(m.w);
+                a.T[mc] = double(m.T);
+            }
+        }
+        const unsigned at = (unsigned)fresh(cxy);
+        const long long plane = (long long)a.pxy * k;
+        const unsigned where = own ? at * (unsigned)sizeof(T) : NOWHERE;
+        sfor<QT>([&](auto N) {
+            constexpr int n = decltype(N)::value;
+            T* d = static_cast<T*>(n < Q ? a.fdst : a.gdst) + plane + (long long)vel_of(n) * a.ps;
+            plane_store(S::cvt(n < Q ? f[n < Q ? n : 0] : g[n < Q ? 0 : n - Q], 0u), plane_of(d), where);
+        });
+        const unsigned fwhere = own ? at * (unsigned)sizeof(FT) : NOWHERE;
+        FT* fp = static_cast<FT*>(a.force_out) + plane;
+        for (int d = ROT ? 0 : 2; d < 3; ++d) plane_store(FT(F[d]), plane_of(fp + d * a.ps), fwhere);
+    };
+
+    const int p0 = max(zs - 1, 0), p1 = min(ze, a.nz - 1);
+    made[0] = made[1] = made[2] = before[0] = before[1] = before[2] = R(0);
+    load(p0);
+    int p = p0;
+    do {
+        produce(p);
+        load(min(p + 1, p1));
+        lds_barrier();
+        if (p == zs) take_up(p);
+        // as many stores as the second step makes, all dropped
+        sfor<QT>([&](auto N) {
+            plane_store(T(0), plane_of(static_cast<T*>(a.fdst) + (long long)decltype(N)::value * 64), NOWHERE);
+        });
+        for (int d = ROT ? 0 : 2; d < 3; ++d)
+            plane_store(FT(0), plane_of(static_cast<FT*>(a.force_out) + d * 64), NOWHERE);
+        for (int d = 0; d < 3; ++d) before[d] = made[d];
+        lds_barrier();
+    } while (++p <= zs);
+    for (; p <= p1; ++p) {
+        produce(p);
+        load(min(p + 1, p1));
+        lds_barrier();
+        finish(p - 1);
+        for (int d = 0; d < 3; ++d) before[d] = made[d];
+        take_up(p);
+        lds_barrier();
+    }
+    if (ze == a.nz) finish(a.nz - 1);
+}
+
+template <class S, bool ROT, bool MACRO>
+__global__ __launch_bounds__(ThermalPairShape<S>::NT, ThermalPairShape<S>::WAVES) void k_thermal_pair(
+    const ThermalPairArgs a) {
+    constexpr int NT = ThermalPairShape<S>::NT;
+    __shared__ typename S::T buf[2][QT][NT];
+    const int wg = xcd_order(blockIdx.x, gridDim.x);
+    const PairTiles& t = a.t;
+    const int bx = wg % t.ntx, by = (wg / t.ntx) % t.nty, bz = wg / (t.ntx * t.nty);
+    const int x0 = bx * t.tx - t.hx, y0 = by * t.ty - t.hy;
+    if (x0 >= 1 && x0 + t.w <= a.nx - 1 && y0 >= 1 && y0 + t.h <= a.ny - 1)
+        thermal_pair<S, ROT, MACRO, false, NT>(a, x0, y0, bz * t.cz, buf);
+    else
+        thermal_pair<S, ROT, MACRO, true, NT>(a, x0, y0, bz * t.cz, buf);
 }
 
 // Equilibrium start (initial.F90:172-182) and the first collision from the
@@ -409,22 +661,37 @@ int finish_sums(lbm_ctx* c, double* out) {
 
 size_t thermal_force_elem(const lbm_ctx* c) { return c->p.storage == LBM_STORE_F64 ? sizeof(double) : sizeof(float); }
 
+// The tiles of the two-step kernel; false: one step per launch (FP16, which is
+// bound by VALU issue; a loopback to rehearse; or where one-step launches are
+// faster).
+bool thermal_pair_plan(const lbm_params& p, int cus, PairTiles* t) {
+    if (p.halo_loopback) return false;
+    switch (p.storage) {
+    case LBM_STORE_F64: return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF64>::NT, QT + 1, 8, cus, t);
+    case LBM_STORE_F32: return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF32>::NT, QT + 1, 4, cus, t);
+    }
+    return false;
+}
+
 int thermal_alloc(lbm_ctx* c) {
     const size_t g_bytes = (size_t)c->ps * Q7 * c->elem;
     const size_t f_bytes = 3 * (size_t)c->ps * thermal_force_elem(c);
+    const bool pairs = c->plan->kind == StepPlan::PAIR;  // they read one force and write another
     HIP_TRY(hipMalloc(&c->gbuf[0], g_bytes));
     HIP_TRY(hipMalloc(&c->gbuf[1], g_bytes));
-    HIP_TRY(hipMalloc(&c->force, f_bytes));
+    HIP_TRY(hipMalloc(&c->force_mem, (pairs ? 2 : 1) * f_bytes));
+    c->force = c->force_mem;
+    if (pairs) c->force_next = static_cast<char*>(c->force_mem) + f_bytes;
     HIP_TRY(hipMalloc(&c->temp, (size_t)c->n * sizeof(double)));
     HIP_TRY(hipMalloc(&c->prev_t, 2 * (size_t)c->n * sizeof(double)));
-    c->device_bytes += (long long)(2 * g_bytes + f_bytes + 3 * c->n * sizeof(double));
+    c->device_bytes += (long long)(2 * g_bytes + (pairs ? 2 : 1) * f_bytes + 3 * c->n * sizeof(double));
     return LBM_OK;
 }
 
 void thermal_release(lbm_ctx* c) {
     for (void* b : c->gbuf)
         if (b) (void)hipFree(b);
-    if (c->force) (void)hipFree(c->force);
+    if (c->force_mem) (void)hipFree(c->force_mem);
     if (c->temp) (void)hipFree(c->temp);
     if (c->prev_t) (void)hipFree(c->prev_t);
 }
@@ -451,6 +718,26 @@ ThermalFn thermal_step_fn(const lbm_ctx* c, bool rot, bool macro, bool halo) {
     case LBM_STORE_F16: return ThermalTable<StoreF16>::step[rot][macro][halo];
     default: return ThermalTable<StoreF64>::step[rot][macro][halo];
     }
+}
+
+using ThermalPairFn = void (*)(const ThermalPairArgs);
+
+template <class S>
+struct ThermalPairTable {
+    // step[rotation][macro]
+    static constexpr ThermalPairFn step[2][2] = {{k_thermal_pair<S, false, false>, k_thermal_pair<S, false, true>},
+                                                 {k_thermal_pair<S, true, false>, k_thermal_pair<S, true, true>}};
+};
+
+int launch_thermal_pair(const lbm_ctx* c, const ThermalPairArgs& a, bool rot, bool macro) {
+    const dim3 grid((unsigned)(a.t.ntx * a.t.nty * a.t.ncz));
+    if (c->p.storage == LBM_STORE_F32)
+        hipLaunchKernelGGL(ThermalPairTable<StoreF32>::step[rot][macro], grid, dim3(ThermalPairShape<StoreF32>::NT), 0,
+                           c->stream, a);
+    else
+        hipLaunchKernelGGL(ThermalPairTable<StoreF64>::step[rot][macro], grid, dim3(ThermalPairShape<StoreF64>::NT), 0,
+                           c->stream, a);
+    return lbm_check_launch();
 }
 
 ThermalInitFn thermal_init_fn(const lbm_ctx* c, bool rot) {
@@ -483,7 +770,10 @@ int thermal_step(lbm_ctx* c, int nsteps) {
     const bool halo = c->p.halo_faces != 0;
     const bool loop = c->p.halo_loopback != 0;
     const dim3 grid = thermal_grid(c);
-    for (int s = 0; s < nsteps; ++s) {
+    ThermalPairArgs pa;
+    pa.t = c->plan->pair;
+    const bool pairs = c->plan->kind == StepPlan::PAIR && !step_capturing(c);
+    for (int s = 0; s < nsteps;) {
         if (loop) {
             int rc = halo_loopback_exchange(c);
             if (rc) return rc;
@@ -492,9 +782,20 @@ int thermal_step(lbm_ctx* c, int nsteps) {
         a.fdst = c->buf[1 - c->cur];
         a.gsrc = c->gbuf[c->cur];
         a.gdst = c->gbuf[1 - c->cur];
+        a.force = c->force;
         a.seed = (unsigned)(c->itc + s + 1);
-        hipLaunchKernelGGL(thermal_step_fn(c, rot, s == nsteps - 1, halo), grid, c->block, c->step_lds_halo,
-                           c->stream, a);
+        if (pairs && (nsteps - s) % 2 == 0) {
+            static_cast<ThermalArgs&>(pa) = a;
+            pa.force_out = c->force_next;
+            int rc = launch_thermal_pair(c, pa, rot, s + 2 == nsteps);
+            if (rc) return rc;
+            std::swap(c->force, c->force_next);
+            s += 2;
+        } else {
+            hipLaunchKernelGGL(thermal_step_fn(c, rot, s == nsteps - 1, halo), grid, c->block, c->step_lds_halo,
+                               c->stream, a);
+            s += 1;
+        }
         c->cur = 1 - c->cur;
     }
     return lbm_check_launch();

@@ -4,10 +4,13 @@ against the one-step kernel, which a caller's block shape selects: every cell
 makes the same operations, so fields, lid density and residual agree bit for
 bit.  Shapes sit at the tiles' edges: one cell past a tile, boxes thinner than
 a tile, one plane per chunk, odd numbers of steps (the rest goes one by one)."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from mglc_amd.lbm import Cavity, CavityConfig
+from mglc_amd.hip import Stream, runtime
+from mglc_amd.lbm import Cavity, CavityConfig, ThermalConfig
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +62,56 @@ def test_restart_between_groups_of_steps():
         b.step(5)
         for g, r in zip(a.macro(), b.macro()):
             assert np.array_equal(g, r)
+
+
+THERMAL_SHAPES = [(3, 4, 5), (33, 30, 40), (51, 51, 51), (64, 31, 90), (128, 40, 36), (65, 100, 33)]
+
+
+@pytest.mark.parametrize("storage,axis,ekman", [("f64", 1, None), ("f64", 2, 1e-3), ("f32", 0, None),
+                                                ("f32", 1, 1e-3)])
+@pytest.mark.parametrize("shape", THERMAL_SHAPES, ids=["x".join(map(str, s)) for s in THERMAL_SHAPES])
+def test_two_buoyancy_steps_per_launch_equal_single_steps(shape, storage, axis, ekman):
+    nx, ny, nz = shape
+    start = start_fields(shape)
+    T = np.random.default_rng(5).uniform(-0.4, 0.4, (nz, ny, nx))
+    print(f"[gpu] multistep thermal {shape} {storage} {axis} {ekman}", flush=True)
+    out = []
+    for kw in (dict(), dict(block_x=64, block_y=1)):
+        cfg = ThermalConfig(nx, ny, nz, Rayleigh=2e4, N=max(shape), Ekman=ekman, thermal_axis=axis, storage=storage, **kw)
+        with Cavity(cfg) as c:
+            c.load_fields(*start, T)
+            c.step(7)
+            e1 = c.check_thermal()
+            c.step(6)
+            out.append((*c.macro(), c.temperature(), np.array([e1, c.check_thermal(), c.nusselt()])))
+    for g, r, name in zip(*out, ("rho", "u", "v", "w", "T", "sums")):
+        assert np.array_equal(g, r), (name, float(np.abs(g - r).max()))
+
+
+def test_steps_captured_into_a_graph_replay():
+    """Under stream capture steps go one per launch, so a graph of an even number
+    of them leaves the buffers in place and every replay goes on from the last."""
+    shape = (65, 40, 70)
+    start = start_fields(shape)
+    hip = runtime()
+    stream, graph, ex = Stream(), ctypes.c_void_p(), ctypes.c_void_p()
+    with Cavity(CavityConfig(*shape, tauf=0.58), stream=stream.handle.value) as a, \
+            Cavity(CavityConfig(*shape, tauf=0.58), stream=stream.handle.value) as b:
+        for c in (a, b):
+            c.load_fields(*start)
+            c.step(2)
+            c.synchronize()
+        assert hip.hipStreamBeginCapture(stream.handle, 2) == 0  # relaxed
+        a.step(4)
+        assert hip.hipStreamEndCapture(stream.handle, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+        try:
+            for _ in range(3):
+                assert hip.hipGraphLaunch(ex, stream.handle) == 0
+                b.step(4)
+                for x, y in zip(a.macro(), b.macro()):
+                    assert np.array_equal(x, y)
+        finally:
+            hip.hipGraphExecDestroy(ex)
+            hip.hipGraphDestroy(graph)
+    stream.close()
