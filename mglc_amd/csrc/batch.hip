@@ -233,6 +233,7 @@ struct lbm_batch {
     double* macro = nullptr;       // 4 * total_cells
     unsigned* ctr = nullptr;       // device step counter
     hipStream_t stream = nullptr;
+    int device = 0;
     float scale = 1.0f, inv_scale = 1.0f;
     long long itc = 0;
     bool initialised = false;
@@ -424,6 +425,7 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
     b->total_cells = moff;
     b->total_lid = loff;
     b->total_tiles = (int)tiles;
+    (void)hipGetDevice(&b->device);
     hipError_t e = hipStreamCreate(&b->stream);
     for (auto& p : b->buf)
         if (e == hipSuccess) e = hipMalloc(&p, b->elem * (size_t)off);
@@ -466,6 +468,7 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
         a.v = b->macro + 2 * b->total_cells + in.macro_off;
         a.w = b->macro + 3 * b->total_cells + in.macro_off;
     }
+    lbm_staging_user(+1);
     *out = b;
     return LBM_OK;
 }
@@ -475,6 +478,7 @@ int lbm_batch_destroy(lbm_batch* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     release(b);
     delete b;
+    lbm_staging_user(-1);
     return LBM_OK;
 }
 
@@ -626,12 +630,10 @@ int lbm_batch_download_macro(lbm_batch* b, int instance, double* rho, double* u,
     if (!b->initialised) return lbm_fail(LBM_ERR_STATE, "lbm_batch_download_macro before lbm_batch_initial");
     const BatchInst& in = b->host[instance];
     double* dst[4] = {rho, u, v, w};
+    lbm_copy copies[4];
     for (int q = 0; q < 4; ++q)
-        if (dst[q])
-            HIP_TRY(hipMemcpyAsync(dst[q], b->macro + q * b->total_cells + in.macro_off, sizeof(double) * in.ncells,
-                                   hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    return LBM_OK;
+        copies[q] = {dst[q], b->macro + q * b->total_cells + in.macro_off, sizeof(double) * in.ncells};
+    return lbm_download(b->device, b->stream, copies, 4);
 }
 
 int lbm_batch_get_info(const lbm_batch* b, lbm_batch_info* info) {

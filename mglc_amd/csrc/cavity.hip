@@ -939,6 +939,7 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
         delete c;
         return lbm_fail(LBM_ERR_HIP, "lbm_create: clearing the halo failed");
     }
+    lbm_staging_user(+1);
     *out = c;
     return LBM_OK;
 }
@@ -948,6 +949,7 @@ int lbm_destroy(lbm_ctx* c) {
     (void)hipStreamSynchronize(c->stream);
     release(c);
     delete c;
+    lbm_staging_user(-1);
     return LBM_OK;
 }
 
@@ -1195,9 +1197,8 @@ int lbm_download_temperature(lbm_ctx* c, double* T) {
     if (!c || !T) return lbm_fail(LBM_ERR_ARG, "lbm_download_temperature: null argument");
     if (!c->p.thermal) return lbm_fail(LBM_ERR_STATE, "lbm_download_temperature on an isothermal context");
     if (!c->initialised) return lbm_fail(LBM_ERR_STATE, "lbm_download_temperature before lbm_initial");
-    HIP_TRY(hipMemcpyAsync(T, c->temp, sizeof(double) * c->n, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    const lbm_copy copy = {T, c->temp, sizeof(double) * c->n};
+    return lbm_download(c->device, c->stream, &copy, 1);
 }
 
 int lbm_halo_layout(const lbm_ctx* c, int region, long long* offset, long long* count) {
@@ -1264,12 +1265,9 @@ int lbm_download_macro(lbm_ctx* c, double* rho, double* u, double* v, double* w)
     if (!c->initialised) return lbm_fail(LBM_ERR_STATE, "lbm_download_macro before lbm_initial");
     if (c->in_step) return lbm_fail(LBM_ERR_STATE, "lbm_download_macro between lbm_step_begin and lbm_step_end");
     double* dst[4] = {rho, u, v, w};
-    const size_t bytes = sizeof(double) * c->n;
-    for (int q = 0; q < 4; ++q)
-        if (dst[q])
-            HIP_TRY(hipMemcpyAsync(dst[q], c->macro + q * c->n, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    lbm_copy copies[4];
+    for (int q = 0; q < 4; ++q) copies[q] = {dst[q], c->macro + q * c->n, sizeof(double) * c->n};
+    return lbm_download(c->device, c->stream, copies, 4);
 }
 
 int lbm_synchronize(lbm_ctx* c) {

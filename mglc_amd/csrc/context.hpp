@@ -19,6 +19,18 @@ int lbm_check_launch();
                             __FILE__, __LINE__);                                               \
     } while (0)
 
+// Device arrays to host memory (download.hip); returns when they are there.
+// Entries without a dst are left out.
+struct lbm_copy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+int lbm_download(int device, hipStream_t stream, const lbm_copy* copies, int count);
+// A context or batch comes (+1) or goes (-1): the staging memory of the downloads
+// goes with the last.
+void lbm_staging_user(int change);
+
 // Deterministic FP64 reductions: a fixed grid of per-block partials, then one
 // block sums the partials in a fixed order.
 constexpr int RED_THREADS = 256;

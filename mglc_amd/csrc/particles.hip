@@ -1575,9 +1575,8 @@ int lbm_particles_get(lbm_ctx* c, double* centers, double* U, double* omega, dou
 
 int lbm_particles_map(lbm_ctx* c, int* owner) {
     if (!c || !c->part || !owner) return lbm_fail(LBM_ERR_STATE, "lbm_particles_map: no particles attached");
-    HIP_TRY(hipMemcpyAsync(owner, c->part->owner[c->part->cur], sizeof(int) * c->n, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    const lbm_copy copy = {owner, c->part->owner[c->part->cur], sizeof(int) * c->n};
+    return lbm_download(c->device, c->stream, &copy, 1);
 }
 
 }  // extern "C"

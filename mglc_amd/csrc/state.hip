@@ -129,12 +129,12 @@ int lbm_save_state(lbm_ctx* c, void* blob, size_t bytes) {
     size_t off = sizeof h;
     Section s[9];
     const int k = sections(c, s);
+    lbm_copy copies[9];
     for (int q = 0; q < k; ++q) {
-        HIP_TRY(hipMemcpyAsync(out + off, s[q].dev, s[q].bytes, hipMemcpyDeviceToHost, c->stream));
+        copies[q] = {out + off, s[q].dev, s[q].bytes};
         off += s[q].bytes;
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    return lbm_download(c->device, c->stream, copies, k);
 }
 
 int lbm_load_state(lbm_ctx* c, const void* blob, size_t bytes) {
