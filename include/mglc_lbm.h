@@ -313,10 +313,11 @@ int lbm_particles_map(lbm_ctx *ctx, int *owner);
 
 /* ---- batched cavities ----------------------------------------------------
  * Many independent lid-driven cavities of uneven sizes, Re and U0 stepped
- * together: one persistent kernel walks 64-cell tiles of every instance
- * through a per-instance offset table; whole 100-step blocks are replayed
- * from a captured hipGraph; the persistent launch shape is picked by
- * lbm_batch_autotune.  Each instance reproduces a single-context run of the
+ * together: two steps per launch over the tiles of every instance where that
+ * is faster (FP64, FP32), else one kernel walks 64-cell tiles of every instance
+ * through a per-instance offset table, its launch shape picked by
+ * lbm_batch_autotune; whole 100-step blocks are replayed from a captured
+ * hipGraph.  Each instance reproduces a single-context run of the
  * same parameters exactly.  No reference counterpart: the reference runs one
  * cavity per program (mpi_3d_blocked/main.f90). */
 typedef struct lbm_batch lbm_batch;
@@ -324,7 +325,7 @@ typedef struct lbm_batch lbm_batch;
 typedef struct lbm_batch_info {
     long long instances, total_cells, total_tiles, steps_done, device_bytes;
     double bytes_per_lup;       /* 2*19*sizeof(store) */
-    int threads, blocks;        /* persistent launch shape in use */
+    int threads, blocks;        /* shape of the one-step launches */
     int graph_steps;            /* steps per captured graph */
     int cells_per_thread;       /* cells each thread updates per step (1, 2 or 4) */
     void *stream;               /* the batch's own hipStream_t */
@@ -336,17 +337,20 @@ int lbm_batch_create(const lbm_params *params, int count, lbm_batch **batch);
 int lbm_batch_destroy(lbm_batch *batch);
 /* Reference initial state (initial.f90:46-73) in every instance. */
 int lbm_batch_initial(lbm_batch *batch);
-/* nsteps steps of every instance: the persistent kernel, graph-replayed in
- * blocks of 100 steps.  Macro fields of the last step are kept. */
+/* nsteps steps of every instance, graph-replayed in blocks of 100 steps.  Macro fields of the last step are kept. */
 int lbm_batch_step(lbm_batch *batch, int nsteps);
 /* The same steps with one single-domain launch per instance per step (the
  * instances launched one at a time): the baseline the batch is measured
  * against. */
 int lbm_batch_step_each(lbm_batch *batch, int nsteps);
 /* Time trial_steps steps at each candidate launch shape (64/128/256 threads,
- * 4..64 waves per CU, 1/2/4 cells per thread), keep the fastest, and restart
- * from the initial state.  The cells per thread chosen are in lbm_batch_info. */
+ * 4..128 waves per CU, 1/2/4 cells per thread), keep the fastest, and restart
+ * from the initial state.  Two steps per launch, where planned, are timed
+ * against the fastest shape.  The cells per thread chosen are in
+ * lbm_batch_info. */
 int lbm_batch_autotune(lbm_batch *batch, int trial_steps, int *threads, int *blocks);
+/* Step with this shape from now on, one step per launch (as does
+ * lbm_batch_set_cells_per_thread).  Results do not depend on it. */
 int lbm_batch_set_launch(lbm_batch *batch, int threads, int blocks);
 /* Each wave takes cells_per_thread consecutive 64-cell tiles per turn (1, 2
  * or 4): a thread updates that many cells per step.  Results do not depend on

@@ -1,10 +1,11 @@
 // batch.hip -- many independent lid-driven cavities of uneven sizes stepped
-// together: one persistent kernel walks a flat list of 64-cell tiles of every
-// instance (per-instance offset table in device memory), steps are replayed
-// from a hipGraph holding 100 step launches, and the persistent launch shape
-// is chosen by timing candidates (autotune).  Each cell is updated by the
-// same per-cell code as the single-domain kernel (step.hpp), so every
-// instance reproduces a single-domain run of it exactly.
+// together.  Two steps per launch (pair.hpp) over a flat list of every
+// instance's tiles where that is faster; else one kernel walks a flat list of
+// 64-cell tiles of every instance (per-instance offset table in device memory),
+// its launch shape chosen by timing candidates (autotune).  Steps are replayed
+// from a hipGraph holding 100 of them.  Each cell is updated by the same code as
+// in the single-domain kernels, so every instance reproduces a single-domain run
+// of it exactly.
 //
 // Device layout: instance m's lattice is the single-domain SoA layout of its
 // own size, placed at element offset off[m] inside two shared buffers (A-B);
@@ -14,11 +15,13 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstring>
 #include <new>
 #include <vector>
 
 #include "collide.hpp"
 #include "context.hpp"
+#include "pair.hpp"
 #include "step.hpp"
 
 using namespace lbm;
@@ -124,6 +127,47 @@ __global__ __launch_bounds__(256) void k_batch_step(const BatchArgs b) {
     }
 }
 
+// Two steps of every instance in one launch (pair.hpp): a block walks one tile
+// of one instance along z.  Bound as the single-domain kernel, by the memory
+// pattern of its planes, and in small batches by the last blocks, which is what
+// the plan's chunk lengths balance.  Measured on MI355X, us a step, one step and
+// two steps per launch: 24 cavities of 32^3-64^3 (2.3 M cells) FP32 64.2 and
+// 49.2, FP64 123 and 91; 8 of them (1.0 M) 30.3 and 22.8, 58.3 and 41.1; 64
+// cavities of 32^3-96^3 (21 M) 586 and 360, 1216 and 693.
+template <class S, int COLL, bool MACRO>
+__global__ __launch_bounds__(PairShape<S>::NT, PairShape<S>::WAVES) void k_batch_pair(
+    const BatchArgs b, const PairBlock* __restrict__ blocks, const PairTiles* __restrict__ tiles, double* lid_out) {
+    using T = typename S::T;
+    __shared__ T buf[2][Q][PairShape<S>::NT];
+    const PairBlock blk = blocks[blockIdx.x];
+    const BatchInst& in = b.inst[blk.box];
+    const PairTiles t = tiles[blk.box];
+    PairArgs a;
+    a.src = static_cast<const T*>(b.src) + in.off;
+    a.dst = static_cast<T*>(b.dst) + in.off;
+    a.nx = in.nx;
+    a.ny = in.ny;
+    a.nz = in.nz;
+    a.px = in.px;
+    a.pxy = in.pxy;
+    a.ps = in.ps;
+    a.u_lid = in.u_lid;
+    a.snu = in.snu;
+    a.sq = in.sq;
+    a.scale = b.scale;
+    a.inv_scale = b.inv_scale;
+    a.meq12_rho = b.meq12_rho;
+    a.lid_rho = b.lid_rho + in.lid_off;
+    a.lid_out = lid_out + in.lid_off;
+    a.rho = b.rho + in.macro_off;
+    a.u = b.u + in.macro_off;
+    a.v = b.v + in.macro_off;
+    a.w = b.w + in.macro_off;
+    a.seed = 0;
+    cavity_pair_at<S, COLL, MACRO, PairShape<S>::NT>(a, t, blk.x0, blk.y0, blk.zs, buf,
+                                                     [](int, int, int, bool) { return NoPost{}; });
+}
+
 // Equilibrium start + first collision of every instance (the initial state of
 // initial.f90), from the macro arrays (rho = rho0, u = U0 on each top layer).
 template <class S, int COLL>
@@ -217,6 +261,14 @@ struct BatchTable {
     static constexpr BatchInitFn init[2] = {k_batch_init<S, COLL_MRT>, k_batch_init<S, COLL_BGK>};
 };
 
+using BatchPairFn = void (*)(const BatchArgs, const PairBlock*, const PairTiles*, double*);
+template <class S>
+struct BatchPairTable {
+    // step[collision][macro]
+    static constexpr BatchPairFn step[2][2] = {{k_batch_pair<S, COLL_MRT, false>, k_batch_pair<S, COLL_MRT, true>},
+                                               {k_batch_pair<S, COLL_BGK, false>, k_batch_pair<S, COLL_BGK, true>}};
+};
+
 }  // namespace
 
 struct lbm_batch {
@@ -229,7 +281,13 @@ struct lbm_batch {
     int total_tiles = 0;
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;
-    double* lid_rho = nullptr;
+    double* lid[2] = {nullptr, nullptr};  // lid densities: lid[lcur] the current ones, the other what a
+    int lcur = 0;                         // launch of two steps writes
+    // two steps per launch, where they are faster and the caller set no launch shape
+    int npair = 0;                 // blocks of such a launch (0: none planned)
+    bool pairs = false;            // in use
+    PairTiles* pair_tiles = nullptr;   // (one allocation)
+    PairBlock* pair_blocks = nullptr;
     double* macro = nullptr;       // 4 * total_cells
     unsigned* ctr = nullptr;       // device step counter
     hipStream_t stream = nullptr;
@@ -243,6 +301,8 @@ struct lbm_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int graph_cur = -1;            // buffer parity the graph was captured for
+    int graph_lcur = 0;            // and of the lid densities
+    bool graph_pairs = false;
     int graph_threads = 0, graph_blocks = 0, graph_cpt = 0;
     std::vector<StepArgs> single; // per-instance arguments of the single-domain kernel (baseline)
     long long device_bytes = 0;
@@ -255,7 +315,7 @@ BatchArgs batch_args(const lbm_batch* b) {
     a.inst = b->inst;
     a.ninst = b->ninst;
     a.total_tiles = b->total_tiles;
-    a.lid_rho = b->lid_rho;
+    a.lid_rho = b->lid[b->lcur];
     a.rho = b->macro;
     a.u = b->macro + b->total_cells;
     a.v = b->macro + 2 * b->total_cells;
@@ -296,6 +356,35 @@ void launch_batch_step(lbm_batch* b, int cur, bool macro, int step_add) {
     hipLaunchKernelGGL(batch_step_fn(b, macro), dim3(b->blocks), dim3(b->threads), 0, b->stream, a);
 }
 
+// Two steps in one launch: both parities flip.
+void launch_batch_pair(lbm_batch* b, int cur, bool macro) {
+    BatchArgs a = batch_args(b);
+    a.src = b->buf[cur];
+    a.dst = b->buf[1 - cur];
+    const int coll = b->p0.collision == LBM_BGK ? COLL_BGK : COLL_MRT;
+    const bool f32 = b->p0.storage == LBM_STORE_F32;
+    const BatchPairFn fn = f32 ? BatchPairTable<StoreF32>::step[coll][macro] : BatchPairTable<StoreF64>::step[coll][macro];
+    hipLaunchKernelGGL(fn, dim3((unsigned)b->npair), dim3(f32 ? PairShape<StoreF32>::NT : PairShape<StoreF64>::NT), 0,
+                       b->stream, a, b->pair_blocks, b->pair_tiles, b->lid[1 - b->lcur]);
+    b->lcur = 1 - b->lcur;
+}
+
+// nsteps steps from buffer `cur` (in pairs, the odd one first); the last writes
+// the macro fields.  Returns the buffer they end in.
+int launch_steps(lbm_batch* b, int cur, int nsteps) {
+    for (int s = 0; s < nsteps;) {
+        if (b->pairs && (nsteps - s) % 2 == 0) {
+            launch_batch_pair(b, cur, s + 2 == nsteps);
+            s += 2;
+        } else {
+            launch_batch_step(b, cur, s + 1 == nsteps, s);
+            s += 1;
+        }
+        cur = 1 - cur;
+    }
+    return cur;
+}
+
 // The device step counter moves past a sequence of n steps (one launch per
 // sequence instead of one per step).
 void advance_counter(lbm_batch* b, int n) {
@@ -315,11 +404,7 @@ void drop_graph(lbm_batch* b) {
 int capture_graph(lbm_batch* b, int cur) {
     drop_graph(b);
     HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeGlobal));
-    int c = cur;
-    for (int s = 0; s < GRAPH_STEPS; ++s) {
-        launch_batch_step(b, c, s == GRAPH_STEPS - 1, s);
-        c = 1 - c;
-    }
+    (void)launch_steps(b, cur, GRAPH_STEPS);  // (ends in the parities it began with)
     advance_counter(b, GRAPH_STEPS);
     hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
     if (e != hipSuccess) {
@@ -328,19 +413,55 @@ int capture_graph(lbm_batch* b, int cur) {
     }
     HIP_TRY(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
     b->graph_cur = cur;
+    b->graph_lcur = b->lcur;
+    b->graph_pairs = b->pairs;
     b->graph_threads = b->threads;
     b->graph_blocks = b->blocks;
     b->graph_cpt = b->cpt;
     return LBM_OK;
 }
 
-int default_blocks(int threads) {
-    int dev = 0, cus = 256;
+int device_cus() {
+    int dev = 0, cus = 0;
     (void)hipGetDevice(&dev);
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
-    return cus * (2048 / threads);  // enough waves to fill every CU
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    return cus;
+}
+
+// Blocks of the one-step launches: as many as there are tiles for, up to 512
+// waves per CU: a wave that walks few tiles leaves its CU to the next one early.
+// Measured on MI355X on 32, 128 and 512 waves per CU: 24 cavities of 32^3-64^3
+// FP32 69.9, 65.9 and 64.4 us a step, FP16 63.8, 54.8 and 54.5; 64 cavities of
+// 32^3-96^3 FP32 637, 628 and 589.
+int default_blocks(int threads, int tiles) {
+    const int waves = threads / 64;
+    return std::min(device_cus() * (512 / waves), (tiles - 1) / waves + 1);
+}
+
+// The blocks of the two-step launches, where they are faster.
+hipError_t plan_pairs(lbm_batch* b) try {
+    std::vector<PairBox> boxes;
+    for (const BatchInst& in : b->host) boxes.push_back({in.nx, in.ny, in.nz});
+    std::vector<PairTiles> tiles;
+    std::vector<PairBlock> blocks;
+    if (!pair_batch_plan(boxes, b->p0.storage, device_cus(), &tiles, &blocks)) return hipSuccess;
+    const size_t nt = sizeof(PairTiles) * tiles.size(), nb = sizeof(PairBlock) * blocks.size();
+    std::vector<char> both(nt + nb);
+    std::memcpy(both.data(), tiles.data(), nt);
+    std::memcpy(both.data() + nt, blocks.data(), nb);
+    hipError_t e = hipMalloc(&b->pair_tiles, nt + nb);
+    if (e == hipSuccess) e = hipMemcpy(b->pair_tiles, both.data(), nt + nb, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        b->pair_blocks = reinterpret_cast<PairBlock*>(b->pair_tiles + tiles.size());
+        b->npair = (int)blocks.size();
+        b->pairs = true;
+    }
+    return e;
+} catch (...) {
+    return hipErrorOutOfMemory;
 }
 
 void release(lbm_batch* b) {
@@ -348,7 +469,8 @@ void release(lbm_batch* b) {
     for (void* p : b->buf)
         if (p) (void)hipFree(p);
     if (b->inst) (void)hipFree(b->inst);
-    if (b->lid_rho) (void)hipFree(b->lid_rho);
+    if (b->lid[0]) (void)hipFree(b->lid[0]);  // both
+    if (b->pair_tiles) (void)hipFree(b->pair_tiles);
     if (b->macro) (void)hipFree(b->macro);
     if (b->ctr) (void)hipFree(b->ctr);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -430,20 +552,22 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
     for (auto& p : b->buf)
         if (e == hipSuccess) e = hipMalloc(&p, b->elem * (size_t)off);
     if (e == hipSuccess) e = hipMalloc(&b->inst, sizeof(BatchInst) * count);
-    if (e == hipSuccess) e = hipMalloc(&b->lid_rho, sizeof(double) * loff);
+    if (e == hipSuccess) e = hipMalloc(&b->lid[0], sizeof(double) * 2 * loff);
+    if (e == hipSuccess) b->lid[1] = b->lid[0] + loff;
     if (e == hipSuccess) e = hipMalloc(&b->macro, sizeof(double) * 4 * moff);
     if (e == hipSuccess) e = hipMalloc(&b->ctr, sizeof(unsigned));
     if (e == hipSuccess)
         e = hipMemcpy(b->inst, b->host.data(), sizeof(BatchInst) * count, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = plan_pairs(b);
     if (e != hipSuccess) {
         release(b);
         delete b;
         (void)hipGetLastError();
         return lbm_fail(LBM_ERR_NOMEM, "lbm_batch_create: %s", hipGetErrorString(e));
     }
-    b->device_bytes = (long long)(2 * b->elem * off + sizeof(double) * (loff + 4 * moff) + sizeof(BatchInst) * count);
+    b->device_bytes = (long long)(2 * b->elem * off + sizeof(double) * (2 * loff + 4 * moff) + sizeof(BatchInst) * count);
     b->threads = 256;
-    b->blocks = default_blocks(b->threads);
+    b->blocks = default_blocks(b->threads, b->total_tiles);
     // single-domain arguments per instance, for the one-launch-per-instance baseline
     b->single.resize(count);
     for (int m = 0; m < count; ++m) {
@@ -462,7 +586,6 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
         a.scale = b->scale;
         a.inv_scale = b->inv_scale;
         a.meq12_rho = p0.meq12_rho;
-        a.lid_rho = b->lid_rho + in.lid_off;
         a.rho = b->macro + in.macro_off;
         a.u = b->macro + b->total_cells + in.macro_off;
         a.v = b->macro + 2 * b->total_cells + in.macro_off;
@@ -489,7 +612,7 @@ int lbm_batch_initial(lbm_batch* b) {
                        b->macro + 3 * b->total_cells, b->total_cells);
     BatchArgs a = batch_args(b);
     a.dst = b->buf[0];
-    hipLaunchKernelGGL(batch_init_fn(b), dim3(default_blocks(256)), dim3(256), 0, b->stream, a);
+    hipLaunchKernelGGL(batch_init_fn(b), dim3(default_blocks(256, b->total_tiles)), dim3(256), 0, b->stream, a);
     hipLaunchKernelGGL(k_counter_set, dim3(1), dim3(1), 0, b->stream, b->ctr, 1u);
     int rc = lbm_check_launch();
     if (rc) return rc;
@@ -507,7 +630,8 @@ int lbm_batch_step(lbm_batch* b, int nsteps) {
     // graph replays for whole 100-step blocks, direct launches for the rest
     int remaining = nsteps;
     while (remaining >= GRAPH_STEPS) {
-        if (!b->graph_exec || b->graph_cur != b->cur || b->graph_threads != b->threads ||
+        if (!b->graph_exec || b->graph_cur != b->cur || b->graph_lcur != b->lcur || b->graph_pairs != b->pairs ||
+            b->graph_threads != b->threads ||
             b->graph_blocks != b->blocks || b->graph_cpt != b->cpt) {
             int rc = capture_graph(b, b->cur);
             if (rc) return rc;
@@ -515,10 +639,7 @@ int lbm_batch_step(lbm_batch* b, int nsteps) {
         HIP_TRY(hipGraphLaunch(b->graph_exec, b->stream));
         remaining -= GRAPH_STEPS;  // even, so the current buffer is unchanged
     }
-    for (int s = 0; s < remaining; ++s) {
-        launch_batch_step(b, b->cur, s == remaining - 1, s);
-        b->cur = 1 - b->cur;
-    }
+    b->cur = launch_steps(b, b->cur, remaining);
     advance_counter(b, remaining);
     b->itc += nsteps;
     return lbm_check_launch();
@@ -534,6 +655,7 @@ int lbm_batch_step_each(lbm_batch* b, int nsteps) {
             StepArgs a = b->single[m];
             a.src = static_cast<const char*>(b->buf[b->cur]) + b->elem * b->host[m].off;
             a.dst = static_cast<char*>(b->buf[1 - b->cur]) + b->elem * b->host[m].off;
+            a.lid_rho = b->lid[b->lcur] + b->host[m].lid_off;
             a.seed = (unsigned)(b->itc + s + 1);
             int rc = lbm_launch_cavity_step(a, b->p0.storage, b->p0.collision, macro, b->stream);
             if (rc) return rc;
@@ -550,21 +672,17 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, int* best_threads, int* be
     if (trial_steps < 1) trial_steps = 4;
     int rc = lbm_batch_initial(b);
     if (rc) return rc;
-    int dev = 0, cus = 256;
-    (void)hipGetDevice(&dev);
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-        cus = prop.multiProcessorCount;
+    const int cus = device_cus();
     hipEvent_t e0, e1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     float best = 1e30f;
     int bt = b->threads, bb = b->blocks, bc = b->cpt;
     const int threads_c[3] = {64, 128, 256};
-    const int waves_per_cu_c[5] = {4, 8, 16, 32, 64};
+    const int waves_per_cu_c[6] = {4, 8, 16, 32, 64, 128};
     for (int ci = 0; ci < 3; ++ci)
     for (int ti = 0; ti < 3; ++ti)
-        for (int wi = 0; wi < 5; ++wi) {
+        for (int wi = 0; wi < 6; ++wi) {
             b->cpt = CPT_CHOICES[ci];
             b->threads = threads_c[ti];
             b->blocks = std::max(1, cus * waves_per_cu_c[wi] / (threads_c[ti] / 64));
@@ -587,6 +705,21 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, int* best_threads, int* be
                 bc = b->cpt;
             }
         }
+    b->pairs = false;
+    if (b->npair) {  // two steps per launch, against the best of the others
+        launch_batch_pair(b, b->cur, false);
+        b->cur = 1 - b->cur;
+        (void)hipEventRecord(e0, b->stream);
+        for (int s = 0; s < trial_steps; ++s) {
+            launch_batch_pair(b, b->cur, false);
+            b->cur = 1 - b->cur;
+        }
+        (void)hipEventRecord(e1, b->stream);
+        (void)hipEventSynchronize(e1);
+        float ms = 0.0f;
+        (void)hipEventElapsedTime(&ms, e0, e1);
+        b->pairs = ms < 2 * best;
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     b->threads = bt;
@@ -606,6 +739,7 @@ int lbm_batch_set_launch(lbm_batch* b, int threads, int blocks) {
         return lbm_fail(LBM_ERR_ARG, "lbm_batch_set_launch: %d threads x %d blocks", threads, blocks);
     b->threads = threads;
     b->blocks = blocks;
+    b->pairs = false;  // the caller's own launch shape: one-step launches
     return LBM_OK;
 }
 
@@ -614,6 +748,7 @@ int lbm_batch_set_cells_per_thread(lbm_batch* b, int cells_per_thread) {
     if (cells_per_thread != 1 && cells_per_thread != 2 && cells_per_thread != 4)
         return lbm_fail(LBM_ERR_ARG, "lbm_batch_set_cells_per_thread: %d (1, 2 or 4)", cells_per_thread);
     b->cpt = cells_per_thread;
+    b->pairs = false;
     return LBM_OK;
 }
 

@@ -1,27 +1,16 @@
 // pair.hip -- launches of the two-step kernel (pair.hpp) for one cavity.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <functional>
+#include <utility>
+
 #include "context.hpp"
 #include "pair.hpp"
 
 using namespace lbm;
 
 namespace {
-
-// Threads of a block (= cells of a plane with its rim), and the waves per SIMD
-// its registers must allow: two planes of 19 populations fill the LDS of a CU in
-// FP64 and FP32 (one block per CU; in FP32 two blocks of 512, with their larger
-// share of rim, took 8 % more time at 256^3).
-template <class S>
-struct PairShape;
-template <>
-struct PairShape<StoreF64> {
-    static constexpr int NT = 512, WAVES = 2;
-};
-template <>
-struct PairShape<StoreF32> {
-    static constexpr int NT = 1024, WAVES = 4;
-};
 
 template <class S, int COLL, bool MACRO, bool LOOP>
 __global__ __launch_bounds__(PairShape<S>::NT, PairShape<S>::WAVES) void k_cavity_pair(const PairArgs a) {
@@ -72,55 +61,172 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
 // 5 us and 5.2 TB/s of its traffic.
 // FP16 keeps the one-step kernel: it is bound by VALU issue, of which the rim
 // takes a third more (276 against 238 us a step at 256^3).
-bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out) {
-    const double bytes = elem, share = pops / 19.0;
-    const bool cached = double(nx) * ny * nz * 2 * pops * bytes < 200e6;
-    const long long plane = ((long long)nx + 15) / 16 * 16 * ny;
-    if (plane * (long long)bytes >= PLANE_RANGE) return false;  // the lanes' offsets
-    double best = 1e30;
-    auto consider = [&](int tx) {
-        PairTiles t{};
-        t.tx = tx;
-        t.ntx = (nx + tx - 1) / tx;
-        t.hx = t.ntx > 1;
-        t.w = tx + 2 * t.hx;
-        if (t.w > nt) return;
-        const int rows = nt / t.w;
-        if (rows >= ny) {
-            t.ty = ny;
-        } else if (rows >= 3) {
-            t.nty = (ny + rows - 3) / (rows - 2);
-            t.ty = (ny + t.nty - 1) / t.nty;  // even tiles
-        } else {
-            return;
+namespace {
+
+// Tiles of width tx for an nx x ny plane; false where nt threads cannot hold them.
+bool tiles_of_width(int nx, int ny, int nt, int tx, PairTiles* out) {
+    PairTiles t{};
+    t.tx = tx;
+    t.ntx = (nx + tx - 1) / tx;
+    t.hx = t.ntx > 1;
+    t.w = tx + 2 * t.hx;
+    if (t.w > nt) return false;
+    const int rows = nt / t.w;
+    if (rows >= ny) {
+        t.ty = ny;
+    } else if (rows >= 3) {
+        t.nty = (ny + rows - 3) / (rows - 2);
+        t.ty = (ny + t.nty - 1) / t.nty;  // even tiles
+    } else {
+        return false;
+    }
+    t.nty = (ny + t.ty - 1) / t.ty;
+    t.hy = t.nty > 1;
+    t.h = t.ty + 2 * t.hy;
+    *out = t;
+    return true;
+}
+
+template <class F>
+void for_widths(int nx, F&& f) {
+    for (int tx = 32; tx < nx && tx <= 128; tx += 32) f(tx);
+    for (int n = 1; n <= 4; ++n) f((nx + n - 1) / n);
+}
+
+// us of a turn (see above); busy: the share of the CUs at work.
+double turn_us(const PairTiles& t, double bytes, int pops, bool cached, double busy) {
+    const double moved = t.h * (t.w * bytes + 128.0) + t.tx * t.ty * bytes;
+    double turn = (cached ? 5.0e-4 : 7.7e-4) * (pops / 19.0) * moved * (0.5 + 0.5 * busy);
+    if (!cached && t.tx % 16 != 0 && t.ntx > 1) turn *= 1.2;
+    return turn < 4.3 ? 4.3 : turn;
+}
+
+// us of a launch of blocks of given times and counts, one block per CU.
+double launch_us(std::vector<std::pair<double, long long>> runs, int cus) {
+    std::sort(runs.rbegin(), runs.rend());
+    std::vector<double> free(cus, 0.0);  // a heap: when each CU is free, the first in front
+    double end = 0;
+    long long steps = 0;
+    for (const auto& r : runs)
+        for (long long n = 0; n < r.second; ++n) {
+            if (++steps > 16LL * cus) {  // long launches: the mean, and the last blocks
+                double rest = r.first * double(r.second - n);
+                for (const auto* q = &r + 1; q != runs.data() + runs.size(); ++q) rest += q->first * double(q->second);
+                return end + rest / cus;
+            }
+            std::pop_heap(free.begin(), free.end(), std::greater<double>());
+            free.back() += r.first;
+            end = std::max(end, free.back());
+            std::push_heap(free.begin(), free.end(), std::greater<double>());
         }
-        t.nty = (ny + t.ty - 1) / t.ty;
-        t.hy = t.nty > 1;
-        t.h = t.ty + 2 * t.hy;
+    return end;
+}
+
+double one_step_us(double cells, double bytes, int pops) { return cells * 2 * pops * bytes / 5.2e6 + 5.0; }
+bool in_cache(double cells, double bytes, int pops) { return cells * 2 * pops * bytes < 200e6; }
+
+}  // namespace
+
+bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out) {
+    const double bytes = elem, cells = double(nx) * ny * nz;
+    const bool cached = in_cache(cells, bytes, pops);
+    if (((long long)nx + 15) / 16 * 16 * ny * elem >= (long long)PLANE_RANGE) return false;  // the lanes' offsets
+    double best = 1e30;
+    for_widths(nx, [&](int tx) {
+        PairTiles t;
+        if (!tiles_of_width(nx, ny, nt, tx, &t)) return;
         for (int ncz = 1; ncz <= nz; ++ncz) {
             t.cz = (nz + ncz - 1) / ncz;
             t.ncz = (nz + t.cz - 1) / t.cz;
             const long long blocks = (long long)t.ntx * t.nty * t.ncz;
             if (blocks > (1 << 24)) break;
             const long long rounds = (blocks + cus - 1) / cus;
-            const double busy = double(blocks) / double(rounds * cus);
-            const double moved = t.h * (t.w * bytes + 128.0) + t.tx * t.ty * bytes;
-            double turn = (cached ? 5.0e-4 : 7.7e-4) * share * moved * (0.5 + 0.5 * busy);
-            if (!cached && t.tx % 16 != 0 && t.ntx > 1) turn *= 1.2;
-            if (turn < 4.3) turn = 4.3;
+            const double turn = turn_us(t, bytes, pops, cached, double(blocks) / double(rounds * cus));
             const double time = (double(rounds) * (t.cz + 2) * turn + 4.0) / 2;
             if (time < best) {
                 best = time;
                 *out = t;
             }
         }
-    };
-    for (int tx = 32; tx < nx && tx <= 128; tx += 32) consider(tx);
-    for (int n = 1; n <= 4; ++n) consider((nx + n - 1) / n);
-    const double one = double(nx) * ny * nz * 2 * pops * bytes / 5.2e6 + 5.0;
+    });
+    const double one = one_step_us(cells, bytes, pops);
     // (a margin for what the model misses: 0.85 on small boxes, where FP32 with
     // temperature at 51^3 took 10.9 us in pairs, 8.8 one by one)
     return best < (one < 12.0 ? 0.85 : 0.95) * one;
+}
+
+bool pair_batch_plan(const std::vector<PairBox>& boxes, int storage, int cus, std::vector<PairTiles>* tiles,
+                     std::vector<PairBlock>* blocks) {
+    if (storage == LBM_STORE_F16) return false;
+    const bool f64 = storage == LBM_STORE_F64;
+    const int nt = f64 ? PairShape<StoreF64>::NT : PairShape<StoreF32>::NT;
+    const double bytes = f64 ? 8.0 : 4.0;
+    double cells = 0;
+    for (const PairBox& b : boxes) {
+        if (((long long)b.nx + 15) / 16 * 16 * b.ny * (f64 ? 8 : 4) >= (long long)PLANE_RANGE) return false;
+        cells += double(b.nx) * b.ny * b.nz;
+    }
+    const bool cached = in_cache(cells, bytes, Q);
+    // each box's tiles in the plane: those whose turns take least together
+    std::vector<PairTiles> cand(boxes.size());
+    std::vector<double> turn(boxes.size());
+    for (size_t m = 0; m < boxes.size(); ++m) {
+        double least = 1e30;
+        for_widths(boxes[m].nx, [&](int tx) {
+            PairTiles t;
+            if (!tiles_of_width(boxes[m].nx, boxes[m].ny, nt, tx, &t)) return;
+            const double us = turn_us(t, bytes, Q, cached, 1.0);
+            if (us * t.ntx * t.nty < least) {
+                least = us * t.ntx * t.nty;
+                turn[m] = us;
+                cand[m] = t;
+            }
+        });
+        if (least > 1e29) return false;
+    }
+    // Chunks of about one time for all boxes: long ones repeat fewer planes, short
+    // ones leave less of the chip idle at the end.  A launch is played through: its
+    // blocks go to the CUs in order, the longest first.
+    double best = 1e30;
+    long long last = 0;
+    std::vector<std::pair<double, long long>> runs(boxes.size());  // a block's time, how many
+    for (double limit = 1000.0; limit > 10.0; limit *= 0.97) {
+        double total = 0;
+        long long count = 0;
+        for (size_t m = 0; m < boxes.size(); ++m) {
+            PairTiles& t = cand[m];
+            const int nz = boxes[m].nz;
+            const int most = std::min(nz, std::max(1, (int)(limit / turn[m]) - 2));  // planes of a chunk
+            t.ncz = (nz + most - 1) / most;
+            t.cz = (nz + t.ncz - 1) / t.ncz;
+            t.ncz = (nz + t.cz - 1) / t.cz;
+            runs[m] = {(t.cz + 2) * turn[m], (long long)t.ntx * t.nty * t.ncz};
+            total += runs[m].first * double(runs[m].second);
+            count += runs[m].second;
+        }
+        if (count == last) continue;  // the same chunks as before
+        last = count;
+        if ((total / cus + 4.0) / 2 >= best) break;
+        const double time = (launch_us(runs, cus) + 4.0) / 2;
+        if (time < best) {
+            best = time;
+            *tiles = cand;
+        }
+    }
+    if (best >= 0.95 * one_step_us(cells, bytes, Q)) return false;
+    blocks->clear();
+    for (size_t m = 0; m < boxes.size(); ++m) {
+        const PairTiles& t = (*tiles)[m];
+        for (int z = 0; z < t.ncz; ++z)
+            for (int y = 0; y < t.nty; ++y)
+                for (int x = 0; x < t.ntx; ++x)
+                    blocks->push_back({(int)m, x * t.tx - t.hx, y * t.ty - t.hy, z * t.cz});
+    }
+    // the longest first
+    std::stable_sort(blocks->begin(), blocks->end(), [&](const PairBlock& a, const PairBlock& b) {
+        return ((*tiles)[a.box].cz + 2) * turn[a.box] > ((*tiles)[b.box].cz + 2) * turn[b.box];
+    });
+    return true;
 }
 
 }  // namespace lbm

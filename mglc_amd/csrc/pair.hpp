@@ -20,6 +20,8 @@
 // of the current one and are in flight behind it and the barriers, which
 // order LDS accesses only.
 #pragma once
+#include <vector>
+
 #include "step.hpp"
 
 namespace lbm {
@@ -258,15 +260,36 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
     if (ze == a.nz) finish(a.nz - 1);  // the top chunk's last plane needs none above it
 }
 
+// Threads of a block (= cells of a plane with its rim), and the waves per SIMD
+// its registers must allow: two planes of 19 populations fill the LDS of a CU in
+// FP64 and FP32 (one block per CU; in FP32 two blocks of 512, with their larger
+// share of rim, took 8 % more time at 256^3).
+template <class S>
+struct PairShape;
+template <>
+struct PairShape<StoreF64> {
+    static constexpr int NT = 512, WAVES = 2;
+};
+template <>
+struct PairShape<StoreF32> {
+    static constexpr int NT = 1024, WAVES = 4;
+};
+
+template <class S, int COLL, bool MACRO, int NT, class MakePost>
+__device__ __forceinline__ void cavity_pair_at(const PairArgs& a, const PairTiles& t, int x0, int y0, int zs,
+                                               typename S::T (&buf)[2][Q][NT], MakePost&& make_post) {
+    if (x0 >= 1 && x0 + t.w <= a.nx - 1 && y0 >= 1 && y0 + t.h <= a.ny - 1)
+        cavity_pair<S, COLL, MACRO, false, NT>(a, t, x0, y0, zs, buf, make_post);
+    else
+        cavity_pair<S, COLL, MACRO, true, NT>(a, t, x0, y0, zs, buf, make_post);
+}
+
 template <class S, int COLL, bool MACRO, int NT, class MakePost>
 __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& t, int wg,
                                             typename S::T (&buf)[2][Q][NT], MakePost&& make_post) {
     const int bx = wg % t.ntx, by = (wg / t.ntx) % t.nty, bz = wg / (t.ntx * t.nty);
     const int x0 = bx * t.tx - t.hx, y0 = by * t.ty - t.hy;
-    if (x0 >= 1 && x0 + t.w <= a.nx - 1 && y0 >= 1 && y0 + t.h <= a.ny - 1)
-        cavity_pair<S, COLL, MACRO, false, NT>(a, t, x0, y0, bz * t.cz, buf, make_post);
-    else
-        cavity_pair<S, COLL, MACRO, true, NT>(a, t, x0, y0, bz * t.cz, buf, make_post);
+    cavity_pair_at<S, COLL, MACRO, NT>(a, t, x0, y0, bz * t.cz, buf, make_post);
 }
 
 // The tiles of the two-step kernel for a box on a device of `cus` CUs; false:
@@ -276,6 +299,17 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out);
 // The same for a two-step kernel with blocks of nt threads that moves `pops`
 // values of `elem` bytes per cell and step each way.
 bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out);
+
+// Many boxes in one launch: each box's tiles and the flat list of blocks; false:
+// the one-step kernel is faster.
+struct PairBox {
+    int nx, ny, nz;
+};
+struct PairBlock {
+    int box, x0, y0, zs;  // the block's first cell with its rim, and its first plane
+};
+bool pair_batch_plan(const std::vector<PairBox>& boxes, int storage, int cus, std::vector<PairTiles>* tiles,
+                     std::vector<PairBlock>* blocks);
 
 }  // namespace lbm
 

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from mglc_amd.hip import Stream, runtime
-from mglc_amd.lbm import Cavity, CavityConfig, ThermalConfig
+from mglc_amd.lbm import Batch, Cavity, CavityConfig, ThermalConfig
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +115,26 @@ def test_steps_captured_into_a_graph_replay():
             hip.hipGraphExecDestroy(ex)
             hip.hipGraphDestroy(graph)
     stream.close()
+
+
+@pytest.mark.parametrize("storage,collision", [("f64", "mrt"), ("f64", "bgk"), ("f32", "mrt"), ("f32", "bgk")])
+def test_batch_of_two_steps_per_launch_equals_one_launch_per_instance(storage, collision):
+    """Uneven boxes (one plane per chunk up to several tiles each way), odd step
+    counts, a graph replay, and one-step launches in between."""
+    shapes = [(n + d, n, n + 2 * d) for n in (5, 17, 33, 65, 48, 64, 64, 64) for d in (0, 3)]
+    cfgs = [CavityConfig(*s, tauf=0.58, U0=0.05 + 0.005 * m, storage=storage, collision=collision)
+            for m, s in enumerate(shapes)]
+    print(f"[gpu] multistep batch {storage} {collision}", flush=True)
+    with Batch(cfgs) as a, Batch(cfgs) as b:
+        a.initial()
+        b.initial()
+        for n in (7, 2, 201):
+            a.step(n)
+            b.step_each(n)
+            for m in range(len(cfgs)):
+                assert all(np.array_equal(x, y) for x, y in zip(a.macro(m), b.macro(m))), (n, shapes[m])
+        a.set_launch(128, 300)
+        a.step(103)
+        b.step_each(103)
+        for m in range(len(cfgs)):
+            assert all(np.array_equal(x, y) for x, y in zip(a.macro(m), b.macro(m))), shapes[m]
