@@ -356,8 +356,8 @@ __device__ __forceinline__ void collide_forced(R f[Q], const Moments<R>& m, cons
 }
 
 // ---- moment transforms -----------------------------------------------------------------
-// For the matrix-core form of the FP16 step and the refill of uncovered nodes,
-// which replaces moments.
+// For the matrix-core form of the FP16 step, the fluid around spheres and the
+// refill of uncovered nodes, which replaces moments.
 // m = M f computed from the opposite-pair sums s_p = f_a + f_abar (even rows)
 // and differences d_p = f_a - f_abar (odd rows); f_post = M^-1 m* likewise
 // from even/odd partial sums E, O with f_a = E + O, f_abar = E - O.

@@ -602,6 +602,61 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_links(const PArgs a) {
     }
 }
 
+// The fluid's moments and collision in the moments' own form (macro.f90:6-25,
+// collision.f90:15-202), summed in the reference's order.  The pair form of
+// relax() would gain nothing here: the fluid kernel is bound by memory (FP32
+// 192^3: 197 us with either).  What it would change is rounding, and a sphere
+// compares: a position that rounds otherwise moves, now and then, the step in
+// which a node changes owner, and the fluid around that node with it (FP32, 1728
+// spheres, 60 steps: one run in some ten, by 2e-4 of the velocity there).
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ Moments<R> fluid_moments(const R f[Q]) {
+    R s = f[0], j[3] = {R(-0.0), R(-0.0), R(-0.0)};
+    sfor<Q - 1>([&](auto B) {
+        constexpr int a = decltype(B)::value + 1;
+        s = s + f[a];
+        if constexpr (EX[a] != 0) j[0] = mac<EX[a]>(j[0], f[a]);
+        if constexpr (EY[a] != 0) j[1] = mac<EY[a]>(j[1], f[a]);
+        if constexpr (EZ[a] != 0) j[2] = mac<EZ[a]>(j[2], f[a]);
+    });
+    Moments<R> m;
+    m.sum = s;
+    m.rho = S::SHIFT ? R(1) + s : s;
+    m.u = j[0] / m.rho;
+    m.v = j[1] / m.rho;
+    m.w = j[2] / m.rho;
+    return m;
+}
+
+template <class S, int COLL, class R = typename S::Real>
+__device__ __forceinline__ void fluid_collide(R f[Q], const Moments<R>& q, const PArgs& a) {
+    const R snu = R(a.snu), sq = R(a.sq);
+    if constexpr (COLL == COLL_BGK) {
+        const R us2 = q.u * q.u + q.v * q.v + q.w * q.w;
+        sfor<Q>([&](auto B) {
+            constexpr int bd = decltype(B)::value;
+            R un = R(-0.0);
+            if constexpr (EX[bd] != 0) un = mac<EX[bd]>(un, q.u);
+            if constexpr (EY[bd] != 0) un = mac<EY[bd]>(un, q.v);
+            if constexpr (EZ[bd] != 0) un = mac<EZ[bd]>(un, q.w);
+            constexpr R wa = R(weight(bd));
+            const R feq = wa * (q.sum + q.rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
+            f[bd] = f[bd] - snu * (f[bd] - feq);
+        });
+    } else {
+        R m[Q], meq[Q];
+        mrt_forward(f, m);
+        mrt_meq(q.rho, q.sum, q.u, q.v, q.w, a.meq12_rho != 0, meq);
+        sfor<Q>([&](auto K) {
+            constexpr int k = decltype(K)::value;
+            constexpr int kind = rate_kind<k>();
+            if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]);
+            else if constexpr (kind == 2) m[k] = m[k] - sq * (m[k] - meq[k]);
+        });
+        mrt_inverse(m, f);
+    }
+}
+
 // The 19 populations node (i, j, k) pulls from the source buffer: pull
 // streaming (fluid.F90:75-161) with halfway bounce-back at the box walls -- a
 // pull out of a solid node reads the interpolated bounce-back value k_links
@@ -636,7 +691,7 @@ __device__ __forceinline__ double pulled_rho(const PArgs& a, int i, int j, int k
     using R = typename S::Real;
     R f[Q];
     pull_node<S>(a, i, j, k, f);
-    const Moments<R> mo = moments<S>(f, a.inv_scale);
+    const Moments<R> mo = fluid_moments<S>(f);
     return density_f64<S>(mo.sum, a.inv_scale);
 }
 
@@ -659,7 +714,7 @@ __global__ __launch_bounds__(256) void k_particle_step(const PArgs a) {
         const int c = i + a.px * (j + a.ny * k);
         R f[Q];
         pull_node<S>(a, i, j, k, f);
-        const Moments<R> mo = moments<S>(f, a.inv_scale);
+        const Moments<R> mo = fluid_moments<S>(f);
         if (a.owner[m] < 0) {
             const double rho = density_f64<S>(mo.sum, a.inv_scale);
             rho_fluid = rho;
@@ -671,7 +726,7 @@ __global__ __launch_bounds__(256) void k_particle_step(const PArgs a) {
                 a.w[m] = double(mo.w);
             }
         }
-        collide<S, COLL>(f, mo, a);
+        fluid_collide<S, COLL>(f, mo, a);
         T* __restrict__ dst = static_cast<T*>(a.dst);
         sfor<Q>([&](auto B) {
             constexpr int bd = decltype(B)::value;
@@ -993,7 +1048,7 @@ __global__ __launch_bounds__(256) void k_particle_init_fields(const PArgs a) {
         f[bd] = S::SHIFT ? R(fe - weight(bd)) : R(fe);
     });
     const Moments<R> mo = moments_of<S>(a.rho0, 0.0, 0.0, 0.0, a.scale);
-    collide<S, COLL>(f, mo, a);
+    fluid_collide<S, COLL>(f, mo, a);
     const int c = i + a.px * (j + a.ny * k);
     T* __restrict__ dst = static_cast<T*>(a.dst);
     sfor<Q>([&](auto B) {
@@ -1072,14 +1127,14 @@ __device__ __forceinline__ void refill_node(const PArgs& a, int i, int j, int k,
     mrt_inverse(mm, fr);
     R f[Q];
     for (int al = 0; al < Q; ++al) f[al] = S::SHIFT ? R(fr[al] - weight(al)) : R(fr[al]);
-    const Moments<R> mo = moments<S>(f, a.inv_scale);
+    const Moments<R> mo = fluid_moments<S>(f);
     const double rho_new = density_f64<S>(mo.sum, a.inv_scale);
     atomicAdd(&a.chain->ref, to_fix(rho_new - a.rho_solid));
     a.rho[m] = rho_new;
     a.u[m] = double(mo.u);
     a.v[m] = double(mo.v);
     a.w[m] = double(mo.w);
-    collide<S, COLL>(f, mo, a);
+    fluid_collide<S, COLL>(f, mo, a);
     const long long c = i + (long long)a.px * (j + (long long)a.ny * k);
     T* __restrict__ dst = static_cast<T*>(a.dst);
     for (int al = 0; al < Q; ++al) st<S>(dst + (long long)al * a.ps + c, f[al], 0u);
