@@ -230,13 +230,6 @@ __device__ __forceinline__ double stream_rho_avg(const PArgs& a) {
     return (ch->sum + (double)(long long)ch->ref / FIX_ONE) / ch->count;
 }
 
-// Absolute population a of a stored state at storage index c.
-template <class S>
-__device__ __forceinline__ double abs_pop(const typename S::T* buf, long long ps, long long c, int a) {
-    const double g = double(ld<S>(buf + (long long)a * ps + c));
-    return S::SHIFT ? g + weight(a) : g;
-}
-
 // Bounding box (0-based cell indices, clamped) of sphere `id` with `margin`.
 __device__ __forceinline__ void sphere_box(const PArgs& a, const double* xc, int id, int margin, int lo[3], int hi[3]) {
     const int n[3] = {a.nx, a.ny, a.nz};
@@ -320,20 +313,22 @@ struct SphereNow {
 //     fluid node's pull along abar reads), and the momentum exchange
 //     (e_a - u_w) f_post(a, x) - (e_abar - u_w) f(abar, x) with its torque
 //     (particle_force.F90:31-92), added to acc.
+template <class S>
 struct LinkWork {
     long long c;
     int al;
     bool near, fl1, in2;
     int o2;
-    double x0, y0, z0, qq, fa, s1, s2;
+    double x0, y0, z0, qq;
+    typename S::Real fa, s1, s2;  // as loaded: converting them here would wait for the loads
 };
 
 template <class S>
-__device__ __forceinline__ LinkWork link_begin(const PArgs& a, const SphereNow& sp, const int (&lo)[3], unsigned it,
+__device__ __forceinline__ LinkWork<S> link_begin(const PArgs& a, const SphereNow& sp, const int (&lo)[3], unsigned it,
                                                bool fl1) {
     using T = typename S::T;
     const T* src = static_cast<const T*>(a.src);
-    LinkWork w;
+    LinkWork<S> w;
     const int al = (int)(it & 31u), bd = OPP[al];
     w.al = al;
     const int i = lo[0] + (int)(it >> 23), j = lo[1] + (int)((it >> 14) & 511u),
@@ -356,20 +351,22 @@ __device__ __forceinline__ LinkWork link_begin(const PArgs& a, const SphereNow& 
     const long long c1 = ci1 + (long long)a.px * (cj1 + (long long)a.ny * ck1);
     const long long c2 = ci2 + (long long)a.px * (cj2 + (long long)a.ny * ck2);
     w.o2 = near ? a.owner[ci2 + (long long)a.nx * (cj2 + (long long)a.ny * ck2)] : 0;
-    w.fa = abs_pop<S>(src, a.ps, c, al);
-    w.s1 = abs_pop<S>(src, a.ps, c1, near ? al : bd);
-    w.s2 = abs_pop<S>(src, a.ps, near ? c2 : c, near ? al : bd);
+    w.fa = ld<S>(src + (long long)al * a.ps + c);
+    w.s1 = ld<S>(src + (long long)(near ? al : bd) * a.ps + c1);
+    w.s2 = ld<S>(src + (long long)(near ? al : bd) * a.ps + (near ? c2 : c));
     return w;
 }
 
 template <class S>
-__device__ __forceinline__ void link_end(const PArgs& a, const SphereNow& sp, const LinkWork& w, double (&acc)[6]) {
+__device__ __forceinline__ void link_end(const PArgs& a, const SphereNow& sp, const LinkWork<S>& w, double (&acc)[6]) {
     using T = typename S::T;
     using R = typename S::Real;
     T* src_w = static_cast<T*>(a.src_w);
     const int al = w.al, bd = OPP[al];
     const double cx = sp.c[0], cy = sp.c[1], cz = sp.c[2];
-    const double x0 = w.x0, y0 = w.y0, z0 = w.z0, qq = w.qq, fa = w.fa, s1 = w.s1, s2 = w.s2;
+    const double x0 = w.x0, y0 = w.y0, z0 = w.z0, qq = w.qq;
+    const double shift = S::SHIFT ? weight(al) : 0.0;  // weight(al) = weight(bd)
+    const double fa = double(w.fa) + shift, s1 = double(w.s1) + shift, s2 = double(w.s2) + shift;
     const bool fl1 = w.fl1, fl2 = w.in2 && w.o2 < 0;
     const double rx0 = x0 - cx, ry0 = y0 - cy, rz0 = z0 - cz;
     const double wx = sp.om[1] * rz0 - sp.om[2] * ry0, wy = sp.om[2] * rx0 - sp.om[0] * rz0,
@@ -431,7 +428,12 @@ __device__ __forceinline__ void link_end(const PArgs& a, const SphereNow& sp, co
 // spheres of one region of the box, fetched less or the same and ran no
 // faster, and neither did more or fewer registers (occupancy); the link pass
 // is bound by its scattered gathers, so what counts is fewer of them and
-// more of them in flight.
+// more of them in flight.  With 1728
+// spheres of radius 6 a launch went from 268 to 236 us with the halvings of calq
+// that end far from the surface taken at once, and to 211 us with calq's band
+// drawn just outside the stop test and the populations kept as loaded until
+// link_end (with no halvings at all: 201).  128 and 512 threads a block: 252 and
+// 239 us; registers for 4 waves per SIMD: the same 211.
 template <class S>
 __global__ __launch_bounds__(SCAN_THREADS) void k_links(const PArgs a) {
     __shared__ int halt;  // read once, so the whole block leaves together (barriers follow)
@@ -582,8 +584,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_links(const PArgs a) {
         const int ee = min(e1, pos - 1);  // past the end: a copy of the last link, computed and dropped
         const unsigned it0 = list[e], it1 = list[ee];
         const bool f0 = fluid1[e] != 0, f1 = fluid1[ee] != 0;
-        const LinkWork w0 = link_begin<S>(a, sp, lo, it0, f0);
-        const LinkWork w1 = link_begin<S>(a, sp, lo, it1, f1);
+        const LinkWork<S> w0 = link_begin<S>(a, sp, lo, it0, f0);
+        const LinkWork<S> w1 = link_begin<S>(a, sp, lo, it1, f1);
         link_end<S>(a, sp, w0, acc);
         if (e1 < pos) link_end<S>(a, sp, w1, acc);
     }
