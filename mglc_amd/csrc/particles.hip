@@ -116,7 +116,7 @@ struct ParticleState {
 namespace {
 
 constexpr double PI = 3.14159265358979323846;
-constexpr int REFILL_BLOCKS = 128;  // k_refill_proc: lanes walk the list with a grid stride
+constexpr int REFILL_BLOCKS = 1024; // k_refill_proc: blocks of one wave, entries dealt to the blocks in turn
 constexpr int GRAPH_STEPS = 10;     // steps per graph replay; even, so the buffers end where they started
 constexpr int SUM_BLOCKS = 256;      // k_refill_scan: at least this many blocks (slices of the fluid sums)
 constexpr int UPDATE_CHUNK = 1024;  // k_particle_update: spheres staged in LDS at a time (32 KiB)
@@ -1185,11 +1185,15 @@ __global__ __launch_bounds__(RED_THREADS) void k_refill_scan(const PArgs a) {
     }
 }
 
+// One lane per listed node.  A refill is 57 scattered loads, so consecutive
+// entries go to different blocks: a full wave's lines would queue in one CU
+// while the others idle (192^3, 1728 spheres: 26.4 us a launch with the list's
+// entries in full waves of 128 blocks, 11.4 dealt to 1024).
 template <class S, int COLL>
-__global__ __launch_bounds__(256) void k_refill_proc(const PArgs a) {
+__global__ __launch_bounds__(64) void k_refill_proc(const PArgs a) {
     if (stopped(a)) return;
     const int count = min(*a.refill_count, a.refill_cap);
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) {
+    for (int t = threadIdx.x * gridDim.x + blockIdx.x; t < count; t += gridDim.x * blockDim.x) {
         const long long m = a.refill[2 * t];
         const int id = a.refill[2 * t + 1];
         const int i = (int)(m % a.nx), j = (int)((m / a.nx) % a.ny), k = (int)(m / ((long long)a.nx * a.ny));
@@ -1384,7 +1388,7 @@ void particle_launches(lbm_ctx* c, hipStream_t st, bool macro) {
     hipLaunchKernelGGL(k_refill_scan, dim3(scan_blocks(np)), dim3(RED_THREADS), 0, st, a);
     hipLaunchKernelGGL(k_fluid_chain, dim3(1), dim3(RED_THREADS), 0, st, a, scan_blocks(np), s->scal);
     a.step_off = 0;
-    hipLaunchKernelGGL((k_refill_proc<S, COLL>), dim3(REFILL_BLOCKS), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_refill_proc<S, COLL>), dim3(REFILL_BLOCKS), dim3(64), 0, st, a);
     s->cur = 1 - s->cur;
     c->cur = 1 - c->cur;
 }
