@@ -122,7 +122,7 @@ def device_warmup(make_ctx, stream, ms=150.0, chunk=20):
     throwaway context of the same configuration (its state is discarded, the
     measured context's is untouched) for about `ms` of device time.  A GPU
     that idled while the host worked (downloads, the previous variant's
-    comparison) starts slow; the VALU-bound FP16 step is the most
+    comparison) starts slow; the FP16 step, near its instruction issue, is the most
     clock-sensitive."""
     from mglc_amd.hip import Event
     done = 0.0
@@ -153,6 +153,9 @@ def traffic_from_profiles(workload_key):
 
 
 def roofline(bytes_per_launch, ms_per_launch, traffic=None):
+    """The rate of a step's algorithmic bytes (one pass over the lattice per
+    step) against the HBM peak.  Launches that make two steps move fewer, so
+    frac may pass 1; `traffic` is what the counters saw per step."""
     achieved = bytes_per_launch / (ms_per_launch * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic}
@@ -228,8 +231,8 @@ def run_storage(args, storage, stream):
     with make() as cav:
         cav.initial()
         warm_ms = device_warmup(make, stream) if args.device_warmup else 0.0
-        # with the loopback every timed step is one launch of the step kernel,
-        # which also writes the outgoing halo (the first, untimed step call
+        # with the loopback the step kernels (FP64 and FP32: two steps per
+        # launch) also write the outgoing halo (the first, untimed step call
         # exchanged the initial state's halo once)
         ms, wall = timed(cav.step, stream, args)
         # a step call writes the macroscopic fields on its last step only:
@@ -356,7 +359,7 @@ def bench_cavity(args, stream):
     m0 = float(primary["fields"][0].size)
     workload = f"lid-driven cavity D3Q19 {args.n}^3 Re=1000 U0=0.1 {args.collision.upper()}"
     config = {"workload": workload, "cells": args.n ** 3, "collision": args.collision,
-              "storage": "f64", "pattern": "A-B pull", "kernel": "k_cavity_step",
+              "storage": "f64", "pattern": "A-B pull, two steps per pass", "kernel": "k_cavity_pair",
               "halo": "6 faces x 5 pops + 12 edges looped back every step (written by the step kernel)"
               if args.halo_loopback else "none",
               "kernel_ms_per_step": round(primary["ms_kernel"] / args.steps, 4),
@@ -418,7 +421,7 @@ def bench_batch(args, stream_unused):
     config = {"workload": f"64 lid-driven cavities D3Q19, N in {{32,48,64,80,96}}^3 (seed 12345), Re U[100,1000], "
                           f"U0 U[0.05,0.1], {args.collision.upper()}, FP32 storage",
               "cells": cells, "instances": len(cfgs), "sizes_present": sizes, "storage": "f32",
-              "kernel": "k_batch_step (persistent, 100-step hipGraph replays)", "threads": threads,
+              "kernel": "k_batch_pair (two steps per launch, 100-step hipGraph replays)", "threads": threads,
               "blocks": blocks, "cells_per_thread": info.cells_per_thread, "graph_steps": info.graph_steps}
     line = line_head(args, mlups, ms / args.steps, "f32", "synthetic (reference initial state per instance)", config)
     # kernel time per launch: the graph holds one step kernel per step and
@@ -580,7 +583,7 @@ def bench_thermal(args, stream):
     bpl = primary["info"].bytes_per_lup
     nu_vol, nu_wall = primary["nu"]
     config = {"workload": f"buoyancy-driven cavity D3Q19+D3Q7 {n}^3 Ra=1e5 Pr=0.71 walls +-0.5, MRT, FP64",
-              "cells": cells, "storage": "f64", "kernel": "k_thermal_step", "bytes_per_lup": bpl,
+              "cells": cells, "storage": "f64", "kernel": "k_thermal_pair", "bytes_per_lup": bpl,
               "device_warmup_ms": primary["warm"]}
     line = line_head(args, mlups, ms / args.steps, "f64",
                      "synthetic (rho=1, u=0, T=0 plus seeded noise +-1e-4, held wall layers)", config)

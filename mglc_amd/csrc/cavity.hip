@@ -860,8 +860,8 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
     // HBM stream keeps more of its locality.  Measured at 256^3 (MRT,
     // alternating runs): 16 waves per CU (four blocks of 256) instead of the
     // 32 the registers allow make the step 0.8-1.8 % faster in FP64 and
-    // 2.6-3.6 % in FP32; FP16, bound by VALU issue, loses 25 % and keeps every
-    // wave, and so do the kernels that read a halo (4 % slower capped: more
+    // 2.6-3.6 % in FP32; FP16 loses 5-25 % (12 waves per CU: half its rate) and
+    // keeps every wave, and so do the kernels that read a halo (4 % slower capped: more
     // registers and work per wave).  The cap is an LDS reservation per block
     // (the CU's LDS over the blocks of the allowed waves) that the kernels
     // never touch.  An explicit waves_per_cu applies to the fused step (also

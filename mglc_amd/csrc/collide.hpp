@@ -246,7 +246,7 @@ __device__ __forceinline__ Moments<R> moments_of(double rho, double u, double v,
 //   f_a, f_abar  +=  Snu/2 (s_eq - s)  +-  Sq/2 (d_eq - d).
 // BGK is the case Sq = Snu = 1/tau.  Against the 19 x 19 transforms the step
 // kernel went from 533 to 389 VALU instructions in FP32 and from 646 to 509 in
-// FP16, which is bound by their issue: 266 -> 249 ms for 800 steps of 256^3
+// FP16, whose time is near its issue: 266 -> 249 ms for 800 steps of 256^3
 // with the fields copied out (about 255 -> 234 us a step).  FP64 and FP32,
 // bound by memory, kept their time.
 // The form updates f by the change alone, so a population's rounding error is

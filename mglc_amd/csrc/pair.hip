@@ -59,8 +59,8 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
 // 32 x 13 with 240 of 256), 0.5 ns in the cache.  Rows that are not whole 64-byte
 // groups cost 1.1 to 1.4 times that outside the cache.  A one-step launch takes
 // 5 us and 5.2 TB/s of its traffic.
-// FP16 keeps the one-step kernel: it is bound by VALU issue, of which the rim
-// takes a third more (276 against 238 us a step at 256^3).
+// FP16 keeps the one-step kernel: half the bytes, but the rim adds a third to its
+// VALU issue, which alone takes 217 us (276 against 238 us a step at 256^3).
 namespace {
 
 // Tiles of width tx for an nx x ny plane; false where nt threads cannot hold them.

@@ -1,7 +1,7 @@
 // thermal.hip -- buoyancy-driven cavity on one MI355X: D3Q19 MRT flow with the
 // Guo body force (Boussinesq + Coriolis) coupled to a D3Q7 MRT temperature
-// field, fused into one pass per step; the thermal residual and the Nusselt
-// reductions.
+// field, fused into one pass per step or per two steps; the thermal residual and
+// the Nusselt reductions.
 //
 // Reference step (bouyancy3d_mpi.F90:222-248, module.F90, evolution_f.F90,
 // evolution_g.F90):
@@ -10,12 +10,12 @@
 //   collisionT (previous u, T), streamingT, bouncebackT
 //   macro (u = (sum f e + F/2) / rho), macroT (T = sum g)
 // Stored between steps: f_post (19), g_post (7) and the force F of the last
-// collision (macro of the next step needs F/2).  One kernel per step:
+// collision (macro of the next step needs F/2).  A step:
 //   pull f and g (+ walls) -> macro with the stored F -> new F -> collide f
 //   and g -> store.
 // Device layout: the SoA layout of the isothermal path; g uses the same
-// population stride; F is three FP64 arrays (only Fz is touched when the
-// rotation rate is zero).
+// population stride; F is three arrays (only Fz is touched when the rotation rate
+// is zero), of which a two-step launch reads one copy and writes another.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -661,8 +661,8 @@ int finish_sums(lbm_ctx* c, double* out) {
 
 size_t thermal_force_elem(const lbm_ctx* c) { return c->p.storage == LBM_STORE_F64 ? sizeof(double) : sizeof(float); }
 
-// The tiles of the two-step kernel; false: one step per launch (FP16, which is
-// bound by VALU issue; a loopback to rehearse; or where one-step launches are
+// The tiles of the two-step kernel; false: one step per launch (FP16, which
+// the rim's extra arithmetic slows; a loopback to rehearse; or where one-step launches are
 // faster).
 bool thermal_pair_plan(const lbm_params& p, int cus, PairTiles* t) {
     if (p.halo_loopback) return false;
