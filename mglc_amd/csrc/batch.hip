@@ -165,7 +165,7 @@ __global__ __launch_bounds__(PairShape<S>::NT, PairShape<S>::WAVES) void k_batch
     a.w = b.w + in.macro_off;
     a.seed = 0;
     cavity_pair_at<S, COLL, MACRO, PairShape<S>::NT>(a, t, blk.x0, blk.y0, blk.zs, buf,
-                                                     [](int, int, int, bool) { return NoPost{}; });
+                                                     [](auto, int, int, int, bool) { return NoPost{}; });
 }
 
 // Equilibrium start + first collision of every instance (the initial state of

@@ -16,8 +16,8 @@ template <class S, int COLL, bool MACRO, bool LOOP>
 __global__ __launch_bounds__(PairShape<S>::NT, PairShape<S>::WAVES) void k_cavity_pair(const PairArgs a) {
     __shared__ typename S::T buf[2][Q][PairShape<S>::NT];
     const int wg = xcd_order(blockIdx.x, gridDim.x);
-    cavity_pair<S, COLL, MACRO, PairShape<S>::NT>(a, a.t, wg, buf, [&](int i, int j, int k, bool mid) {
-        if constexpr (LOOP) return LoopbackHalo<S>{a, mid ? a.halo_mid : a.halo_out, i, j, k};
+    cavity_pair<S, COLL, MACRO, PairShape<S>::NT>(a, a.t, wg, buf, [&](auto edge, int i, int j, int k, bool mid) {
+        if constexpr (LOOP) return LoopbackHalo<S, !decltype(edge)::value>{a, mid ? a.halo_mid : a.halo_out, i, j, k};
         else return NoPost{};
     });
 }

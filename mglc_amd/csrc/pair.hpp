@@ -92,7 +92,7 @@ constexpr int up_slot(int al) { return al == 5 ? 0 : (al < 15 ? al - 10 : al - 1
 static_assert(up_slot(5) == 0 && up_slot(11) == 1 && up_slot(12) == 2 && up_slot(15) == 3 && up_slot(16) == 4,
               "the five velocities with e_z = +1");
 
-// make_post(i, j, k, mid): the hook that sees a cell's stored populations, after the first
+// make_post(edge, i, j, k, mid): the hook that sees a cell's stored populations, after the first
 // (mid) or the second step.
 // EDGE: some cell of the block, rim included, lies on an x or y wall.
 template <class S, int COLL, bool MACRO, bool EDGE, int NT, class MakePost>
@@ -170,7 +170,7 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
             out[al] = S::cvt(f[al], store_random<S, al>(h));
             buf[p & 1][al][tid] = out[al];
         });
-        const auto post = make_post(fresh(i), fresh(j), p, true);
+        const auto post = make_post(std::bool_constant<EDGE>{}, fresh(i), fresh(j), p, true);
         if (post.active() && own && p >= zs && p < ze) post.store(out);
     };
     // Step 2's pull of population al at plane k: from the neighbour's column in
@@ -233,7 +233,7 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
             out[al] = S::cvt(f[al], store_random<S, al>(h));
             plane_store(out[al], plane_of(d + (long long)al * a.ps), where);
         });
-        const auto post = make_post(fresh(i), fresh(j), k, false);
+        const auto post = make_post(std::bool_constant<EDGE>{}, fresh(i), fresh(j), k, false);
         if (post.active() && own) post.store(out);
     };
 

@@ -59,73 +59,59 @@ struct NoPost {
 // or unpack kernel.  (Across GPUs the same stores would go to the
 // neighbour's halo over the peer link.)
 // Only cells on the box's faces store anything and the hook is skipped (one
-// branch) elsewhere.  The x faces are the one lane at each end of a row: it
-// writes its five leaving populations through a base pointer computed once;
-// the rows on y or z faces (whole waves) write theirs and the edges'.
-template <class S>
+// branch) elsewhere.  A box is at least two cells wide, so a cell lies on at most
+// one face of an axis, and both faces of an axis share their five stores: with
+// stores of its own for each face the two-step kernel (four copies of this hook)
+// outgrew the instruction cache (256^3 looped back 654 -> 644 us a step in FP64,
+// 344 -> 334 in FP32; without the exchange 612 and 310).
+// INSIDE: the cell is known to lie on no x or y face.
+template <class S, bool INSIDE = false>
 struct LoopbackHalo {
     const StepArgs& a;
     void* halo_out;  // the halo written
     int i, j, k;
     bool xlo, xhi, ylo, yhi, zlo, zhi;  // the cell lies on that face of the box
     __device__ __forceinline__ LoopbackHalo(const StepArgs& args, void* out, int ci, int cj, int ck)
-        : a(args), halo_out(out), i(ci), j(cj), k(ck), xlo(ci == 0), xhi(ci == args.nx - 1), ylo(cj == 0),
-          yhi(cj == args.ny - 1), zlo(ck == 0), zhi(ck == args.nz - 1) {}
+        : a(args), halo_out(out), i(ci), j(cj), k(ck), xlo(!INSIDE && ci == 0), xhi(!INSIDE && ci == args.nx - 1),
+          ylo(!INSIDE && cj == 0), yhi(!INSIDE && cj == args.ny - 1), zlo(ck == 0), zhi(ck == args.nz - 1) {}
     __device__ __forceinline__ bool active() const { return xlo || xhi || ylo || yhi || zlo || zhi; }
 
-    // the populations leaving through x face `leave` (sign SX), into the
-    // incoming region of the opposite face
-    template <int SX, class T>
-    __device__ __forceinline__ void x_face(T* out, const T (&v)[Q]) const {
-        constexpr int leave = SX > 0 ? LBM_FACE_XP : LBM_FACE_XM, arrive = leave ^ 1;
+    // the populations leaving through the upper (hi) or lower face of an axis,
+    // into the incoming region of the opposite face; at: the cell's place in a
+    // plane of `plane` elements
+    template <int AXIS, class T>
+    __device__ __forceinline__ void face(T* out, const T (&v)[Q], bool hi, long long plane, long long at) const {
+        constexpr int up = 2 * AXIS + 1, down = 2 * AXIS;
+        const int arrive = hi ? down : up;
         if (!((a.loop_mask >> arrive) & 1u)) return;
-        const long long plane = (long long)a.ny * a.nz;
-        T* b = out + a.hoff[arrive] + j + (long long)a.ny * k;
-        sfor<Q>([&](auto A) {
-            constexpr int al = decltype(A)::value;
-            if constexpr (EX[al] == SX) {
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                b[slot * plane] = v[al];
-            }
+        T* b = out + (hi ? a.hoff[down] : a.hoff[up]) + at;
+        sfor<5>([&](auto B) {
+            constexpr int s = decltype(B)::value, pu = leaving_pop(up, s), pd = leaving_pop(down, s);
+            static_assert(pu > 0 && pd > 0 && cross_slot(down, pu, -1) == s && cross_slot(up, pd, -1) == s,
+                          "a population has the slot it leaves with where it arrives");
+            b[s * plane] = hi ? v[pu] : v[pd];
         });
     }
 
     template <class T>
     __device__ __forceinline__ void store(const T (&v)[Q]) const {
         T* out = static_cast<T*>(halo_out);
-        if (xhi) x_face<+1>(out, v);
-        if (xlo) x_face<-1>(out, v);
+        if (xlo || xhi) face<0>(out, v, xhi, (long long)a.ny * a.nz, j + (long long)a.ny * k);
         if (!(ylo || yhi || zlo || zhi)) return;  // uniform over a wave: its row
+        if (ylo || yhi) face<1>(out, v, yhi, (long long)a.nx * a.nz, i + (long long)a.nx * k);
+        if (zlo || zhi) face<2>(out, v, zhi, (long long)a.nx * a.ny, i + (long long)a.nx * j);
+        if (INSIDE) return;
+        // a diagonal population: on its edge when it leaves through both faces
+        // (an edge always has a y or z component)
         const unsigned m = a.loop_mask;
-        sfor<Q>([&](auto A) {
-            constexpr int al = decltype(A)::value;
+        if ((int)(xlo || xhi) + (int)(ylo || yhi) + (int)(zlo || zhi) < 2) return;
+        sfor<Q - 7>([&](auto A) {
+            constexpr int al = decltype(A)::value + 7;
             constexpr int ex = EX[al], ey = EY[al], ez = EZ[al];
-            const bool lx = ex > 0 ? xhi : (ex < 0 ? xlo : false);
-            bool ly = false, lz = false;
-            if constexpr (ey != 0) {
-                constexpr int leave = ey > 0 ? LBM_FACE_YP : LBM_FACE_YM, arrive = leave ^ 1;
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                ly = ey > 0 ? yhi : ylo;
-                if (ly && ((m >> arrive) & 1u))
-                    out[a.hoff[arrive] + (long long)slot * a.nx * a.nz + i + (long long)a.nx * k] = v[al];
-            }
-            if constexpr (ez != 0) {
-                constexpr int leave = ez > 0 ? LBM_FACE_ZP : LBM_FACE_ZM, arrive = leave ^ 1;
-                constexpr int slot = cross_slot(arrive, al, -1);
-                static_assert(slot >= 0 && slot < 5, "a population leaving through a face has one of its 5 slots");
-                lz = ez > 0 ? zhi : zlo;
-                if (lz && ((m >> arrive) & 1u))
-                    out[a.hoff[arrive] + (long long)slot * a.nx * a.ny + i + (long long)a.nx * j] = v[al];
-            }
-            if constexpr (al >= 7) {
-                // a diagonal population: on its edge when it leaves through both
-                // faces (an edge always has a y or z component)
-                constexpr int r = edge_region(al), fa = edge_free_axis(al);
-                const bool on = (ex == 0 || lx) && (ey == 0 || ly) && (ez == 0 || lz);
-                if (on && ((m >> r) & 1u)) out[a.hoff[r] + (fa == 0 ? i : (fa == 1 ? j : k))] = v[al];
-            }
+            const bool lx = ex > 0 ? xhi : xlo, ly = ey > 0 ? yhi : ylo, lz = ez > 0 ? zhi : zlo;
+            constexpr int r = edge_region(al), fa = edge_free_axis(al);
+            const bool on = (ex == 0 || lx) && (ey == 0 || ly) && (ez == 0 || lz);
+            if (on && ((m >> r) & 1u)) out[a.hoff[r] + (fa == 0 ? i : (fa == 1 ? j : k))] = v[al];
         });
     }
 };
