@@ -34,14 +34,18 @@ struct PairTable {
          {k_cavity_pair<S, COLL_BGK, true, false>, k_cavity_pair<S, COLL_BGK, true, true>}}};
 };
 
+// What a turn takes at least, and how its bytes count in the cache (see below).
+constexpr PairCost COST_F64{4.3, 1.0, 0.7}, COST_F32{5.5, 1.2, 0.7};
+constexpr PairCost COST_F64_LOOP{5.8, 1.2, 0.7}, COST_F32_LOOP{7.2, 1.5, 0.7};  // with the looped-back halo's stores
+
 }  // namespace
 
 namespace lbm {
 
-bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
+bool pair_plan(int nx, int ny, int nz, int storage, bool loop, int cus, PairTiles* out) {
     switch (storage) {
-    case LBM_STORE_F64: return pair_plan(nx, ny, nz, PairShape<StoreF64>::NT, Q, 8, cus, out);
-    case LBM_STORE_F32: return pair_plan(nx, ny, nz, PairShape<StoreF32>::NT, Q, 4, cus, out);
+    case LBM_STORE_F64: return pair_plan(nx, ny, nz, PairShape<StoreF64>::NT, Q, 8, loop ? COST_F64_LOOP : COST_F64, cus, out);
+    case LBM_STORE_F32: return pair_plan(nx, ny, nz, PairShape<StoreF32>::NT, Q, 4, loop ? COST_F32_LOOP : COST_F32, cus, out);
     }
     return false;  // FP16: see below
 }
@@ -50,7 +54,10 @@ bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out) {
 //
 // Time goes by turns (planes) of the busiest CU: with one block per CU a launch
 // takes ceil(blocks / CUs) rounds of cz + 2 turns.  A turn takes at least 4.3 us
-// (65^3 and 96^3, which lie in the memory-side cache).  On large boxes it is
+// in FP64, 5.5 in FP32 (twice the cells), 5.8 and 7.2 with the looped-back halo,
+// 5.1 and 5.8 with temperature (medians over 2000 random boxes of 16 to 256 cells a
+// side; with one 4.3 us for all, 8 % of the boxes ran slower in pairs, by up to a
+// fifth; now 1 %, by up to a tenth).  On large boxes it is
 // bound by memory (256^3 FP64: 622 us a step without the arithmetic and LDS, 627
 // with them) and goes as the bytes it moves, a row of the tile and its rim
 // costing 128 bytes more per population than it holds (the lines at its ends):
@@ -94,11 +101,11 @@ void for_widths(int nx, F&& f) {
 }
 
 // us of a turn (see above); busy: the share of the CUs at work.
-double turn_us(const PairTiles& t, double bytes, int pops, bool cached, double busy) {
+double turn_us(const PairTiles& t, double bytes, int pops, PairCost cost, bool cached, double busy) {
     const double moved = t.h * (t.w * bytes + 128.0) + t.tx * t.ty * bytes;
-    double turn = (cached ? 5.0e-4 : 7.7e-4) * (pops / 19.0) * moved * (0.5 + 0.5 * busy);
+    double turn = (cached ? 5.0e-4 * cost.cached : 7.7e-4) * (pops / 19.0) * moved * (0.5 + 0.5 * busy);
     if (!cached && t.tx % 16 != 0 && t.ntx > 1) turn *= 1.2;
-    return turn < 4.3 ? 4.3 : turn;
+    return std::max(turn, cost.least);
 }
 
 // us of a launch of blocks of given times and counts, one block per CU.
@@ -127,7 +134,7 @@ bool in_cache(double cells, double bytes, int pops) { return cells * 2 * pops * 
 
 }  // namespace
 
-bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out) {
+bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, PairCost cost, int cus, PairTiles* out) {
     const double bytes = elem, cells = double(nx) * ny * nz;
     const bool cached = in_cache(cells, bytes, pops);
     if (((long long)nx + 15) / 16 * 16 * ny * elem >= (long long)PLANE_RANGE) return false;  // the lanes' offsets
@@ -141,7 +148,7 @@ bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, Pair
             const long long blocks = (long long)t.ntx * t.nty * t.ncz;
             if (blocks > (1 << 24)) break;
             const long long rounds = (blocks + cus - 1) / cus;
-            const double turn = turn_us(t, bytes, pops, cached, double(blocks) / double(rounds * cus));
+            const double turn = turn_us(t, bytes, pops, cost, cached, double(blocks) / double(rounds * cus));
             const double time = (double(rounds) * (t.cz + 2) * turn + 4.0) / 2;
             if (time < best) {
                 best = time;
@@ -149,10 +156,12 @@ bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, Pair
             }
         }
     });
-    const double one = one_step_us(cells, bytes, pops);
-    // (a margin for what the model misses: 0.85 on small boxes, where FP32 with
-    // temperature at 51^3 took 10.9 us in pairs, 8.8 one by one)
-    return best < (one < 12.0 ? 0.85 : 0.95) * one;
+    // one step per launch: a row's last wave is part empty, which counts where the
+    // lattices lie in the cache
+    const double lanes = double((nx + 63) / 64 * 64) * ny * nz;
+    const double one = one_step_us(cached ? std::max(cells, cost.lanes * lanes) : cells, bytes, pops);
+    // (margins for what the model misses)
+    return best < (one < 16.0 ? 0.9 : 0.95) * one;
 }
 
 bool pair_batch_plan(const std::vector<PairBox>& boxes, int storage, int cus, std::vector<PairTiles>* tiles,
@@ -175,7 +184,7 @@ bool pair_batch_plan(const std::vector<PairBox>& boxes, int storage, int cus, st
         for_widths(boxes[m].nx, [&](int tx) {
             PairTiles t;
             if (!tiles_of_width(boxes[m].nx, boxes[m].ny, nt, tx, &t)) return;
-            const double us = turn_us(t, bytes, Q, cached, 1.0);
+            const double us = turn_us(t, bytes, Q, f64 ? COST_F64 : COST_F32, cached, 1.0);
             if (us * t.ntx * t.nty < least) {
                 least = us * t.ntx * t.nty;
                 turn[m] = us;

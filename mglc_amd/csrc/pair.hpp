@@ -294,11 +294,16 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
 
 // The tiles of the two-step kernel for a box on a device of `cus` CUs; false:
 // the one-step kernel is faster.
-bool pair_plan(int nx, int ny, int nz, int storage, int cus, PairTiles* out);
+bool pair_plan(int nx, int ny, int nz, int storage, bool loop, int cus, PairTiles* out);
 
 // The same for a two-step kernel with blocks of nt threads that moves `pops`
 // values of `elem` bytes per cell and step each way.
-bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, int cus, PairTiles* out);
+struct PairCost {
+    double least;   // us of a turn at least
+    double cached;  // times what a turn's bytes take where the lattices lie in the cache
+    double lanes;   // what a row's idle lanes cost the one-step kernel there, as a share of cells
+};
+bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, PairCost cost, int cus, PairTiles* out);
 
 // Many boxes in one launch: each box's tiles and the flat list of blocks; false:
 // the one-step kernel is faster.

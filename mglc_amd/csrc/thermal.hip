@@ -667,8 +667,10 @@ size_t thermal_force_elem(const lbm_ctx* c) { return c->p.storage == LBM_STORE_F
 bool thermal_pair_plan(const lbm_params& p, int cus, PairTiles* t) {
     if (p.halo_loopback) return false;
     switch (p.storage) {
-    case LBM_STORE_F64: return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF64>::NT, QT + 1, 8, cus, t);
-    case LBM_STORE_F32: return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF32>::NT, QT + 1, 4, cus, t);
+    case LBM_STORE_F64:
+        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF64>::NT, QT + 1, 8, {5.1, 1.2, 0.5}, cus, t);
+    case LBM_STORE_F32:
+        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF32>::NT, QT + 1, 4, {5.8, 1.3, 0.5}, cus, t);
     }
     return false;
 }
