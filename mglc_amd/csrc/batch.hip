@@ -208,6 +208,7 @@ __global__ __launch_bounds__(256) void k_batch_init(const BatchArgs b) {
         InstView a;
         a.snu = in.snu;
         a.sq = in.sq;
+        a.scale = b.scale;
         a.meq12_rho = b.meq12_rho;
         collide<S, COLL>(f, q, a);
         T* dst = static_cast<T*>(b.dst) + in.off;

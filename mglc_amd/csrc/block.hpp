@@ -69,10 +69,10 @@ __device__ __forceinline__ void cavity_block(const BlockArgs& a, const BlockTile
     sfor<Q>([&](auto A) { f[decltype(A)::value] = S::val(held[decltype(A)::value]); });
     for (int step = 1;; ++step) {
         if (top) {
-            f[13] = lid_bounce<S>(f[13], rho_top, a.u_lid, a.scale, true);
-            f[14] = lid_bounce<S>(f[14], rho_top, a.u_lid, a.scale, false);
+            f[13] = lid_bounce<S, COLL>(f[13], rho_top, a.u_lid, a.scale, true);
+            f[14] = lid_bounce<S, COLL>(f[14], rho_top, a.u_lid, a.scale, false);
         }
-        const Moments<R> m = moments<S>(f, a.inv_scale);
+        const Moments<R> m = moments<S, COLL>(f, a.inv_scale);
         if (top) rho_top = density_f64<S>(m.sum, a.inv_scale);
         const bool last = step == b.steps;
         if constexpr (MACRO) {

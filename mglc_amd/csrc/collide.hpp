@@ -45,6 +45,11 @@ __device__ __forceinline__ R mac(R acc, R x) {
 // the velocity (a ratio) and rho = 1 + drho, so it runs in those units and only
 // these two need the scale: no population is scaled on load or store, and a
 // power-of-two scale changes no bit of the result.
+// MOMENTS: the collision runs in the reference's 19 moments (collide_moments);
+// else in pair form (relax).  FP16 keeps the moments: in pair form its kernel
+// takes 509 VALU instructions instead of 646 (256^3: 234 us a step against 255),
+// but the last bits of a population then differ, and with them which way its
+// store rounds, so that a run goes another, equally far off, way.
 // Stores are non-temporal: the next step reads the written lattice only after
 // the whole sweep, so caching the lines on the way out buys nothing (measured
 // 2-4% faster at 256^3).
@@ -54,6 +59,7 @@ struct StoreF64 {
     using Real = double;
     static constexpr bool SHIFT = false;
     static constexpr bool SCALED = false;
+    static constexpr bool MOMENTS = false;
     static constexpr bool RANDOM = false;
     static constexpr int BYTES = 8;
     __device__ __forceinline__ static Real val(T v) { return v; }
@@ -65,6 +71,7 @@ struct StoreF32 {
     using Real = float;
     static constexpr bool SHIFT = true;
     static constexpr bool SCALED = false;
+    static constexpr bool MOMENTS = false;
     static constexpr bool RANDOM = false;
     static constexpr int BYTES = 4;
     __device__ __forceinline__ static Real val(T v) { return v; }
@@ -102,6 +109,7 @@ struct StoreF16 {
     using Real = float;
     static constexpr bool SHIFT = true;
     static constexpr bool SCALED = true;
+    static constexpr bool MOMENTS = true;
     static constexpr bool RANDOM = true;
     static constexpr int BYTES = 2;
     __device__ __forceinline__ static Real val(T v) { return static_cast<float>(v); }
@@ -136,6 +144,13 @@ __device__ __forceinline__ unsigned store_random(unsigned h) {
     else
         return 0u;
 }
+
+enum { COLL_MRT = 0, COLL_BGK = 1 };
+
+// The collision runs as the reference writes it (collide_moments), not in pair
+// form.
+template <class S, int COLL>
+constexpr bool reference_form = S::MOMENTS;
 
 // ---- macroscopic moments (macro.f90:6-25) ---------------------------------------
 template <class R>
@@ -206,16 +221,53 @@ __device__ __forceinline__ void population_sums(const R f[Q], R& sum, R j[3]) {
     j[2] = (f[5] - f[6]) + ((xz1 + xz2) + (yz1 + yz2));
 }
 
+// The same sums with a = 0..18 in order, as the reference accumulates them.
+template <class R>
+__device__ __forceinline__ void population_sums_in_order(const R f[Q], R& sum, R j[3]) {
+    sum = f[0];
+    for (int d = 0; d < 3; ++d) j[d] = R(-0.0);
+    sfor<Q - 1>([&](auto B) {
+        constexpr int a = decltype(B)::value + 1;
+        sum = sum + f[a];
+        if constexpr (EX[a] != 0) j[0] = mac<EX[a]>(j[0], f[a]);
+        if constexpr (EY[a] != 0) j[1] = mac<EY[a]>(j[1], f[a]);
+        if constexpr (EZ[a] != 0) j[2] = mac<EZ[a]>(j[2], f[a]);
+    });
+}
+
 template <class S, class R = typename S::Real>
+__device__ __forceinline__ void velocity_by_division(Moments<R>& m, float inv_scale) {
+    if constexpr (S::SCALED) {
+        m.u = m.j[0] * R(inv_scale) / m.rho;
+        m.v = m.j[1] * R(inv_scale) / m.rho;
+        m.w = m.j[2] * R(inv_scale) / m.rho;
+    } else {
+        m.u = m.j[0] / m.rho;
+        m.v = m.j[1] / m.rho;
+        m.w = m.j[2] / m.rho;
+    }
+}
+
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ Moments<R> moments_in_order(const R f[Q], float inv_scale) {
+    Moments<R> m;
+    population_sums_in_order(f, m.sum, m.j);
+    m.rho = density<S>(m.sum, inv_scale);
+    velocity_by_division<S>(m, inv_scale);
+    return m;
+}
+
+template <class S, int COLL, class R = typename S::Real>
 __device__ __forceinline__ Moments<R> moments(const R f[Q], float inv_scale) {
 #pragma clang fp contract(off)
+    if constexpr (reference_form<S, COLL>) return moments_in_order<S>(f, inv_scale);
     Moments<R> m;
     population_sums(f, m.sum, m.j);
     m.rho = density<S>(m.sum, inv_scale);
-    const R r = rcp_near(m.rho), k = S::SCALED ? R(inv_scale) : R(1);
-    m.u = quotient(m.j[0] * k, m.rho, r);
-    m.v = quotient(m.j[1] * k, m.rho, r);
-    m.w = quotient(m.j[2] * k, m.rho, r);
+    const R r = rcp_near(m.rho);
+    m.u = quotient(m.j[0], m.rho, r);
+    m.v = quotient(m.j[1], m.rho, r);
+    m.w = quotient(m.j[2], m.rho, r);
     return m;
 }
 
@@ -244,11 +296,9 @@ __device__ __forceinline__ Moments<R> moments_of(double rho, double u, double v,
 // differences d = f_a - f_abar (j, which must not change, is seen to below).
 // So M, the rates and M^-1 are exactly
 //   f_a, f_abar  +=  Snu/2 (s_eq - s)  +-  Sq/2 (d_eq - d).
-// BGK is the case Sq = Snu = 1/tau.  Against the 19 x 19 transforms the step
-// kernel went from 533 to 389 VALU instructions in FP32 and from 646 to 509 in
-// FP16, whose time is near its issue: 266 -> 249 ms for 800 steps of 256^3
-// with the fields copied out (about 255 -> 234 us a step).  FP64 and FP32,
-// bound by memory, kept their time.
+// BGK is the case Sq = Snu = 1/tau.  Against the 19 x 19 transforms the FP32 step
+// kernel went from 533 to 389 VALU instructions; FP64 and FP32, bound by memory,
+// kept their time.
 // The form updates f by the change alone, so a population's rounding error is
 // that of the change and two sums instead of that of ten moments: after 300
 // FP32 steps at 256^3 the velocity is 1e-7 off FP64 where it was 4e-6.
@@ -356,8 +406,8 @@ __device__ __forceinline__ void collide_forced(R f[Q], const Moments<R>& m, cons
 }
 
 // ---- moment transforms -----------------------------------------------------------------
-// For the matrix-core form of the FP16 step, the fluid around spheres and the
-// refill of uncovered nodes, which replaces moments.
+// For the FP16 step, the fluid around spheres and the refill of uncovered nodes,
+// which replaces moments.
 // m = M f computed from the opposite-pair sums s_p = f_a + f_abar (even rows)
 // and differences d_p = f_a - f_abar (odd rows); f_post = M^-1 m* likewise
 // from even/odd partial sums E, O with f_a = E + O, f_abar = E - O.
@@ -412,16 +462,23 @@ __device__ __forceinline__ void mrt_inverse(const R m[Q], R f[Q]) {
     });
 }
 
-// Equilibrium moments (collision.f90:73-91) of rho = 1 + drho with M w =
+// Equilibrium moments (collision.f90:73-91).  SHIFT: of rho = 1 + drho with M w =
 // (1, -11, 3, 0, ...) subtracted, which leaves drho in rows 0..2.
 // meq12_rho selects the thermal form -rho/2 (v^2 - w^2) (evolution_f.F90:75);
-// the cavity form has no rho (collision.f90:85).
-template <class R>
-__device__ __forceinline__ void mrt_meq(R rho, R drho, R u, R v, R w, bool meq12_rho, R meq[Q]) {
+// the cavity form has no rho (collision.f90:85).  In stored units with rho, drho
+// and one times the scale.
+template <bool SHIFT, class R>
+__device__ __forceinline__ void mrt_meq(R rho, R drho, R u, R v, R w, bool meq12_rho, R meq[Q], R one = R(1)) {
     const R us2 = u * u + v * v + w * w;
-    meq[0] = drho;
-    meq[1] = R(-11) * drho + R(19) * rho * us2;
-    meq[2] = R(3) * drho - R(11.0 / 2.0) * rho * us2;
+    if constexpr (SHIFT) {
+        meq[0] = drho;
+        meq[1] = R(-11) * drho + R(19) * rho * us2;
+        meq[2] = R(3) * drho - R(11.0 / 2.0) * rho * us2;
+    } else {
+        meq[0] = rho;
+        meq[1] = rho * (R(-11) + R(19) * us2);
+        meq[2] = rho * (R(3) - R(11.0 / 2.0) * us2);
+    }
     meq[3] = rho * u;
     meq[4] = R(-2.0 / 3.0) * rho * u;
     meq[5] = rho * v;
@@ -431,7 +488,7 @@ __device__ __forceinline__ void mrt_meq(R rho, R drho, R u, R v, R w, bool meq12
     meq[9] = rho * (R(2) * u * u - v * v - w * w);
     meq[10] = R(-0.5) * rho * (R(2) * u * u - v * v - w * w);
     meq[11] = rho * (v * v - w * w);
-    meq[12] = meq12_rho ? R(-0.5) * rho * (v * v - w * w) : R(-0.5) * (v * v - w * w);
+    meq[12] = meq12_rho ? R(-0.5) * rho * (v * v - w * w) : R(-0.5) * one * (v * v - w * w);
     meq[13] = rho * u * v;
     meq[14] = rho * v * w;
     meq[15] = rho * u * w;
@@ -445,6 +502,103 @@ __device__ __forceinline__ void mrt_meq(R rho, R drho, R u, R v, R w, bool meq12
 template <int k>
 constexpr int rate_kind() {
     return (k == 0 || k == 3 || k == 5 || k == 7) ? 0 : ((k == 4 || k == 6 || k == 8 || k >= 16) ? 2 : 1);
+}
+
+// The collision in the moments' own form (collision.f90:15-202; BGK:
+// collision.f90:192-198, feq of initial.f90:63-73), for moments_in_order.  With
+// f - w stored the w-part of feq drops out: w (drho + rho (3 e.u + 4.5 (e.u)^2 -
+// 1.5 u.u)).
+template <class S, bool BGK, class R = typename S::Real>
+__device__ __forceinline__ void collide_moments(R f[Q], const Moments<R>& q, R snu, R sq, bool meq12_rho, float scale) {
+    R one = R(1), rho = q.rho;
+    if constexpr (S::SCALED) {
+        one = R(scale);
+        rho = q.rho * one;
+    }
+    if constexpr (BGK) {
+        const R us2 = q.u * q.u + q.v * q.v + q.w * q.w;
+        sfor<Q>([&](auto B) {
+            constexpr int a = decltype(B)::value;
+            R un = R(-0.0);
+            if constexpr (EX[a] != 0) un = mac<EX[a]>(un, q.u);
+            if constexpr (EY[a] != 0) un = mac<EY[a]>(un, q.v);
+            if constexpr (EZ[a] != 0) un = mac<EZ[a]>(un, q.w);
+            constexpr R wa = R(weight(a));
+            R feq;
+            if constexpr (S::SHIFT)
+                feq = wa * (q.sum + rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
+            else
+                feq = rho * wa * (R(1) + R(3) * un + R(4.5) * un * un - R(1.5) * us2);
+            f[a] = f[a] - snu * (f[a] - feq);
+        });
+    } else {
+        R m[Q], meq[Q];
+        mrt_forward(f, m);
+        mrt_meq<S::SHIFT>(rho, q.sum, q.u, q.v, q.w, meq12_rho, meq, one);
+        sfor<Q>([&](auto K) {
+            constexpr int k = decltype(K)::value;
+            constexpr int kind = rate_kind<k>();
+            if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]);
+            else if constexpr (kind == 2) m[k] = m[k] - sq * (m[k] - meq[k]);
+        });
+        mrt_inverse(m, f);
+    }
+}
+
+// The same with the Guo source in moment space (evolution_f.F90:58-129):
+// m* = m - s (m - meq) + (1 - s/2) S, meq in the thermal form (row 12 with rho).
+// Forces in stored units.
+template <class S, class R = typename S::Real>
+__device__ __forceinline__ void collide_moments_forced(R f[Q], const Moments<R>& q, const R (&F)[3], R snu, R sq,
+                                                       float scale) {
+    const R u = q.u, v = q.v, w = q.w, rho = S::SCALED ? q.rho * R(scale) : q.rho;
+    const R Fx = F[0], Fy = F[1], Fz = F[2];
+    R m[Q], meq[Q], s[Q];
+    mrt_forward(f, m);
+    const R us2 = u * u + v * v + w * w;
+    meq[0] = q.sum;
+    meq[1] = R(-11.0) * q.sum + R(19.0) * rho * us2;
+    meq[2] = R(3.0) * q.sum - R(11.0 / 2.0) * rho * us2;
+    meq[3] = rho * u;
+    meq[4] = R(-2.0 / 3.0) * meq[3];
+    meq[5] = rho * v;
+    meq[6] = R(-2.0 / 3.0) * meq[5];
+    meq[7] = rho * w;
+    meq[8] = R(-2.0 / 3.0) * meq[7];
+    meq[9] = rho * (R(2.0) * u * u - v * v - w * w);
+    meq[10] = R(-0.5) * meq[9];
+    meq[11] = rho * (v * v - w * w);
+    meq[12] = R(-0.5) * meq[11];
+    meq[13] = rho * (u * v);
+    meq[14] = rho * (v * w);
+    meq[15] = rho * (w * u);
+    meq[16] = meq[17] = meq[18] = R(0.0);
+    const R uF = u * Fx + v * Fy + w * Fz;
+    s[0] = R(0.0);
+    s[1] = R(38.0) * uF;
+    s[2] = R(-11.0) * uF;
+    s[3] = Fx;
+    s[4] = R(-2.0 / 3.0) * Fx;
+    s[5] = Fy;
+    s[6] = R(-2.0 / 3.0) * Fy;
+    s[7] = Fz;
+    s[8] = R(-2.0 / 3.0) * Fz;
+    s[9] = R(4.0) * u * Fx - R(2.0) * v * Fy - R(2.0) * w * Fz;
+    s[10] = R(-2.0) * u * Fx + v * Fy + w * Fz;
+    s[11] = R(2.0) * v * Fy - R(2.0) * w * Fz;
+    s[12] = -v * Fy + w * Fz;
+    s[13] = u * Fy + v * Fx;
+    s[14] = v * Fz + w * Fy;
+    s[15] = u * Fz + w * Fx;
+    s[16] = s[17] = s[18] = R(0.0);
+    sfor<Q>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        constexpr int kind = rate_kind<k>();
+        if constexpr (kind == 0) m[k] = m[k] + s[k];
+        else if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]) + (R(1.0) - R(0.5) * snu) * s[k];
+        else m[k] = m[k] - sq * (m[k] - meq[k]) + (R(1.0) - R(0.5) * sq) * s[k];
+    });
+    mrt_inverse(m, f);
 }
 
 // D3Q7 MRT for the temperature (evolution_g.F90:1-57): n = N g,

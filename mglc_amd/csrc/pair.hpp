@@ -148,8 +148,8 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
     };
     // the lid's momentum on the two populations that come down along x
     auto lid = [&](R(&f)[Q], double rho) {
-        f[13] = lid_bounce<S>(f[13], rho, a.u_lid, a.scale, true);
-        f[14] = lid_bounce<S>(f[14], rho, a.u_lid, a.scale, false);
+        f[13] = lid_bounce<S, COLL>(f[13], rho, a.u_lid, a.scale, true);
+        f[14] = lid_bounce<S, COLL>(f[14], rho, a.u_lid, a.scale, false);
     };
     // step 1 on plane p, from `in` into LDS
     auto produce = [&](int p) {
@@ -160,7 +160,7 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
         });
         const bool top = p == a.nz - 1;
         if (top) lid(f, rho_top);
-        const Moments<R> m = moments<S>(f, a.inv_scale);
+        const Moments<R> m = moments<S, COLL>(f, a.inv_scale);
         if (top) rho_top = density_f64<S>(m.sum, a.inv_scale);
         collide<S, COLL>(f, m, a);
         const unsigned h = cell_random<S>(cxy + (long long)a.pxy * p, a.seed);
@@ -212,7 +212,7 @@ __device__ __forceinline__ void cavity_pair(const PairArgs& a, const PairTiles& 
             else f[al] = pull(A, k, c);
         });
         if (top) lid(f, rho_top);
-        const Moments<R> m = moments<S>(f, a.inv_scale);
+        const Moments<R> m = moments<S, COLL>(f, a.inv_scale);
         if (top && own) a.lid_out[lid_idx] = density_f64<S>(m.sum, a.inv_scale);
         if constexpr (MACRO) {
             if (own) {

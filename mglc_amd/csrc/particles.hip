@@ -604,8 +604,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_links(const PArgs a) {
     }
 }
 
-// The fluid's moments and collision in the moments' own form (macro.f90:6-25,
-// collision.f90:15-202), summed in the reference's order.  The pair form of
+// The fluid's moments and collision in the moments' own form.  The pair form of
 // relax() would gain nothing here: the fluid kernel is bound by memory (FP32
 // 192^3: 197 us with either).  What it would change is rounding, and a sphere
 // compares: a position that rounds otherwise moves, now and then, the step in
@@ -613,50 +612,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_links(const PArgs a) {
 // spheres, 60 steps: one run in some ten, by 2e-4 of the velocity there).
 template <class S, class R = typename S::Real>
 __device__ __forceinline__ Moments<R> fluid_moments(const R f[Q]) {
-    R s = f[0], j[3] = {R(-0.0), R(-0.0), R(-0.0)};
-    sfor<Q - 1>([&](auto B) {
-        constexpr int a = decltype(B)::value + 1;
-        s = s + f[a];
-        if constexpr (EX[a] != 0) j[0] = mac<EX[a]>(j[0], f[a]);
-        if constexpr (EY[a] != 0) j[1] = mac<EY[a]>(j[1], f[a]);
-        if constexpr (EZ[a] != 0) j[2] = mac<EZ[a]>(j[2], f[a]);
-    });
-    Moments<R> m;
-    m.sum = s;
-    m.rho = S::SHIFT ? R(1) + s : s;
-    m.u = j[0] / m.rho;
-    m.v = j[1] / m.rho;
-    m.w = j[2] / m.rho;
-    return m;
+    return moments_in_order<S>(f, 1.0f);
 }
 
 template <class S, int COLL, class R = typename S::Real>
 __device__ __forceinline__ void fluid_collide(R f[Q], const Moments<R>& q, const PArgs& a) {
-    const R snu = R(a.snu), sq = R(a.sq);
-    if constexpr (COLL == COLL_BGK) {
-        const R us2 = q.u * q.u + q.v * q.v + q.w * q.w;
-        sfor<Q>([&](auto B) {
-            constexpr int bd = decltype(B)::value;
-            R un = R(-0.0);
-            if constexpr (EX[bd] != 0) un = mac<EX[bd]>(un, q.u);
-            if constexpr (EY[bd] != 0) un = mac<EY[bd]>(un, q.v);
-            if constexpr (EZ[bd] != 0) un = mac<EZ[bd]>(un, q.w);
-            constexpr R wa = R(weight(bd));
-            const R feq = wa * (q.sum + q.rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
-            f[bd] = f[bd] - snu * (f[bd] - feq);
-        });
-    } else {
-        R m[Q], meq[Q];
-        mrt_forward(f, m);
-        mrt_meq(q.rho, q.sum, q.u, q.v, q.w, a.meq12_rho != 0, meq);
-        sfor<Q>([&](auto K) {
-            constexpr int k = decltype(K)::value;
-            constexpr int kind = rate_kind<k>();
-            if constexpr (kind == 1) m[k] = m[k] - snu * (m[k] - meq[k]);
-            else if constexpr (kind == 2) m[k] = m[k] - sq * (m[k] - meq[k]);
-        });
-        mrt_inverse(m, f);
-    }
+    collide_moments<S, COLL == COLL_BGK>(f, q, R(a.snu), R(a.sq), a.meq12_rho != 0, 1.0f);
 }
 
 // The 19 populations node (i, j, k) pulls from the source buffer: pull

@@ -116,13 +116,13 @@ struct LoopbackHalo {
     }
 };
 
-enum { COLL_MRT = 0, COLL_BGK = 1 };
-
 template <class S, int COLL, class Args>
 __device__ __forceinline__ void collide(typename S::Real f[Q], const Moments<typename S::Real>& q, const Args& a) {
     using R = typename S::Real;
     const R snu = R(a.snu);
-    if constexpr (COLL == COLL_BGK)
+    if constexpr (reference_form<S, COLL>)
+        collide_moments<S, COLL == COLL_BGK>(f, q, snu, R(a.sq), a.meq12_rho != 0, a.scale);
+    else if constexpr (COLL == COLL_BGK)
         collide_flow<S, false>(f, q, snu, snu, R(0));
     else
         collide_flow<S, true>(f, q, snu, R(a.sq), a.meq12_rho ? R(0) : R(0.5) * snu);
@@ -131,12 +131,15 @@ __device__ __forceinline__ void collide(typename S::Real f[Q], const Moments<typ
 // The moving lid on the two populations that come down along x
 // (bounce_back.f90:77-78): f(14) = f_post(11) - rho/6 U0, f(13) = f_post(12) -
 // rho/6 (-U0); val is the bounced value, forward for f(13).
-template <class S, class R = typename S::Real>
+template <class S, int COLL, class R = typename S::Real>
 __device__ __forceinline__ R lid_bounce(R val, double rho_lid, double u_lid, float scale, bool forward) {
 #pragma clang fp contract(off)
-    double t = rho_lid / 6.0 * u_lid;
-    if constexpr (S::SCALED) t = t * double(scale);
-    return forward ? R(double(val) + t) : R(double(val) - t);
+    const double t = rho_lid / 6.0;
+    if constexpr (reference_form<S, COLL>) {  // contracted, as the collision there
+        const double lid = S::SCALED ? u_lid * double(scale) : u_lid;
+        return R(fma_(forward ? t : -t, lid, double(val)));
+    }
+    return forward ? R(double(val) + t * u_lid) : R(double(val) - t * u_lid);
 }
 
 // Value pulled from outside the domain for population al at cell (i, j, k):
@@ -145,7 +148,7 @@ __device__ __forceinline__ R lid_bounce(R val, double rho_lid, double u_lid, flo
 // (f(a, x) = f_post(abar, x), bounce_back.f90:6-83), with the moving-lid term
 // when the pull crosses the top wall.  A wall crossed anywhere wins, as the
 // reference's bounceback overwrites what streaming pulled from its halo.
-template <class S, int al, bool HALO, class Args>
+template <class S, int COLL, int al, bool HALO, class Args>
 __device__ __forceinline__ typename S::Real pull_outside(const Args& a, const typename S::T* src,
                                                          int i, int j, int k, int c, bool top,
                                                          double rho_lid) {
@@ -189,7 +192,7 @@ __device__ __forceinline__ typename S::Real pull_outside(const Args& a, const ty
         // the lid is applied last, so it wins over the side walls on these two
         // populations
         if (lid) {
-            val = lid_bounce<S>(val, rho_lid, a.u_lid, a.scale, ex > 0);
+            val = lid_bounce<S, COLL>(val, rho_lid, a.u_lid, a.scale, ex > 0);
         }
     }
     return val;
@@ -219,7 +222,7 @@ __device__ __forceinline__ void mfma_cell(const Args& a, const _Float16* src, _F
             constexpr int al = decltype(A)::value;
             if constexpr (EX[al] != 0) {
                 if ((unsigned)(i - EX[al]) >= (unsigned)a.nx)
-                    h[al] = (_Float16)pull_outside<S, al, HALO>(a, src, i, j, k, c, false, 0.0);
+                    h[al] = (_Float16)pull_outside<S, COLL_MRT, al, HALO>(a, src, i, j, k, c, false, 0.0);
             }
         });
     }
@@ -236,7 +239,7 @@ __device__ __forceinline__ void mfma_cell(const Args& a, const _Float16* src, _F
         a.w[mm] = double(w);
     }
     float meq[Q];
-    mrt_meq(rho, drho, u, v, w, a.meq12_rho != 0, meq);
+    mrt_meq<true>(rho, drho, u, v, w, a.meq12_rho != 0, meq);
     const float snu = float(a.snu), sq = float(a.sq);
     sfor<Q>([&](auto K) {
         constexpr int kk = decltype(K)::value;
@@ -307,7 +310,7 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
                 constexpr int al = decltype(A)::value;
                 if constexpr (EX[al] != 0) {
                     if ((unsigned)(i - EX[al]) >= (unsigned)a.nx)
-                        f[al] = pull_outside<S, al, HALO>(a, src, i, j, k, c, top, rho_lid);
+                        f[al] = pull_outside<S, COLL, al, HALO>(a, src, i, j, k, c, top, rho_lid);
                 }
             });
         }
@@ -327,13 +330,13 @@ __device__ __forceinline__ void cavity_cell(const Args& a, int i, int j, int k, 
                     const long long off = (long long)ex + (long long)ey * a.px + (long long)ez * a.pxy;
                     f[al] = ld<S>(base + (c - off));
                 } else {
-                    f[al] = pull_outside<S, al, HALO>(a, src, i, j, k, c, top, rho_lid);
+                    f[al] = pull_outside<S, COLL, al, HALO>(a, src, i, j, k, c, top, rho_lid);
                 }
             }
         });
     }
 
-    const Moments<R> q = moments<S>(f, a.inv_scale);
+    const Moments<R> q = moments<S, COLL>(f, a.inv_scale);
     if (top) a.lid_rho[lid_idx] = density_f64<S>(q.sum, a.inv_scale);
     if constexpr (MACRO) {
         const long long m = i + (long long)a.nx * (j + (long long)a.ny * k);

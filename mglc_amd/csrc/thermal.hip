@@ -80,13 +80,18 @@ template <class S, class R = typename S::Real>
 __device__ __forceinline__ Moments<R> thermal_moments(const R f[Q], const R (&F0)[3], float inv_scale) {
 #pragma clang fp contract(off)
     Moments<R> m;
-    population_sums(f, m.sum, m.j);
+    if constexpr (S::MOMENTS) population_sums_in_order(f, m.sum, m.j);
+    else population_sums(f, m.sum, m.j);
     m.rho = density<S>(m.sum, inv_scale);
     for (int d = 0; d < 3; ++d) m.j[d] = fma_(R(0.5), F0[d], m.j[d]);
-    const R r = rcp_near(m.rho), k = S::SCALED ? R(inv_scale) : R(1);
-    m.u = quotient(m.j[0] * k, m.rho, r);
-    m.v = quotient(m.j[1] * k, m.rho, r);
-    m.w = quotient(m.j[2] * k, m.rho, r);
+    if constexpr (S::MOMENTS) {
+        velocity_by_division<S>(m, inv_scale);
+    } else {
+        const R r = rcp_near(m.rho);
+        m.u = quotient(m.j[0], m.rho, r);
+        m.v = quotient(m.j[1], m.rho, r);
+        m.w = quotient(m.j[2], m.rho, r);
+    }
     return m;
 }
 
@@ -95,9 +100,9 @@ __device__ __forceinline__ Moments<R> thermal_moments(const R f[Q], const R (&F0
 template <class S, class R = typename S::Real>
 __device__ __forceinline__ R held_wall(const ThermalArgs& a, R bb, bool hot) {
 #pragma clang fp contract(off)
-    R wall = R(a.cw) * R(hot ? a.t_hot : a.t_cold);
-    if constexpr (S::SCALED) wall = wall * R(a.scale);
-    return wall - bb;
+    const R t = R(hot ? a.t_hot : a.t_cold);
+    if constexpr (S::SCALED) return fma_(R(a.cw), t * R(a.scale), -bb);
+    else return R(a.cw) * t - bb;
 }
 
 // The force of the next collision (evolution_f.F90:103-105) from this step's
@@ -108,6 +113,22 @@ __device__ __forceinline__ void body_force(const ThermalArgs& a, const Moments<R
     F[0] = ROT ? R(-2.0) * q.rho * q.v * R(a.omega_rot) : R(0.0);
     F[1] = ROT ? R(2.0) * q.rho * q.u * R(a.omega_rot) : R(0.0);
     F[2] = q.rho * R(a.g_beta) * (T - R(a.t_ref));
+}
+
+// The flow's collision with the new force F and the last one F0 (stored units).  In
+// moments the force is formed here, its last products free to contract into the
+// sums they go to.
+template <class S, bool ROT, class R>
+__device__ __forceinline__ void collide_flow_forced(const ThermalArgs& a, R (&f)[Q], const Moments<R>& q, R T,
+                                                    const R (&F)[3], const R (&F0)[3]) {
+    if constexpr (S::MOMENTS) {
+        const R rho = S::SCALED ? q.rho * R(a.scale) : q.rho;
+        const R Fc[3] = {ROT ? R(-2.0) * rho * q.v * R(a.omega_rot) : R(0.0),
+                         ROT ? R(2.0) * rho * q.u * R(a.omega_rot) : R(0.0), rho * R(a.g_beta) * (T - R(a.t_ref))};
+        collide_moments_forced<S>(f, q, Fc, R(a.snu), R(a.sq), a.scale);
+    } else {
+        collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
+    }
 }
 
 // macroT (evolution_g.F90:202-218): T = sum g, in stored units.
@@ -154,7 +175,7 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
                 // from the halo where every crossed face borders a neighbour,
                 // else bounce-back (no lid: top = false)
                 f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off))
-                           : pull_outside<S, al, true>(a, fsrc, i, j, k, c, false, 0.0);
+                           : pull_outside<S, COLL_MRT, al, true>(a, fsrc, i, j, k, c, false, 0.0);
             } else {
                 f[al] = in ? ld_stream<S>(fsrc + (al * a.ps + c - off))
                            : ld_stream<S>(fsrc + (OPP[al] * a.ps + c));
@@ -209,8 +230,7 @@ __global__ __launch_bounds__(256) void k_thermal_step(const ThermalArgs a) {
     }
     R Fnew[3];  // next collision: force from this step's fields
     body_force<ROT>(a, q, T, Fnew);
-    const R F[3] = {Fnew[0] * unit, Fnew[1] * unit, Fnew[2] * unit};
-    collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
+    collide_flow_forced<S, ROT>(a, f, q, T, Fnew, F0);
     collide_d3q7<R>(g, Ts, u, v, w, R(a.para_a), R(a.qd), R(a.qnu));
     ST* fdst = static_cast<ST*>(a.fdst);
     ST* gdst = static_cast<ST*>(a.gdst);
@@ -341,7 +361,7 @@ __device__ __forceinline__ void thermal_pair(const ThermalPairArgs& a, int x0, i
         const Moments<R> q = thermal_moments<S>(f, F0, a.inv_scale);
         const R Ts = temperature_sum(g);
         body_force<ROT>(a, q, Ts, F);
-        collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
+        collide_flow_forced<S, ROT>(a, f, q, Ts, F, F0);
         collide_d3q7<R>(g, Ts, q.u, q.v, q.w, R(a.para_a), R(a.qd), R(a.qnu));
         return Fields{density_f64<S>(q.sum, a.inv_scale), q.u, q.v, q.w, Ts};
     };
@@ -501,8 +521,11 @@ __global__ __launch_bounds__(256) void k_thermal_init(const ThermalArgs a, const
     const double Fy = 2.0 * rho * u * a.omega_rot;
     const double Fz = rho * a.g_beta * (T - a.t_ref);
     // f = f_eq carries the whole of rho u: no force before it (F0 = 0)
-    const R F[3] = {R(Fx * a.scale), R(Fy * a.scale), R(Fz * a.scale)}, F0[3] = {R(0), R(0), R(0)};
-    collide_forced<S>(f, moments_of<S>(rho, u, v, w, a.scale), F, F0, R(a.snu), R(a.sq));
+    const Moments<R> q = moments_of<S>(rho, u, v, w, a.scale);
+    const R unit = S::SCALED ? R(a.scale) : R(1), F[3] = {R(Fx) * unit, R(Fy) * unit, R(Fz) * unit};
+    const R F0[3] = {R(0), R(0), R(0)};
+    if constexpr (S::MOMENTS) collide_moments_forced<S>(f, q, F, R(a.snu), R(a.sq), a.scale);
+    else collide_forced<S>(f, q, F, F0, R(a.snu), R(a.sq));
     collide_d3q7<R>(g, R(T * a.scale), R(u), R(v), R(w), R(a.para_a), R(a.qd), R(a.qnu));
     using Tst = typename S::T;
     Tst* fdst = static_cast<Tst*>(a.fdst);
