@@ -150,7 +150,7 @@ enum { COLL_MRT = 0, COLL_BGK = 1 };
 // The collision runs as the reference writes it (collide_moments), not in pair
 // form.
 template <class S, int COLL>
-constexpr bool reference_form = S::MOMENTS;
+constexpr bool reference_form = S::MOMENTS || (COLL == COLL_BGK && sizeof(typename S::Real) == 8);
 
 // ---- macroscopic moments (macro.f90:6-25) ---------------------------------------
 template <class R>
@@ -301,15 +301,20 @@ __device__ __forceinline__ Moments<R> moments_of(double rho, double u, double v,
 // kept their time.
 // The form updates f by the change alone, so a population's rounding error is
 // that of the change and two sums instead of that of ten moments: after 300
-// FP32 steps at 256^3 the velocity is 1e-7 off FP64 where it was 4e-6.
+// FP32 steps at 256^3 the velocity is 1e-7 off FP64 where it was 4e-6.  In
+// FP64 (40 x 120 x 33, 400 steps, against 80-bit arithmetic) its rms error is
+// 1.3e-16 where the transforms' is 2.5e-16.
 // Mass and momentum are kept by construction, not by coefficients that cancel:
 // f_0 loses what the pair sums gain, and the differences along the axes are
 // what the diagonals leave of the momentum's gain.  Rounded weights
 // (1/18, 1/36, 1/6) do not add up to 1, and in FP32 their few 1e-8 per step
-// act on every cell the same way: mass drifted by 2.4e-7 in 20000 steps.  The
-// FP64 path is compared with the reference's program, whose rounded M^-1 sums
-// to 1 - 2^-54 over a population's column of rho: it loses that share of rho
-// per step (1.1e-12 in 20000 steps), and so does f_0 here.
+// act on every cell the same way: mass drifted by 2.4e-7 in 20000 steps.
+// FP64 follows the transforms in this: M^-1 in FP64 gives back 1 - 2^-54 of rho, so
+// a run in transforms loses that share a step (measured over 20000 steps at 17^3,
+// 64^3 and, with buoyancy, 128^3: 1.107e-12, 1.104e-12, 1.104e-12; the oracle at
+// 128^3: 1.110e-12), and so does f_0 here (1.110e-12).  Without it the density is
+// 1.1e-13 off a 64-bit run in transforms after 2000 steps at 17^3, with it 2e-15.
+// BGK has no M^-1, and in FP64 is taken as the reference writes it.
 //   base  Snu times the sum (rho or its excess), in stored units
 //   C     Snu j: even part    w (base - 3/2 u.C + 9/2 (e.u)(e.C)) - Snu/2 s
 //   B2    Sq j / 12: odd part of the diagonals   e.B2 - Sq/2 d
@@ -318,7 +323,7 @@ __device__ __forceinline__ Moments<R> moments_of(double rho, double u, double v,
 //         evolution_f.F90:75 has it): Snu (rho - 1)(v^2 - w^2) / 2 along row 12
 //         of M^-1, which is -+1/12 on the y / z axes, +-1/24 on the xy / xz
 //         diagonals
-constexpr double REFERENCE_LOSS = 0x1p-54;
+constexpr double TRANSFORM_LOSS = 0x1p-54;
 template <bool ROW12, bool GAIN, class R>
 __device__ __forceinline__ void relax(R f[Q], R sum, R base, const R (&C)[3], const R (&B2)[3], const R (&gain)[3], R u, R v,
                                       R w, R hs, R hd, R k12) {
@@ -363,7 +368,7 @@ __device__ __forceinline__ void relax(R f[Q], R sum, R base, const R (&C)[3], co
     if constexpr (GAIN)
         for (int d = 0; d < 3; ++d) y[d] = y[d] + gain[d];
     R even = (((x[0] + x[1]) + x[2]) + ((x[3] + x[4]) + (x[5] + x[6]))) + (x[7] + x[8]);
-    if constexpr (sizeof(R) == 8) even = fma_(R(0.5 * REFERENCE_LOSS), sum, even);
+    if constexpr (sizeof(R) == 8) even = fma_(R(0.5 * TRANSFORM_LOSS), sum, even);
     f[0] = fma_(R(-2), even, f[0]);
     sfor<NPAIR>([&](auto P) {
         constexpr int p = decltype(P)::value, a = PAIR_A[p], b = OPP[a];
@@ -372,7 +377,7 @@ __device__ __forceinline__ void relax(R f[Q], R sum, R base, const R (&C)[3], co
     });
 }
 
-// One isothermal collision with rates snu, sq (BGK: both 1/tau, no row 12).
+// One isothermal collision with rates snu, sq (FP32 BGK: both 1/tau, no row 12).
 template <class S, bool ROW12, class R = typename S::Real>
 __device__ __forceinline__ void collide_flow(R f[Q], const Moments<R>& m, R snu, R sq, R row12) {
 #pragma clang fp contract(off)
@@ -517,6 +522,9 @@ __device__ __forceinline__ void collide_moments(R f[Q], const Moments<R>& q, R s
     }
     if constexpr (BGK) {
         const R us2 = q.u * q.u + q.v * q.v + q.w * q.w;
+        // FP64: contracted by hand, the same in every kernel (left to the compiler the
+        // block kernel's came out otherwise)
+        const R us2c = fma_(q.w, q.w, fma_(q.u, q.u, q.v * q.v));
         sfor<Q>([&](auto B) {
             constexpr int a = decltype(B)::value;
             R un = R(-0.0);
@@ -524,12 +532,13 @@ __device__ __forceinline__ void collide_moments(R f[Q], const Moments<R>& q, R s
             if constexpr (EY[a] != 0) un = mac<EY[a]>(un, q.v);
             if constexpr (EZ[a] != 0) un = mac<EZ[a]>(un, q.w);
             constexpr R wa = R(weight(a));
-            R feq;
-            if constexpr (S::SHIFT)
-                feq = wa * (q.sum + rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
-            else
-                feq = rho * wa * (R(1) + R(3) * un + R(4.5) * un * un - R(1.5) * us2);
-            f[a] = f[a] - snu * (f[a] - feq);
+            if constexpr (S::SHIFT) {
+                const R feq = wa * (q.sum + rho * (R(3) * un + R(4.5) * un * un - R(1.5) * us2));
+                f[a] = f[a] - snu * (f[a] - feq);
+            } else {
+                const R X = fma_(R(-1.5), us2c, fma_(R(4.5) * un, un, fma_(R(3), un, R(1))));
+                f[a] = fma_(-snu, fma_(-(rho * wa), X, f[a]), f[a]);
+            }
         });
     } else {
         R m[Q], meq[Q];
