@@ -1068,19 +1068,20 @@ int lbm_step(lbm_ctx* c, int nsteps) {
     }
     const unsigned lds = c->p.halo_faces ? c->step_lds_halo : c->step_lds;  // by default the halo-reading
                                                                             // kernel keeps every wave
-    // as many steps per launch as the plan makes; what is left of the count goes
-    // first, one by one
+    // as many steps per launch as the plan makes, in an even number of such
+    // launches; what is left of the count goes first
     PairArgs pa;
     BlockArgs ba;
     const StepPlan& plan = *c->plan;
     const int group = plan.kind == StepPlan::ONE || step_capturing(c) ? 1 : plan.kind == StepPlan::BLOCK ? plan.block.steps : 2;
+    StepGroups groups(nsteps, group);
     for (int s = 0; s < nsteps;) {
         a.src = c->buf[c->cur];
         a.dst = c->buf[1 - c->cur];
         a.seed = (unsigned)(c->itc + s + 1);
         a.halo = c->hin;
         a.halo_out = c->hin_next;
-        const int take = (nsteps - s) % group ? 1 : group;
+        const int take = groups.next();
         const bool macro = s + take == nsteps;
         int rc = LBM_OK;
         if (take == 1) {
@@ -1088,6 +1089,7 @@ int lbm_step(lbm_ctx* c, int nsteps) {
         } else if (plan.kind == StepPlan::BLOCK) {
             static_cast<StepArgs&>(ba) = a;
             ba.b = plan.block;
+            ba.b.steps = take;  // (fewer than the rim is made for: some of it is not used)
             ba.lid_out = c->lid_next;
             ba.halo[0] = c->hin_next;
             ba.halo[1] = c->hin;

@@ -50,7 +50,7 @@ struct lbm_ctx {
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;                 // buffer holding the current f_post
     double* lid_mem = nullptr;   // both lid densities (nx * ny each): the current one, and the one a launch of
-    double* lid_rho = nullptr;   // several steps writes, swapped after it
+    double* lid_rho = nullptr;   // several steps writes, swapped after it (twice a call: lid_rho is lid_mem between calls)
     double* lid_next = nullptr;
     double* macro = nullptr;     // rho, u, v, w (4 * n)
     double* prev = nullptr;      // up, vp (2 * n)
@@ -71,7 +71,8 @@ struct lbm_ctx {
     // the body force of the last collision, T and its previous check value
     void* gbuf[2] = {nullptr, nullptr};  // 7 * ps each
     void* force = nullptr;       // Fx, Fy, Fz of the last collision (3 * ps; FP64 with FP64 storage, else FP32)
-    void* force_next = nullptr;  // what a launch of two steps writes, swapped with force after it (where they run)
+    void* force_next = nullptr;  // what a launch of two steps writes, swapped with force after it (where they run;
+                                 // twice a call)
     void* force_mem = nullptr;   // both
     double* temp = nullptr;      // T (n)
     double* prev_t = nullptr;    // wp, Tp for the thermal check (2 * n)
@@ -87,8 +88,8 @@ struct lbm_ctx {
 };
 
 // The context's stream is being captured into a graph: then steps go one per
-// launch, so that an even number of them leaves every buffer where it was and
-// the graph can be replayed.
+// launch, and an even number of them leaves every buffer where it was, as an even
+// number of direct steps does, so the graph can be replayed.
 bool step_capturing(const lbm_ctx* c);
 
 // Thermal path (thermal.hip).

@@ -797,7 +797,7 @@ int thermal_step(lbm_ctx* c, int nsteps) {
     const dim3 grid = thermal_grid(c);
     ThermalPairArgs pa;
     pa.t = c->plan->pair;
-    const bool pairs = c->plan->kind == StepPlan::PAIR && !step_capturing(c);
+    StepGroups groups(nsteps, c->plan->kind == StepPlan::PAIR && !step_capturing(c) ? 2 : 1);
     for (int s = 0; s < nsteps;) {
         if (loop) {
             int rc = halo_loopback_exchange(c);
@@ -809,7 +809,7 @@ int thermal_step(lbm_ctx* c, int nsteps) {
         a.gdst = c->gbuf[1 - c->cur];
         a.force = c->force;
         a.seed = (unsigned)(c->itc + s + 1);
-        if (pairs && (nsteps - s) % 2 == 0) {
+        if (groups.next() == 2) {
             static_cast<ThermalArgs&>(pa) = a;
             pa.force_out = c->force_next;
             int rc = launch_thermal_pair(c, pa, rot, s + 2 == nsteps);
