@@ -247,6 +247,11 @@ int lbm_halo_pack(lbm_ctx *ctx, void *dev_send);
  * halo_faces (and edges between two such faces) are read by the next step. */
 int lbm_halo_unpack(lbm_ctx *ctx, const void *dev_recv);
 
+/* Copy the incoming halo as it stands to the device buffer dev_recv (same
+ * layout): what the last lbm_halo_unpack brought or, with halo_loopback, what
+ * the last step wrote for the next one.  Diagnostics; queued on ctx's stream. */
+int lbm_halo_incoming(lbm_ctx *ctx, void *dev_recv);
+
 /* Copy rho, u, v, w of the last step to host arrays (nx*ny*nz each, x
  * fastest; any pointer may be NULL to skip that field). */
 int lbm_download_macro(lbm_ctx *ctx, double *rho, double *u, double *v, double *w);
@@ -255,6 +260,11 @@ int lbm_download_macro(lbm_ctx *ctx, double *rho, double *u, double *v, double *
 int lbm_synchronize(lbm_ctx *ctx);
 
 int lbm_get_info(const lbm_ctx *ctx, lbm_info *info);
+
+/* How lbm_step steps this context: steps made by its largest launches (1, 2 or
+ * 3; 1 also means one step per launch throughout) and, where that is more than
+ * one, the blocks of such a launch along x, y and z (else 0). */
+int lbm_get_plan(const lbm_ctx *ctx, int *steps, int blocks[3]);
 
 /* ---- checkpoint / restart ---------------------------------------------------
  * Replaces backupData (Buoyancy_driven_cavity/fortran/3d/seq/bouyancy3d.F90:
@@ -362,6 +372,9 @@ int lbm_batch_synchronize(lbm_batch *batch);
 int lbm_batch_download_macro(lbm_batch *batch, int instance, double *rho, double *u, double *v,
                              double *w);
 int lbm_batch_get_info(const lbm_batch *batch, lbm_batch_info *info);
+/* How lbm_batch_step steps: steps per launch (2, or 1) and its blocks; graphs:
+ * how many 100-step graphs were captured so far. */
+int lbm_batch_get_plan(const lbm_batch *batch, int *steps, int *blocks, int *graphs);
 /* ---- diagnostics --------------------------------------------------------------
  * No counterpart in the reference.  Measures, on the current device, the HBM
  * bandwidth (GB/s, read + write) the memory system delivers for the step's

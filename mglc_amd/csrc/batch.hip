@@ -301,6 +301,7 @@ struct lbm_batch {
     int cpt = 1;                   // cells per thread (1, 2 or 4)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    int graphs = 0;                // captured so far
     int graph_cur = -1;            // buffer parity the graph was captured for
     int graph_lcur = 0;            // and of the lid densities
     bool graph_pairs = false;
@@ -413,6 +414,7 @@ int capture_graph(lbm_batch* b, int cur) {
         return lbm_fail(LBM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
     }
     HIP_TRY(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
+    b->graphs += 1;
     b->graph_cur = cur;
     b->graph_lcur = b->lcur;
     b->graph_pairs = b->pairs;
@@ -770,6 +772,14 @@ int lbm_batch_download_macro(lbm_batch* b, int instance, double* rho, double* u,
     for (int q = 0; q < 4; ++q)
         copies[q] = {dst[q], b->macro + q * b->total_cells + in.macro_off, sizeof(double) * in.ncells};
     return lbm_download(b->device, b->stream, copies, 4);
+}
+
+int lbm_batch_get_plan(const lbm_batch* b, int* steps, int* blocks, int* graphs) {
+    if (!b || !steps || !blocks || !graphs) return lbm_fail(LBM_ERR_ARG, "lbm_batch_get_plan: null argument");
+    *steps = b->pairs ? 2 : 1;
+    *blocks = b->pairs ? b->npair : b->blocks;
+    *graphs = b->graphs;
+    return LBM_OK;
 }
 
 int lbm_batch_get_info(const lbm_batch* b, lbm_batch_info* info) {

@@ -1256,6 +1256,12 @@ int lbm_step_end(lbm_ctx* c) {
     return LBM_OK;
 }
 
+int lbm_halo_incoming(lbm_ctx* c, void* dev_recv) {
+    if (!c || !dev_recv) return lbm_fail(LBM_ERR_ARG, "lbm_halo_incoming: null argument");
+    HIP_TRY(hipMemcpyAsync(dev_recv, c->hin, c->elem * (size_t)c->htotal, hipMemcpyDeviceToDevice, c->stream));
+    return LBM_OK;
+}
+
 int lbm_halo_unpack(lbm_ctx* c, const void* dev_recv) {
     if (!c || !dev_recv) return lbm_fail(LBM_ERR_ARG, "lbm_halo_unpack: null argument");
     c->halo_fresh = false;  // not the looped-back halo of the current state any more
@@ -1275,6 +1281,16 @@ int lbm_download_macro(lbm_ctx* c, double* rho, double* u, double* v, double* w)
 int lbm_synchronize(lbm_ctx* c) {
     if (!c) return lbm_fail(LBM_ERR_ARG, "lbm_synchronize: null context");
     HIP_TRY(hipStreamSynchronize(c->stream));
+    return LBM_OK;
+}
+
+int lbm_get_plan(const lbm_ctx* c, int* steps, int blocks[3]) {
+    if (!c || !steps || !blocks) return lbm_fail(LBM_ERR_ARG, "lbm_get_plan: null argument");
+    const StepPlan& s = *c->plan;
+    *steps = s.kind == StepPlan::BLOCK ? s.block.steps : s.kind == StepPlan::PAIR ? 2 : 1;
+    const int pair[3] = {s.pair.ntx, s.pair.nty, s.pair.ncz};
+    for (int d = 0; d < 3; ++d)
+        blocks[d] = s.kind == StepPlan::BLOCK ? s.block.n[d] : s.kind == StepPlan::PAIR ? pair[d] : 0;
     return LBM_OK;
 }
 

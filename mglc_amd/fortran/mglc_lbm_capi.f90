@@ -160,6 +160,17 @@ module mglc_lbm_capi
             type(lbm_info), intent(out) :: info
         end function lbm_get_info
 
+        integer(c_int) function lbm_get_plan(ctx, steps, blocks) bind(C, name='lbm_get_plan')
+            import :: c_int, c_ptr
+            type(c_ptr), value :: ctx
+            integer(c_int), intent(out) :: steps, blocks(3)
+        end function lbm_get_plan
+
+        integer(c_int) function lbm_halo_incoming(ctx, dev_recv) bind(C, name='lbm_halo_incoming')
+            import :: c_int, c_ptr
+            type(c_ptr), value :: ctx, dev_recv
+        end function lbm_halo_incoming
+
         integer(c_int) function lbm_set_stream(ctx, hip_stream) bind(C, name='lbm_set_stream')
             import :: c_int, c_ptr
             type(c_ptr), value :: ctx, hip_stream

@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "lbm_batch_get_info", "lbm_particles_init", "lbm_particles_get", "lbm_particles_map",
     "lbm_state_bytes", "lbm_save_state", "lbm_load_state", "lbm_reynolds", "lbm_bandwidth_probe",
     "lbm_step_begin", "lbm_step_end", "lbm_check_sums_noalloc", "lbm_batch_set_cells_per_thread",
+    "lbm_get_plan", "lbm_batch_get_plan", "lbm_halo_incoming",
 )
 
 FACE_XM, FACE_XP, FACE_YM, FACE_YP, FACE_ZM, FACE_ZP = range(6)
@@ -126,6 +127,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.lbm_halo_buffer_bytes.argtypes = [vp, ctypes.POINTER(ctypes.c_size_t)]
     lib.lbm_halo_pack.argtypes = [vp, vp]
     lib.lbm_halo_unpack.argtypes = [vp, vp]
+    lib.lbm_halo_incoming.argtypes = [vp, vp]
+    lib.lbm_get_plan.argtypes = [vp, ctypes.POINTER(ip), ctypes.POINTER(ip)]
     lib.lbm_batch_create.argtypes = [ctypes.POINTER(LbmParams), ip, ctypes.POINTER(vp)]
     lib.lbm_batch_destroy.argtypes = [vp]
     lib.lbm_batch_initial.argtypes = [vp]
@@ -137,6 +140,7 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.lbm_batch_synchronize.argtypes = [vp]
     lib.lbm_batch_download_macro.argtypes = [vp, ip, dp, dp, dp, dp]
     lib.lbm_batch_get_info.argtypes = [vp, ctypes.POINTER(LbmBatchInfo)]
+    lib.lbm_batch_get_plan.argtypes = [vp, ctypes.POINTER(ip), ctypes.POINTER(ip), ctypes.POINTER(ip)]
     lib.lbm_particles_init.argtypes = [vp, ctypes.POINTER(LbmParticleParams), dp, dp, dp, dp]
     lib.lbm_particles_get.argtypes = [vp, dp, dp, dp, dp, dp]
     lib.lbm_particles_map.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
@@ -503,6 +507,16 @@ class Cavity:
     def halo_unpack(self, dev_ptr: int):
         self._call("lbm_halo_unpack", self._ctx, ctypes.c_void_p(dev_ptr))
 
+    def halo_incoming(self, dev_ptr: int):
+        """Copy of the incoming halo as it stands (lbm_halo_incoming)."""
+        self._call("lbm_halo_incoming", self._ctx, ctypes.c_void_p(dev_ptr))
+
+    def plan(self):
+        """(steps of the largest launches, their blocks along x, y, z)."""
+        steps, blocks = ctypes.c_int(), (ctypes.c_int * 3)()
+        self._call("lbm_get_plan", self._ctx, ctypes.byref(steps), blocks)
+        return steps.value, tuple(blocks)
+
     def macro(self):
         out = [np.empty(self.shape, dtype=np.float64) for _ in range(4)]
         self._call("lbm_download_macro", self._ctx, *[_dp(a) for a in out])
@@ -634,6 +648,12 @@ class Batch:
         inf = LbmBatchInfo()
         self._call("lbm_batch_get_info", self._b, ctypes.byref(inf))
         return inf
+
+    def plan(self):
+        """(steps per launch, its blocks, graphs captured so far)."""
+        out = [ctypes.c_int() for _ in range(3)]
+        self._call("lbm_batch_get_plan", self._b, *[ctypes.byref(x) for x in out])
+        return tuple(x.value for x in out)
 
     def close(self):
         if self._b:
