@@ -22,6 +22,7 @@
 #include "collide.hpp"
 #include "context.hpp"
 #include "pair.hpp"
+#include "plan.hpp"
 #include "step.hpp"
 
 using namespace lbm;
@@ -371,11 +372,14 @@ void launch_batch_pair(lbm_batch* b, int cur, bool macro) {
     b->lcur = 1 - b->lcur;
 }
 
-// nsteps steps from buffer `cur` (in pairs, the odd one first); the last writes
-// the macro fields.  Returns the buffer they end in.
+// nsteps steps from buffer `cur`, two per launch in an even number of launches
+// (what is left goes first), so that an even number of steps ends in the buffers
+// and lid densities it began with and the captured graph stays the right one; the
+// last writes the macro fields.  Returns the buffer they end in.
 int launch_steps(lbm_batch* b, int cur, int nsteps) {
+    StepGroups groups(nsteps, b->pairs ? 2 : 1);
     for (int s = 0; s < nsteps;) {
-        if (b->pairs && (nsteps - s) % 2 == 0) {
+        if (groups.next() == 2) {
             launch_batch_pair(b, cur, s + 2 == nsteps);
             s += 2;
         } else {

@@ -110,3 +110,18 @@ def test_batch(storage, collision):
                 assert all(np.array_equal(x, y) for x, y in zip(a.macro(m), b.macro(m))), (n, shapes[m])
         a.set_launch(128, 300)
         assert a.plan()[:2] == (1, 300)
+
+
+@pytest.mark.parametrize("pairs", [True, False])
+def test_batch_keeps_its_graph(pairs):
+    """Calls of an even number of steps replay the graph of the first one."""
+    cfgs = [CavityConfig(n, n, n, tauf=0.58, storage="f32") for n in (64, 64, 48, 64, 65)]
+    print(f"[gpu] route batch graphs {pairs}", flush=True)
+    with Batch(cfgs) as b:
+        if not pairs:
+            b.set_launch(256, 300)
+        assert b.plan()[0] == (2 if pairs else 1)
+        b.initial()
+        for n in (150, 102, 150, 4, 2, 198, 250):
+            b.step(n)
+        assert b.plan()[2] == 1
