@@ -448,27 +448,31 @@ int default_blocks(int threads, int tiles) {
     return std::min(device_cus() * (512 / waves), (tiles - 1) / waves + 1);
 }
 
-// The blocks of the two-step launches, where they are faster.
-hipError_t plan_pairs(lbm_batch* b) try {
+// The blocks of the two-step launches, where they are faster and what they need
+// fits.
+void plan_pairs(lbm_batch* b) try {
     std::vector<PairBox> boxes;
     for (const BatchInst& in : b->host) boxes.push_back({in.nx, in.ny, in.nz});
     std::vector<PairTiles> tiles;
     std::vector<PairBlock> blocks;
-    if (!pair_batch_plan(boxes, b->p0.storage, device_cus(), &tiles, &blocks)) return hipSuccess;
+    if (!pair_batch_plan(boxes, b->p0.storage, device_cus(), &tiles, &blocks)) return;
     const size_t nt = sizeof(PairTiles) * tiles.size(), nb = sizeof(PairBlock) * blocks.size();
     std::vector<char> both(nt + nb);
     std::memcpy(both.data(), tiles.data(), nt);
     std::memcpy(both.data() + nt, blocks.data(), nb);
-    hipError_t e = hipMalloc(&b->pair_tiles, nt + nb);
+    const size_t lid = sizeof(double) * (size_t)b->total_lid;
+    hipError_t e = hipMalloc(&b->lid[1], lid);
+    if (e == hipSuccess) e = hipMalloc(&b->pair_tiles, nt + nb);
     if (e == hipSuccess) e = hipMemcpy(b->pair_tiles, both.data(), nt + nb, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         b->pair_blocks = reinterpret_cast<PairBlock*>(b->pair_tiles + tiles.size());
         b->npair = (int)blocks.size();
         b->pairs = true;
+        b->device_bytes += (long long)(lid + nt + nb);
+    } else {
+        (void)hipGetLastError();
     }
-    return e;
-} catch (...) {
-    return hipErrorOutOfMemory;
+} catch (...) {  // no host memory for the plan
 }
 
 void release(lbm_batch* b) {
@@ -476,7 +480,8 @@ void release(lbm_batch* b) {
     for (void* p : b->buf)
         if (p) (void)hipFree(p);
     if (b->inst) (void)hipFree(b->inst);
-    if (b->lid[0]) (void)hipFree(b->lid[0]);  // both
+    for (double* p : b->lid)
+        if (p) (void)hipFree(p);
     if (b->pair_tiles) (void)hipFree(b->pair_tiles);
     if (b->macro) (void)hipFree(b->macro);
     if (b->ctr) (void)hipFree(b->ctr);
@@ -559,20 +564,19 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
     for (auto& p : b->buf)
         if (e == hipSuccess) e = hipMalloc(&p, b->elem * (size_t)off);
     if (e == hipSuccess) e = hipMalloc(&b->inst, sizeof(BatchInst) * count);
-    if (e == hipSuccess) e = hipMalloc(&b->lid[0], sizeof(double) * 2 * loff);
-    if (e == hipSuccess) b->lid[1] = b->lid[0] + loff;
+    if (e == hipSuccess) e = hipMalloc(&b->lid[0], sizeof(double) * loff);
     if (e == hipSuccess) e = hipMalloc(&b->macro, sizeof(double) * 4 * moff);
     if (e == hipSuccess) e = hipMalloc(&b->ctr, sizeof(unsigned));
     if (e == hipSuccess)
         e = hipMemcpy(b->inst, b->host.data(), sizeof(BatchInst) * count, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = plan_pairs(b);
     if (e != hipSuccess) {
         release(b);
         delete b;
         (void)hipGetLastError();
         return lbm_fail(LBM_ERR_NOMEM, "lbm_batch_create: %s", hipGetErrorString(e));
     }
-    b->device_bytes = (long long)(2 * b->elem * off + sizeof(double) * (2 * loff + 4 * moff) + sizeof(BatchInst) * count);
+    b->device_bytes = (long long)(2 * b->elem * off + sizeof(double) * (loff + 4 * moff) + sizeof(BatchInst) * count);
+    plan_pairs(b);
     b->threads = 256;
     b->blocks = default_blocks(b->threads, b->total_tiles);
     // single-domain arguments per instance, for the one-launch-per-instance baseline

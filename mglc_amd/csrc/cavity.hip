@@ -642,7 +642,8 @@ InitFn init_fn(const lbm_ctx* c) {
 void release(lbm_ctx* c) {
     for (void* b : c->buf)
         if (b) (void)hipFree(b);
-    if (c->lid_mem) (void)hipFree(c->lid_mem);
+    if (c->lid_rho) (void)hipFree(c->lid_rho);
+    if (c->lid_next) (void)hipFree(c->lid_next);
     if (c->macro) (void)hipFree(c->macro);
     if (c->prev) (void)hipFree(c->prev);
     if (c->red) (void)hipFree(c->red);
@@ -896,11 +897,7 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
     hipError_t e = c->plan ? hipSuccess : hipErrorOutOfMemory;
     for (auto& b : c->buf)
         if (e == hipSuccess) e = hipMalloc(&b, lat);
-    if (e == hipSuccess) e = hipMalloc(&c->lid_mem, sizeof(double) * 2 * p->nx * p->ny);
-    if (e == hipSuccess) {
-        c->lid_rho = c->lid_mem;
-        c->lid_next = c->lid_mem + (size_t)p->nx * p->ny;
-    }
+    if (e == hipSuccess) e = hipMalloc(&c->lid_rho, sizeof(double) * p->nx * p->ny);
     if (e == hipSuccess) e = hipMalloc(&c->macro, sizeof(double) * 4 * c->n);
     if (e == hipSuccess) e = hipMalloc(&c->prev, sizeof(double) * 2 * c->n);
     if (e == hipSuccess) e = hipMalloc(&c->red, sizeof(double) * RED_MAX_SUMS * (RED_BLOCKS + 1));
@@ -912,7 +909,7 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
         (void)hipGetLastError();
         return lbm_fail(LBM_ERR_NOMEM, "lbm_create: hipMalloc failed: %s", hipGetErrorString(e));
     }
-    c->device_bytes = (long long)(2 * lat + sizeof(double) * (2 * p->nx * p->ny + 6 * c->n) +
+    c->device_bytes = (long long)(2 * lat + sizeof(double) * (p->nx * p->ny + 6 * c->n) +
                                   sizeof(double) * RED_MAX_SUMS * (RED_BLOCKS + 1) + 2 * c->elem * c->htotal);
     if (p->thermal) {
         int rc = thermal_alloc(c);
@@ -938,6 +935,17 @@ int lbm_create(const lbm_params* p, lbm_ctx** out) {
         release(c);
         delete c;
         return lbm_fail(LBM_ERR_HIP, "lbm_create: clearing the halo failed");
+    }
+    // What launches of several steps need beside the state, last: where it does not
+    // fit any more, steps go one per launch.
+    if (c->plan->kind != StepPlan::ONE) {
+        const size_t lid = sizeof(double) * p->nx * p->ny;
+        e = p->thermal ? thermal_alloc_next(c) : hipMalloc(&c->lid_next, lid);
+        if (e == hipSuccess && !p->thermal) c->device_bytes += (long long)lid;
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            c->plan->kind = StepPlan::ONE;
+        }
     }
     lbm_staging_user(+1);
     *out = c;

@@ -49,9 +49,9 @@ struct lbm_ctx {
     size_t elem = 8;
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;                 // buffer holding the current f_post
-    double* lid_mem = nullptr;   // both lid densities (nx * ny each): the current one, and the one a launch of
-    double* lid_rho = nullptr;   // several steps writes, swapped after it (twice a call: lid_rho is lid_mem between calls)
-    double* lid_next = nullptr;
+    double* lid_rho = nullptr;   // lid density (nx * ny)
+    double* lid_next = nullptr;  // the one a launch of several steps writes, swapped with lid_rho after it (an even
+                                 // number of times a call)
     double* macro = nullptr;     // rho, u, v, w (4 * n)
     double* prev = nullptr;      // up, vp (2 * n)
     double* red = nullptr;       // per-block partials + totals of the FP64 reductions
@@ -71,9 +71,9 @@ struct lbm_ctx {
     // the body force of the last collision, T and its previous check value
     void* gbuf[2] = {nullptr, nullptr};  // 7 * ps each
     void* force = nullptr;       // Fx, Fy, Fz of the last collision (3 * ps; FP64 with FP64 storage, else FP32)
-    void* force_next = nullptr;  // what a launch of two steps writes, swapped with force after it (where they run;
-                                 // twice a call)
-    void* force_mem = nullptr;   // both
+    void* force_next = nullptr;  // what a launch of two steps writes, swapped with force after it (an even number of
+                                 // times a call); without rotation Fz alone is there, at its place of the three
+    void* force_mem[2] = {nullptr, nullptr};  // where force and force_next were allocated
     double* temp = nullptr;      // T (n)
     double* prev_t = nullptr;    // wp, Tp for the thermal check (2 * n)
     ParticleState* part = nullptr;  // moving spheres, when attached
@@ -98,6 +98,8 @@ bool step_capturing(const lbm_ctx* c);
 // runs it between steps.
 int halo_loopback_exchange(lbm_ctx* c);
 int thermal_alloc(lbm_ctx* c);
+// The second force array of launches of two steps (hipErrorOutOfMemory: without).
+hipError_t thermal_alloc_next(lbm_ctx* c);
 size_t thermal_force_elem(const lbm_ctx* c);  // bytes of one stored force component
 void thermal_release(lbm_ctx* c);
 int thermal_load(lbm_ctx* c, const double* d_rho, const double* d_u, const double* d_v, const double* d_w,

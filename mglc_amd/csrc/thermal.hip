@@ -453,7 +453,7 @@ __device__ __forceinline__ void thermal_pair(const ThermalPairArgs& a, int x0, i
             plane_store(T(0), plane_of(static_cast<T*>(a.fdst) + (long long)decltype(N)::value * 64), NOWHERE);
         });
         for (int d = ROT ? 0 : 2; d < 3; ++d)
-            plane_store(FT(0), plane_of(static_cast<FT*>(a.force_out) + d * 64), NOWHERE);
+            plane_store(FT(0), plane_of(static_cast<FT*>(a.force_out) + d * a.ps), NOWHERE);
         for (int d = 0; d < 3; ++d) before[d] = made[d];
         lds_barrier();
     } while (++p <= zs);
@@ -701,22 +701,31 @@ bool thermal_pair_plan(const lbm_params& p, int cus, PairTiles* t) {
 int thermal_alloc(lbm_ctx* c) {
     const size_t g_bytes = (size_t)c->ps * Q7 * c->elem;
     const size_t f_bytes = 3 * (size_t)c->ps * thermal_force_elem(c);
-    const bool pairs = c->plan->kind == StepPlan::PAIR;  // they read one force and write another
     HIP_TRY(hipMalloc(&c->gbuf[0], g_bytes));
     HIP_TRY(hipMalloc(&c->gbuf[1], g_bytes));
-    HIP_TRY(hipMalloc(&c->force_mem, (pairs ? 2 : 1) * f_bytes));
-    c->force = c->force_mem;
-    if (pairs) c->force_next = static_cast<char*>(c->force_mem) + f_bytes;
+    HIP_TRY(hipMalloc(&c->force_mem[0], f_bytes));
+    c->force = c->force_mem[0];
     HIP_TRY(hipMalloc(&c->temp, (size_t)c->n * sizeof(double)));
     HIP_TRY(hipMalloc(&c->prev_t, 2 * (size_t)c->n * sizeof(double)));
-    c->device_bytes += (long long)(2 * g_bytes + (pairs ? 2 : 1) * f_bytes + 3 * c->n * sizeof(double));
+    c->device_bytes += (long long)(2 * g_bytes + f_bytes + 3 * c->n * sizeof(double));
     return LBM_OK;
+}
+
+hipError_t thermal_alloc_next(lbm_ctx* c) {
+    const int first = c->p.omega_rot != 0.0 ? 0 : 2;  // Fz alone without rotation
+    const size_t component = (size_t)c->ps * thermal_force_elem(c), bytes = (3 - first) * component;
+    const hipError_t e = hipMalloc(&c->force_mem[1], bytes);
+    if (e != hipSuccess) return e;
+    c->force_next = static_cast<char*>(c->force_mem[1]) - first * component;
+    c->device_bytes += (long long)bytes;
+    return e;
 }
 
 void thermal_release(lbm_ctx* c) {
     for (void* b : c->gbuf)
         if (b) (void)hipFree(b);
-    if (c->force_mem) (void)hipFree(c->force_mem);
+    for (void* m : c->force_mem)
+        if (m) (void)hipFree(m);
     if (c->temp) (void)hipFree(c->temp);
     if (c->prev_t) (void)hipFree(c->prev_t);
 }
