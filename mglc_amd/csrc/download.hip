@@ -1,17 +1,24 @@
 // download.hip -- device arrays to the caller's (pageable) host memory.
 //
-// A plain copy into pageable memory runs on one host thread, which also takes
-// the page faults of a fresh array: 10 GB/s for the fields of 256^3 (52 ms, as
-// much as 57 FP64 steps).  Large downloads go through pinned staging instead:
-// a few threads each bring chunks into their own two pinned slots (the device
-// copies the next while the thread empties the last into the caller's array).
-// Measured on MI355X, 256^3, four fields into a fresh array: 52 -> 14.4 ms with
-// four threads (eight: 14.1).
+// A plain copy into pageable memory takes the page faults of a fresh array on one
+// thread: 4.4 GB/s, 123 ms for the four fields of 256^3 (as much as 200 FP64
+// steps); into an array in use, 17 GB/s.  Large downloads go through pinned staging
+// instead: the device copies a chunk into one slot while the one before is copied
+// on into the caller's array.  The calling thread does that by itself at no less
+// than the plain copy's rate (measured on MI355X, ms, plain / by itself: 17 MB
+// fresh 3.8 / 3.5, in use 0.98 / 0.67; 134 MB 31 / 27 and 7.7 / 5.0; beside 16
+// threads that keep all 16 CPUs of the process busy, 17 MB 8.1 / 7.7 and 0.98 /
+// 0.70).  Helper threads take chunks beside it (134 MB fresh 10, 537 MB 39), but
+// are never waited for unless they hold one: with every CPU busy a new thread first
+// runs some 4 ms later, and downloads that waited for their threads took 4.0 ms
+// for 17 and 34 MB in use where the plain copy takes 1.0 and 2.0 (so: 0.9, 1.3).
 #include <hip/hip_runtime.h>
 #include <sched.h>
 
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -20,18 +27,26 @@
 
 namespace {
 
-constexpr size_t CHUNK = 2u << 20;         // bytes of a staging slot
+// Bytes of a staging slot.  A copy command costs the device 15 us, after an idle time
+// over 100 until its clocks are up: 134 MB in chunks of 512 KiB took 6.4 and 30 ms, of
+// 1 MiB 4.4 and 20, of 2 MiB 3.5 and 11.5 (plain 7.7 and 20).
+constexpr size_t CHUNK = 2u << 20;
 constexpr int WORKERS = 4, SLOTS = 2;      // 16 MiB of pinned memory
-constexpr size_t STAGED_FROM = 16u << 20;  // smaller downloads: the plain copy (65^3: 0.55 ms either way)
+// Smaller downloads: the plain copy (65^3, 8.8 MB: 2.1 ms fresh, 0.5 in use).  The
+// first download also pins the slots and takes their page faults, 0.4 ms per MiB,
+// which from here on the faults saved pay for (17 MB into a fresh array from a
+// fresh context: 4.3 ms plain, 2.3).
+constexpr size_t STAGED_FROM = 16u << 20;
 
-// The staging memory, one for the process: pinning it takes some ms, which
-// every context would pay on its first output.  It is taken on the first large
-// download, used by one download at a time (another goes the plain way) and
-// given back with the last context.
+// The staging memory, one for the process: taken on the first large download, used
+// by one download at a time (another goes the plain way) and given back with the
+// last context.
 std::mutex g_mu;
+std::condition_variable g_cv;  // g_helpers fell
 char* g_staging = nullptr;
 bool g_in_use = false;
 int g_users = 0;
+int g_helpers = 0;  // helper threads not at their end yet
 
 char* take_staging() {
     std::lock_guard<std::mutex> lock(g_mu);
@@ -59,44 +74,73 @@ struct Chunk {
     size_t bytes;
 };
 
-// Chunks next, next + 1, ... through two pinned slots.  Stops at the first
-// error, which it returns.
-hipError_t work(int device, hipStream_t stream, const std::vector<Chunk>& chunks, std::atomic<size_t>& next,
-                char* slots) {
-    int caller = device;  // the calling thread takes part and keeps its own device
+// One download: its chunks, who takes the next, and how many are still to come.
+// Helpers hold it too, so that one that starts after the end finds nothing left.
+struct Job {
+    int device;
+    hipStream_t stream;
+    std::vector<Chunk> chunks;
+    std::atomic<size_t> next{0};
+    std::atomic<int> err{hipSuccess};  // the first error; the rest of the chunks is then only counted
+    std::mutex mu;
+    std::condition_variable cv;
+    size_t left = 0;
+
+    void done(size_t n) {
+        std::lock_guard<std::mutex> lock(mu);
+        if ((left -= n) == 0) cv.notify_all();
+    }
+    void failed(hipError_t e) {
+        int none = hipSuccess;
+        err.compare_exchange_strong(none, (int)e);
+    }
+};
+
+// Takes chunks through `slots` until none is left.
+void work(Job& job, char* slots, unsigned event_flags) {
+    size_t c = job.next.fetch_add(1);
+    if (c >= job.chunks.size()) return;  // (nothing of the job is touched after its end)
+    int caller = job.device;  // the calling thread keeps its own device
     (void)hipGetDevice(&caller);
-    hipError_t e = hipSetDevice(device);
-    if (e != hipSuccess) return e;
-    hipEvent_t done[SLOTS] = {};
-    for (auto& ev : done)
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    size_t held[SLOTS];
-    bool full[SLOTS] = {};
-    int at = 0;
-    for (bool more = true; e == hipSuccess;) {
-        const size_t c = more ? next.fetch_add(1) : chunks.size();
-        more = c < chunks.size();
-        if (!more && !full[0] && !full[1]) break;
-        if (more) {
-            e = hipMemcpyAsync(slots + at * CHUNK, chunks[c].src, chunks[c].bytes, hipMemcpyDeviceToHost, stream);
-            if (e == hipSuccess) e = hipEventRecord(done[at], stream);
-            held[at] = c;
-            full[at] = e == hipSuccess;
+    hipEvent_t ready[SLOTS] = {};
+    hipError_t e = hipSetDevice(job.device);
+    for (auto& ev : ready)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, event_flags | hipEventDisableTiming);
+    if (e != hipSuccess) job.failed(e);
+    const Chunk* held[SLOTS] = {};
+    size_t finished = 0;  // told to the job at the end: a helper keeps its slots till then
+    for (int at = 0, full = 0; c < job.chunks.size() || full > 0; at = (at + 1) % SLOTS) {
+        char* slot = slots + at * CHUNK;
+        if (held[at]) {
+            e = hipEventSynchronize(ready[at]);
+            if (e == hipSuccess) std::memcpy(held[at]->dst, slot, held[at]->bytes);
+            else job.failed(e);
+            held[at] = nullptr;
+            --full;
+            ++finished;
         }
-        at = 1 - at;  // the slot filled the turn before
-        if (full[at]) {
-            const hipError_t w = hipEventSynchronize(done[at]);
-            if (e == hipSuccess) e = w;
-            if (e == hipSuccess) std::memcpy(chunks[held[at]].dst, slots + at * CHUNK, chunks[held[at]].bytes);
-            full[at] = false;
+        if (c >= job.chunks.size()) continue;
+        if (job.err.load() == hipSuccess) {
+            const Chunk& k = job.chunks[c];
+            e = hipMemcpyAsync(slot, k.src, k.bytes, hipMemcpyDeviceToHost, job.stream);
+            if (e == hipSuccess) e = hipEventRecord(ready[at], job.stream);
+            if (e == hipSuccess) {
+                held[at] = &k;
+                ++full;
+            } else {
+                job.failed(e);
+                (void)hipStreamSynchronize(job.stream);  // no copy into the slot is left
+                ++finished;
+            }
+        } else {
+            ++finished;
         }
+        c = job.next.fetch_add(1);
     }
-    for (int s = 0; s < SLOTS; ++s) {
-        if (full[s]) (void)hipEventSynchronize(done[s]);  // after an error: no copy into the slot is left
-        if (done[s]) (void)hipEventDestroy(done[s]);
-    }
-    if (caller != device) (void)hipSetDevice(caller);
-    return e;
+    for (hipEvent_t ev : ready)
+        if (ev) (void)hipEventDestroy(ev);
+    if (caller != job.device) (void)hipSetDevice(caller);
+    job.done(finished);
 }
 
 // Memory a device copy can write directly (pinned, managed, a device's).
@@ -114,52 +158,66 @@ int host_threads() {
     return n < WORKERS ? n : WORKERS;
 }
 
+void start_helper(const std::shared_ptr<Job>& job, char* slots) {
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        ++g_helpers;
+    }
+    auto over = [] {
+        std::lock_guard<std::mutex> lock(g_mu);
+        --g_helpers;
+        g_cv.notify_all();
+    };
+    try {
+        // (a blocked wait, not a spinning one: the CPU is the other threads')
+        std::thread([job, slots, over] {
+            work(*job, slots, hipEventBlockingSync);
+            over();
+        }).detach();
+    } catch (...) {  // fewer threads, then
+        over();
+    }
+}
+
 // All chunks through the staging memory; false where that cannot be had.
 bool staged(int device, hipStream_t stream, const lbm_copy* copies, int count, hipError_t* err) {
-    char* slots = take_staging();
-    if (!slots) return false;
-    // One thread waits for the work before, not all of them: waiting spins, and with
-    // a caller's own host threads at work it went over the process's CPU share
-    // (128^3 FP16 in two subdomains, 33 MB each, converted by 16 threads after the
-    // copy: 12 to 48 ms a pass with four waiting, 12.0 with one).
-    *err = hipStreamSynchronize(stream);
-    bool ran = *err != hipSuccess;
-    if (!ran) try {
-        std::vector<Chunk> chunks;
+    std::shared_ptr<Job> job;
+    try {
+        job = std::make_shared<Job>();
         for (int q = 0; q < count; ++q)
             for (size_t o = 0; copies[q].dst && o < copies[q].bytes; o += CHUNK)
-                chunks.push_back({static_cast<char*>(copies[q].dst) + o, static_cast<const char*>(copies[q].src) + o,
-                                  copies[q].bytes - o < CHUNK ? copies[q].bytes - o : CHUNK});
-        std::atomic<size_t> next{0};
-        hipError_t e[WORKERS] = {};
-        std::vector<std::thread> threads;
+                job->chunks.push_back({static_cast<char*>(copies[q].dst) + o, static_cast<const char*>(copies[q].src) + o,
+                                       copies[q].bytes - o < CHUNK ? copies[q].bytes - o : CHUNK});
+    } catch (...) {  // no memory for the list of chunks
+        return false;
+    }
+    char* slots = take_staging();
+    if (!slots) return false;
+    job->device = device;
+    job->stream = stream;
+    job->left = job->chunks.size();
+    *err = hipStreamSynchronize(stream);  // one thread waits for the work before, not all of them
+    if (*err == hipSuccess) {
         const int n = host_threads();
-        threads.reserve(n);
-        try {
-            for (int t = 1; t < n; ++t)
-                threads.emplace_back([&, t] { e[t] = work(device, stream, chunks, next, slots + t * SLOTS * CHUNK); });
-        } catch (...) {  // fewer threads, then
-        }
-        e[0] = work(device, stream, chunks, next, slots);
-        for (auto& t : threads) t.join();
-        *err = hipSuccess;
-        for (hipError_t x : e)
-            if (x != hipSuccess) *err = x;
-        ran = true;
-    } catch (...) {  // no memory for the list of chunks: nothing was started
+        for (int t = 1; t < n; ++t) start_helper(job, slots + t * SLOTS * CHUNK);
+        work(*job, slots, hipEventDefault);
+        std::unique_lock<std::mutex> lock(job->mu);
+        job->cv.wait(lock, [&] { return job->left == 0; });
+        *err = (hipError_t)job->err.load();
     }
     std::lock_guard<std::mutex> lock(g_mu);
     g_in_use = false;
     give_back_locked();
-    return ran;
+    return true;
 }
 
 }  // namespace
 
 void lbm_staging_user(int change) {
-    std::lock_guard<std::mutex> lock(g_mu);
+    std::unique_lock<std::mutex> lock(g_mu);
     g_users += change;
     give_back_locked();
+    if (g_users == 0) g_cv.wait(lock, [] { return g_helpers == 0; });  // none is left in the library
 }
 
 int lbm_download(int device, hipStream_t stream, const lbm_copy* copies, int count) {

@@ -62,10 +62,15 @@ print("ok")
 """
 
 
-@pytest.mark.skipif(not shutil.which("gcc"), reason="gcc not available")
-def test_without_room_for_several_steps(tmp_path):
-    shim = tmp_path / "shim.so"
+def build_shim(folder):
+    shim = folder / "shim.so"
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     os.path.join(ROOT, "tests", "hip_memory_shim.c"), "-o", str(shim)], check=True)
+    return shim
+
+
+@pytest.mark.skipif(not shutil.which("gcc"), reason="gcc not available")
+def test_without_room_for_several_steps(tmp_path):
+    shim = build_shim(tmp_path)
     r = subprocess.run([sys.executable, "-c", PROGRAM, str(shim), ROOT], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
