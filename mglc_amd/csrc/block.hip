@@ -36,20 +36,22 @@ struct BlockTable {
 namespace lbm {
 
 // The blocks: as many steps per launch as still leave no CU more than one
-// workgroup (three, else two).  Measured on MI355X, us per step, one-step
-// launches against blocks of 4 x 4 x 3 with three steps at 17^3 (150 workgroups)
-// and of 6^3 with two at 33^3 (216): FP64 5.4 / 3.0 and 6.8 / 5.2, FP32 4.7 / 2.4
-// and 5.6 / 4.7, FP16 5.8 / 2.6 and 6.4 / 4.8; four steps at 17^3 (729
-// workgroups of 2^3) 6.0, two at 51^3 (729 of 6^3) FP64 12.6 against 13.7, FP32
-// 9.8 against 7.7: past one workgroup a CU the repeated rim costs what it saves.
-// Two steps only where the one-step kernel's waves, 64 cells of a row each, are a
-// third empty or more: 128 x 16 x 16 took 4.9 us in blocks, 4.6 without.
-bool block_plan(int nx, int ny, int nz, int cus, BlockTiles* out) {
+// workgroup (three, else two), in as few workgroups as hold the box.  Measured on
+// MI355X, us per step, one-step launches against blocks of 6 x 3 x 3 with three
+// steps at 17^3 (108 workgroups) and of 6 x 5 x 7 with two at 33^3 (210): FP64 5.0 /
+// 2.9 and 6.8 / 5.1, FP32 4.0 / 2.5 and 5.2 / 4.7, FP16 5.7 / 3.0 and 6.5 / 5.2.
+// Four steps at 17^3 (729 workgroups of 2^3) 6.0, two at 51^3 (729 of 6^3) FP64
+// 12.6 against 13.7, FP32 9.8 against 7.7: past one workgroup a CU the repeated
+// rim costs what it saves.  Two steps only where the one-step kernel's waves, 64
+// cells of a row each, are a third empty or more: 128 x 16 x 16 took 4.9 us in
+// blocks, 4.6 without; in FP32 two fifths or more: at 0.6 to 0.65 full, eight
+// random boxes took 0.96 to 1.22 of the blocks' time (83 x 15 x 25: 4.7 and 4.9 us).
+bool block_plan(int nx, int ny, int nz, int storage, int cus, BlockTiles* out) {
     const int n[3] = {nx, ny, nz};
     // (a box this large cannot be covered; it also bounds the search)
     if ((long long)nx * ny * nz > (long long)cus * NT) return false;
     for (int steps = 3; steps >= 2; --steps) {
-        if (steps == 2 && 3 * nx > 2 * 64 * ((nx + 63) / 64)) return false;
+        if (steps == 2 && nx > (storage == LBM_STORE_F32 ? 0.6 : 2.0 / 3.0) * 64 * ((nx + 63) / 64)) return false;
         long long best = cus + 1;
         // parts along each axis; a part is the written cells of a workgroup
         for (int nbz = 1; nbz <= nz && nbz <= cus; ++nbz)

@@ -113,7 +113,7 @@ __device__ __forceinline__ void cavity_block(const BlockArgs& a, const BlockTile
 
 // The blocks for a box on a device of `cus` CUs; false: another kernel is
 // faster.
-bool block_plan(int nx, int ny, int nz, int cus, BlockTiles* out);
+bool block_plan(int nx, int ny, int nz, int storage, int cus, BlockTiles* out);
 
 }  // namespace lbm
 

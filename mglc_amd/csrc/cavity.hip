@@ -48,7 +48,7 @@ StepPlan make_plan(const lbm_params& p, int device) {
     }
     if (p.thermal) {
         if (thermal_pair_plan(p, cus, &s.pair)) s.kind = StepPlan::PAIR;
-    } else if (block_plan(p.nx, p.ny, p.nz, cus, &s.block)) {
+    } else if (block_plan(p.nx, p.ny, p.nz, p.storage, cus, &s.block)) {
         s.kind = StepPlan::BLOCK;
     } else if (pair_plan(p.nx, p.ny, p.nz, p.storage, p.halo_loopback != 0, cus, &s.pair)) {
         s.kind = StepPlan::PAIR;

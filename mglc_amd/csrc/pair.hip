@@ -35,8 +35,8 @@ struct PairTable {
 };
 
 // What a turn takes at least, and how its bytes count in the cache (see below).
-constexpr PairCost COST_F64{4.3, 1.0, 0.7}, COST_F32{5.5, 1.2, 0.7};
-constexpr PairCost COST_F64_LOOP{5.8, 1.2, 0.7}, COST_F32_LOOP{7.2, 1.5, 0.7};  // with the looped-back halo's stores
+constexpr PairCost COST_F64{4.3, 1.0, 0.25}, COST_F32{5.5, 1.2, 0.2};
+constexpr PairCost COST_F64_LOOP{5.8, 1.2, 0.5}, COST_F32_LOOP{7.2, 1.5, 0.3};  // with the looped-back halo's stores
 
 }  // namespace
 
@@ -56,18 +56,20 @@ bool pair_plan(int nx, int ny, int nz, int storage, bool loop, int cus, PairTile
 // takes ceil(blocks / CUs) rounds of cz + 2 turns.  A turn takes at least 4.3 us
 // in FP64, 5.5 in FP32 (twice the cells), 5.8 and 7.2 with the looped-back halo,
 // 5.1 and 5.8 with temperature (medians over 2000 random boxes of 16 to 256 cells a
-// side; with one 4.3 us for all, 8 % of the boxes ran slower in pairs, by up to a
-// fifth; now 1 %, by up to a tenth).  On large boxes it is
-// bound by memory (256^3 FP64: 622 us a step without the arithmetic and LDS, 627
-// with them) and goes as the bytes it moves, a row of the tile and its rim
-// costing 128 bytes more per population than it holds (the lines at its ends):
+// side).  Against one step per launch in transforms, which the pair form replaced:
+// of 1064 random boxes of 12 to 256 cells planned in pairs or blocks 2 ran below
+// 0.97 of its speed (0.94), half at 1.4 and more.  On large boxes a turn is bound
+// by memory (256^3 FP64: 622 us a step without the arithmetic and LDS, 627 with
+// them) and goes as the bytes it moves, a row of the tile and its rim costing 128
+// bytes more per population than it holds (the lines at its ends):
 // FP64 32 x 13 tiles 7.3 us, 64 x 5 5.7; FP32 64 x 13 6.9, 32 x 26 8.0, i.e.
 // 0.77 ns per such byte with every CU busy, less where fewer are (6.5 us for FP64
 // 32 x 13 with 240 of 256), 0.5 ns in the cache.  Rows that are not whole 64-byte
 // groups cost 1.1 to 1.4 times that outside the cache.  A one-step launch takes
 // 5 us and 5.2 TB/s of its traffic.
 // FP16 keeps the one-step kernel: half the bytes, but the rim adds a third to its
-// VALU issue, which alone takes 217 us (276 against 238 us a step at 256^3).
+// VALU issue, which alone takes 217 us (276 against 238 us a step at 256^3, with the
+// collision in pair form; in moments it issues a quarter more).
 namespace {
 
 // Tiles of width tx for an nx x ny plane; false where nt threads cannot hold them.
@@ -138,6 +140,7 @@ bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, PairCost cost
     const double bytes = elem, cells = double(nx) * ny * nz;
     const bool cached = in_cache(cells, bytes, pops);
     if (((long long)nx + 15) / 16 * 16 * ny * elem >= (long long)PLANE_RANGE) return false;  // the lanes' offsets
+    if ((long long)((nx + 63) / 64) * ny * nz <= (long long)cost.held * cus) return false;
     double best = 1e30;
     for_widths(nx, [&](int tx) {
         PairTiles t;
@@ -156,10 +159,13 @@ bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, PairCost cost
             }
         }
     });
-    // one step per launch: a row's last wave is part empty, which counts where the
-    // lattices lie in the cache
-    const double lanes = double((nx + 63) / 64 * 64) * ny * nz;
-    const double one = one_step_us(cached ? std::max(cells, cost.lanes * lanes) : cells, bytes, pops);
+    // One step per launch: a row's last wave is part empty, which counts where the
+    // lattices lie in the cache.  Fitted to 340 random boxes there: per lane, rows a
+    // quarter full took 0.5 (FP64) and 0.36 (FP32) of what full ones take, half full
+    // ones 0.62 and 0.64.  (As 0.7 of a cell per lane, full or not, boxes of 13 to 32
+    // cells along x went in pairs at 0.83 to 0.97 of the one-step kernel's speed.)
+    const double idle = double((nx + 63) / 64 * 64 - nx) * ny * nz;
+    const double one = one_step_us(cached ? cells + cost.lanes * idle : cells, bytes, pops);
     // (margins for what the model misses)
     return best < (one < 16.0 ? 0.9 : 0.95) * one;
 }

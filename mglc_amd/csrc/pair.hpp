@@ -301,7 +301,8 @@ bool pair_plan(int nx, int ny, int nz, int storage, bool loop, int cus, PairTile
 struct PairCost {
     double least;   // us of a turn at least
     double cached;  // times what a turn's bytes take where the lattices lie in the cache
-    double lanes;   // what a row's idle lanes cost the one-step kernel there, as a share of cells
+    double lanes;   // what an idle lane of a row's last wave costs the one-step kernel there, as a share of a cell
+    int held = 0;   // boxes whose one-step waves, up to this many per CU, all run at once keep that kernel
 };
 bool pair_plan(int nx, int ny, int nz, int nt, int pops, int elem, PairCost cost, int cus, PairTiles* out);
 

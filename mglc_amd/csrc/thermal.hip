@@ -691,9 +691,12 @@ bool thermal_pair_plan(const lbm_params& p, int cus, PairTiles* t) {
     if (p.halo_loopback) return false;
     switch (p.storage) {
     case LBM_STORE_F64:
-        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF64>::NT, QT + 1, 8, {5.1, 1.2, 0.5}, cus, t);
+        // Up to 8 waves a CU the one-step kernel takes 8 to 11.8 us whatever the box (95 x
+        // 66 x 15: 9.1, in pairs 11.0; 123 x 56 x 17 10.4 and 11.7; 64 x 67 x 26 10.2 and
+        // 11.1; 57 x 35 x 57 11.7 both), past it 14 and more (62 x 55 x 42 15.7 and 13.0).
+        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF64>::NT, QT + 1, 8, {5.1, 1.2, 0.35, 8}, cus, t);
     case LBM_STORE_F32:
-        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF32>::NT, QT + 1, 4, {5.8, 1.3, 0.5}, cus, t);
+        return pair_plan(p.nx, p.ny, p.nz, ThermalPairShape<StoreF32>::NT, QT + 1, 4, {5.8, 1.3, 0.25}, cus, t);
     }
     return false;
 }
