@@ -441,11 +441,12 @@ int device_cus() {
 // Blocks of the one-step launches: as many as there are tiles for, up to 512
 // waves per CU: a wave that walks few tiles leaves its CU to the next one early.
 // Measured on MI355X on 32, 128 and 512 waves per CU: 24 cavities of 32^3-64^3
-// FP32 69.9, 65.9 and 64.4 us a step, FP16 63.8, 54.8 and 54.5; 64 cavities of
-// 32^3-96^3 FP32 637, 628 and 589.
-int default_blocks(int threads, int tiles) {
+// FP32 69.9, 65.9 and 64.4 us a step; 64 cavities of 32^3-96^3 FP32 637, 628 and 589.
+// FP16 at most 48 (same cavities, on 32, 48, 64 and all there are tiles for: 78.1,
+// 67.8, 68.4 and 75.7; 600, 508, 518 and 585; 14 k tiles 27.3, 27.1, 28.3 and 28.2).
+int default_blocks(int threads, int tiles, int storage) {
     const int waves = threads / 64;
-    return std::min(device_cus() * (512 / waves), (tiles - 1) / waves + 1);
+    return std::min(device_cus() * ((storage == LBM_STORE_F16 ? 48 : 512) / waves), (tiles - 1) / waves + 1);
 }
 
 // The blocks of the two-step launches, where they are faster and what they need
@@ -578,7 +579,7 @@ int lbm_batch_create(const lbm_params* params, int count, lbm_batch** out) {
     b->device_bytes = (long long)(2 * b->elem * off + sizeof(double) * (loff + 4 * moff) + sizeof(BatchInst) * count);
     plan_pairs(b);
     b->threads = 256;
-    b->blocks = default_blocks(b->threads, b->total_tiles);
+    b->blocks = default_blocks(b->threads, b->total_tiles, b->p0.storage);
     // single-domain arguments per instance, for the one-launch-per-instance baseline
     b->single.resize(count);
     for (int m = 0; m < count; ++m) {
@@ -623,7 +624,7 @@ int lbm_batch_initial(lbm_batch* b) {
                        b->macro + 3 * b->total_cells, b->total_cells);
     BatchArgs a = batch_args(b);
     a.dst = b->buf[0];
-    hipLaunchKernelGGL(batch_init_fn(b), dim3(default_blocks(256, b->total_tiles)), dim3(256), 0, b->stream, a);
+    hipLaunchKernelGGL(batch_init_fn(b), dim3(default_blocks(256, b->total_tiles, b->p0.storage)), dim3(256), 0, b->stream, a);
     hipLaunchKernelGGL(k_counter_set, dim3(1), dim3(1), 0, b->stream, b->ctr, 1u);
     int rc = lbm_check_launch();
     if (rc) return rc;
