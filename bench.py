@@ -218,6 +218,14 @@ def oracle_rate(run, cells, budget_s=15.0, max_steps=200):
     return cells * steps / sec / 1e6, steps
 
 
+def launches(steps, blocks):
+    """How the library makes the steps (lbm_get_plan, lbm_batch_get_plan)."""
+    if steps == 1:
+        return "one step per launch"
+    shape = " x ".join(map(str, blocks)) if isinstance(blocks, tuple) else str(blocks)
+    return f"{steps} steps per launch, {shape} blocks"
+
+
 # ---- lid-driven cavity (headline) ------------------------------------------
 def run_storage(args, storage, stream):
     from mglc_amd.lbm import Cavity, CavityConfig
@@ -231,9 +239,8 @@ def run_storage(args, storage, stream):
     with make() as cav:
         cav.initial()
         warm_ms = device_warmup(make, stream) if args.device_warmup else 0.0
-        # with the loopback the step kernels (FP64 and FP32: two steps per
-        # launch) also write the outgoing halo (the first, untimed step call
-        # exchanged the initial state's halo once)
+        # with the loopback the step kernels also write the outgoing halo (the
+        # first, untimed step call exchanged the initial state's halo once)
         ms, wall = timed(cav.step, stream, args)
         # a step call writes the macroscopic fields on its last step only:
         # time single-step calls (each such a step) to split the timed
@@ -242,6 +249,7 @@ def run_storage(args, storage, stream):
                             argparse.Namespace(warmup=1, steps=5))
         ms_macro /= 5
         info = cav.info()
+        plan = cav.plan()
         halo_bytes = cav.halo_buffer_bytes() if args.halo_loopback else 0
         done = args.warmup + args.steps + 6
         if args.accuracy_steps > done:
@@ -262,7 +270,7 @@ def run_storage(args, storage, stream):
                 # a step call writes rho, u, v, w (FP64) on its last step: the K
                 # timed launches write them once
                 bytes_per_launch=info.bytes_per_lup * cells + halo_bytes + 32.0 * cells / args.steps,
-                halo_bytes=halo_bytes, fields=fields,
+                halo_bytes=halo_bytes, fields=fields, plan=plan,
                 steps_total=steps_total)
 
 
@@ -355,18 +363,19 @@ def bench_cavity(args, stream):
                         else round(r["ms_plain_step"], 4),
                         "speedup_vs_f64": round(r["mlups"] / primary["mlups"], 3),
                         "rel_l2_velocity_vs_f64": l2, "mass_drift_vs_f64": drift,
-                        "compared_at_step": r["steps_total"], "device_warmup_ms": r["warm_ms"]}
+                        "compared_at_step": r["steps_total"], "kernel": launches(*r["plan"]),
+                        "device_warmup_ms": r["warm_ms"]}
     m0 = float(primary["fields"][0].size)
     workload = f"lid-driven cavity D3Q19 {args.n}^3 Re=1000 U0=0.1 {args.collision.upper()}"
     config = {"workload": workload, "cells": args.n ** 3, "collision": args.collision,
-              "storage": "f64", "pattern": "A-B pull, two steps per pass", "kernel": "k_cavity_pair",
+              "storage": "f64", "pattern": "A-B pull", "kernel": launches(*primary["plan"]),
               "halo": "6 faces x 5 pops + 12 edges looped back every step (written by the step kernel)"
               if args.halo_loopback else "none",
               "kernel_ms_per_step": round(primary["ms_kernel"] / args.steps, 4),
               "ms_macro_step": round(primary["ms_macro_step"], 4),
               "ms_per_step_without_macro": None if primary["ms_plain_step"] is None
               else round(primary["ms_plain_step"], 4),
-              "waves_per_cu": args.waves_per_cu or "library default (16)",
+              "waves_per_cu": args.waves_per_cu or "library default",
               "bytes_per_launch": {"lattice": int(primary["bytes_per_lup"] * args.n ** 3),
                                    "macro_fields_once_per_K_launches": 32 * args.n ** 3,
                                    "outgoing_halo": int(primary["halo_bytes"])},
@@ -409,6 +418,7 @@ def bench_batch(args, stream_unused):
         b.initial()
         threads, blocks = b.autotune(trial_steps=4)
         info = b.info()
+        plan = b.plan()
         s = Stream(borrowed=info.stream)
         ms, wall = timed(b.step, s, args)
         a2 = argparse.Namespace(warmup=2, steps=each_steps)
@@ -421,11 +431,12 @@ def bench_batch(args, stream_unused):
     config = {"workload": f"64 lid-driven cavities D3Q19, N in {{32,48,64,80,96}}^3 (seed 12345), Re U[100,1000], "
                           f"U0 U[0.05,0.1], {args.collision.upper()}, FP32 storage",
               "cells": cells, "instances": len(cfgs), "sizes_present": sizes, "storage": "f32",
-              "kernel": "k_batch_pair (two steps per launch, 100-step hipGraph replays)", "threads": threads,
-              "blocks": blocks, "cells_per_thread": info.cells_per_thread, "graph_steps": info.graph_steps}
+              "kernel": launches(*plan[:2]) + ", 100-step hipGraph replays",
+              "one_step_shape": {"threads": threads, "blocks": blocks, "cells_per_thread": info.cells_per_thread},
+              "graph_steps": info.graph_steps}
     line = line_head(args, mlups, ms / args.steps, "f32", "synthetic (reference initial state per instance)", config)
-    # kernel time per launch: the graph holds one step kernel per step and
-    # one 1-thread step-counter kernel per 100 steps
+    # time per step: the graph holds the step kernels and one 1-thread
+    # step-counter kernel per 100 steps
     line["roofline"] = roofline(info.bytes_per_lup * cells, ms / args.steps, traffic_from_profiles("batch64 f32"))
     if args.attainable:
         # probed on one cube of about the batch's total cell count (the
@@ -570,7 +581,7 @@ def bench_thermal(args, stream):
             done = args.warmup + args.steps
             if args.accuracy_steps > done:
                 cav.step(args.accuracy_steps - done)
-            out = dict(ms=ms, nu=cav.nusselt(), info=cav.info(), fields=cav.macro(), T=cav.temperature(),
+            out = dict(ms=ms, nu=cav.nusselt(), info=cav.info(), plan=cav.plan(), fields=cav.macro(), T=cav.temperature(),
                        warm=warm)
         return out
 
@@ -579,11 +590,11 @@ def bench_thermal(args, stream):
     cells = n ** 3
     ms = primary["ms"]
     mlups = cells * args.steps / (ms * 1e-3) / 1e6
-    # k_thermal_step: 19 + 7 FP64 populations read and written, Fz read and written
+    # a step: 19 + 7 FP64 populations read and written, Fz read and written
     bpl = primary["info"].bytes_per_lup
     nu_vol, nu_wall = primary["nu"]
     config = {"workload": f"buoyancy-driven cavity D3Q19+D3Q7 {n}^3 Ra=1e5 Pr=0.71 walls +-0.5, MRT, FP64",
-              "cells": cells, "storage": "f64", "kernel": "k_thermal_pair", "bytes_per_lup": bpl,
+              "cells": cells, "storage": "f64", "kernel": launches(*primary["plan"]), "bytes_per_lup": bpl,
               "device_warmup_ms": primary["warm"]}
     line = line_head(args, mlups, ms / args.steps, "f64",
                      "synthetic (rho=1, u=0, T=0 plus seeded noise +-1e-4, held wall layers)", config)
