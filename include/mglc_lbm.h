@@ -158,10 +158,12 @@ int lbm_load_fields(lbm_ctx *ctx, const double *rho, const double *u, const doub
                     const double *w, const double *T);
 
 /* nsteps iterations of collision -> streaming -> bounceback -> macro
- * (main.f90:87-97), fused into one pass over the lattice per step or, in FP64
- * and FP32 with no halo to read, the library's own block shape and no stream
- * capture under way, per two or three steps where that is faster (the same
- * bits).  The macroscopic fields of the last step are kept for lbm_check and
+ * (main.f90:87-97), fused into one pass over the lattice per step or, with no
+ * halo to read, the library's own block shape and no stream capture under way,
+ * per two or three steps where that is faster (the same bits; lbm_get_plan tells
+ * which).  Such launches come in even numbers within a call, whose other steps go
+ * one by one, so that the state is where one launch per step would leave it and a
+ * captured graph of steps can be replayed between calls.  The macroscopic fields of the last step are kept for lbm_check and
  * lbm_download_macro.  With halo_loopback each step writes the next step's
  * halo itself (the current state's halo is exchanged once first when it is
  * not already in place); with halo faces and no loopback the caller

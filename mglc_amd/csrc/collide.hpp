@@ -47,7 +47,7 @@ __device__ __forceinline__ R mac(R acc, R x) {
 // power-of-two scale changes no bit of the result.
 // MOMENTS: the collision runs in the reference's 19 moments (collide_moments);
 // else in pair form (relax).  FP16 keeps the moments: in pair form its kernel
-// takes 509 VALU instructions instead of 646 (256^3: 234 us a step against 255),
+// has 509 VALU instructions instead of 646 (256^3: 231 us a step against 241),
 // but the last bits of a population then differ, and with them which way its
 // store rounds, so that a run goes another, equally far off, way.
 // Stores are non-temporal: the next step reads the written lattice only after

@@ -68,8 +68,9 @@ bool pair_plan(int nx, int ny, int nz, int storage, bool loop, int cus, PairTile
 // groups cost 1.1 to 1.4 times that outside the cache.  A one-step launch takes
 // 5 us and 5.2 TB/s of its traffic.
 // FP16 keeps the one-step kernel: half the bytes, but the rim adds a third to its
-// VALU issue, which alone takes 217 us (276 against 238 us a step at 256^3, with the
-// collision in pair form; in moments it issues a quarter more).
+// VALU issue, which alone takes 205 us of 241 a step at 256^3 (481 instructions a
+// wave; with the collision in pair form, which issues a fifth less, two steps per
+// launch took 276 us a step against 238).
 namespace {
 
 // Tiles of width tx for an nx x ny plane; false where nt threads cannot hold them.
